@@ -193,3 +193,42 @@ def test_lists_survive_a_common_translation(graphs):
     if graphs:
         captures, replays, fallbacks = a.graph_stats()
         assert replays >= 20 and fallbacks == 0, (captures, replays, fallbacks)
+
+
+@pytest.mark.parametrize("beta", [0.0, 2e-5])
+@pytest.mark.parametrize("ratio", [1.0, 1.3, 9.0])
+def test_contact_point_rule_from_grazing_to_swallowed_pairs(ratio, beta):
+    """Isolated pairs whose overlap runs from rounding size to one sphere deep inside the other, anywhere against the
+    bin grid (its faces included): the rule's short cut and its full evaluation give the oracle's list, whether the
+    pairs come from the cell sweep or from candidate lists."""
+    import pyoracle
+
+    rng = np.random.default_rng(int(ratio * 10) + (beta > 0))
+    r, n = 0.001, 12
+    R = r * ratio
+    pitch = 2.6 * (r + R)
+    g = np.stack(np.meshgrid(*[np.arange(n)] * 3, indexing="ij"), -1).reshape(-1, 3) * pitch
+    m = len(g)
+    reach = np.float64(np.float32(r) + np.float32(beta)) + np.float64(np.float32(R) + np.float32(beta))
+    depth = reach * np.concatenate([10.0 ** rng.uniform(-9, -4, m // 2), rng.uniform(1e-4, 0.95, m - m // 2)])
+    d = rng.normal(size=(m, 3))
+    d[::5] = np.eye(3)[rng.integers(0, 3, len(d[::5]))]  # axis-aligned pairs
+    d /= np.linalg.norm(d, axis=1, keepdims=True)
+    a = g + rng.uniform(0, 0.2 * r, (m, 3))
+    a[::3] = np.round(a[::3] / (2 * r)) * (2 * r)  # centres on bin faces
+    b = a + d * (reach - depth)[:, None]
+    xyz = np.stack([a, b], 1).reshape(-1, 3)
+    box = float(xyz.max() - xyz.min() + 2.2 * R)
+    xyz += -box / 2 - xyz.min() + 1.1 * R
+    rad = np.tile(np.array([r, R], np.float32), m)
+    sc = scenes.spheres_scene(xyz, rad, (box, box, box), beta=beta, planes=False)
+    ora = pyoracle.OracleSystem(sc)
+    ora.cd_run()
+    ref = ora.contacts()
+    assert len(ref[0]) > 0.7 * m
+    for skin in (0.0, -1.0):
+        dev = DeviceSystem(sc)
+        dev.set_skin(skin)
+        dev.cd_run()
+        for x, y in zip(dev.contacts()[:3], ref[:3]):
+            assert np.array_equal(x, y), skin
