@@ -60,7 +60,6 @@ def bytes_model(name, k):
         "bside_sort": O * 8 + Np * 8,
         # per contact: ids + type, history in/out, force record out; owner and sphere records (unique footprint)
         "force": C * (9 + 16 + 16 + 48) + S * sph + O * owner_dyn + (C * 4 if k.get("fresh") else 0),
-        "anal_collect": C * 5 + k["geo"] * (4 + 48),
         # cell-list detection: per sphere template + owner pose in; cell, slot, bin count, plane count and plane bits
         # out; one 4-byte RMW per occupied cell
         "cell_assign": S * sph + O * owner_cd + S * (4 + 4 + 2 + 4 + 8) + Nc * 8,
@@ -97,7 +96,6 @@ def bytes_model(name, k):
         "scan_cand": S * 4 * 2,
         # candidate rows copied (sorted) from the slab into id order with their sphere ids, build positions out
         "cand_rows": S * (4 + 4 + 32 + 12) + Nk * (4 + 4 + 4),
-        "anal_final": k["anal_blocks"] * 48 * 4,
         # per owner: own record in/out, MOI, accelerations out; A rows contiguous, B lists gathered
         "owner_update": O * (64 + 64 + 16 + 24 + 8) + C * 48 + Np * (4 + 48),
     }
@@ -133,7 +131,7 @@ def run_inspectors(dev, sc, calls=20):
 def run_device(sc, steps, warmup, update_freq, jit=False, inspect=False, prepare=None, keep_state=False):
     """Warm-up, then `steps` timed steps without kernel events, then as many with events (per-kernel durations).
     keep_state: also return the final owner state (host arrays) in info["state"]."""
-    from deme_amd.abi import ANAL_TILE, DeviceSystem
+    from deme_amd.abi import DeviceSystem
 
     dev = DeviceSystem(sc)
     if prepare is not None:
@@ -164,8 +162,7 @@ def run_device(sc, steps, warmup, update_freq, jit=False, inspect=False, prepare
     info = dict(S=sc.n_spheres, O=sc.n_owners, P=c.nBinSphereTouches, C=c.nContacts, Cprev=c.nPrevContacts,
                 pairs=c.nContacts - c.nSphereGeoContacts, geo=c.nSphereGeoContacts, Ba=c.nActiveBins,
                 nbins=sc.params.nbX * sc.params.nbY * sc.params.nbZ, cells=c.nCells, fresh=update_freq == 1,
-                anal_blocks=(c.nContacts + ANAL_TILE - 1) // ANAL_TILE, cand=n_cand, skin=skin, cand_builds=builds,
-                inspectors=insp,
+                cand=n_cand, skin=skin, cand_builds=builds, inspectors=insp,
                 evented_ms_per_step=1e3 * (te1 - te0) / steps)
     if keep_state:
         info["state"] = dev.get_state()

@@ -61,23 +61,7 @@ __global__ __launch_bounds__(64) void k_plane_pose(KParams P, const deme_anal_ob
     if (a >= nA) return;
     const deme_anal_obj ob = anal[a];
     const OwnerRec o = load_owner(own, ob.owner);
-    double ox, oy, oz;
-    owner_position(P, o.voxel, o.lx, o.ly, o.lz, ox, oy, oz);
-    float px = ob.relPos[0], py = ob.relPos[1], pz = ob.relPos[2];
-    float nx = ob.rot[0], ny = ob.rot[1], nz = ob.rot[2];
-    rotate(px, py, pz, o.qw, o.qx, o.qy, o.qz);
-    rotate(nx, ny, nz, o.qw, o.qx, o.qy, o.qz);
-    PlanePose pp;
-    pp.px = ox + (double)px;
-    pp.py = oy + (double)py;
-    pp.pz = oz + (double)pz;
-    pp.nx = nx;
-    pp.ny = ny;
-    pp.nz = nz;
-    pp.owner = ob.owner;
-    pp.fam = o.fam;
-    pp.type = ob.type;
-    pose[a] = pp;
+    pose[a] = plane_pose_of(P, ob, o);
 }
 
 // Rows a6 + a10 (+ histogram of a8): getNumberOfBinsEachSphereTouches (DEMBinSphereKernels.cu:12-115).

@@ -237,7 +237,7 @@ struct deme_ctx {
     DBuf<float4> hist[2];
     DBuf<uint32_t> idA, map;
     DBuf<ForceRec> frc;           // full contact records, kept by deme_force only
-    DBuf<float> aTerm, bTerm, gTerm;  // owner terms: A side per contact, B side per mirror slot / per plane contact
+    DBuf<float> aTerm, bTerm;  // owner terms: A side per contact, B side per mirror slot
     DBuf<uint8_t> aOn, bOn;           // term written (the pair touches) per contact / per mirror slot
     bool forcesFull = false;
     // adjoint: checkpoints at window starts (+ the final state) and the recorded steps of one window
@@ -263,7 +263,8 @@ struct deme_ctx {
     DBuf<float> lam, lAcc, adjA, adjB, matPart, matGrad;
     DBuf<float4> lDt[2], lDtPrev;
     bool termsReady = false;  // owner terms belong to the current contact list
-    DBuf<float> analPartials, analAcc;
+    DBuf<float> analPartials;  // plane owners' partial sums, one set per force workgroup
+    bool posesValid = false;   // pose[] belongs to the owners' current state (the owner update refreshes it)
     DBuf<double> clock;  // simulation time read by the owner update's motion rules (written before each such update)
     // cell-list detection
     CellGrid grid{};
@@ -414,6 +415,14 @@ int check_ready(deme_ctx* c) {
     return build_scene_planes(c);
 }
 
+// The plane poses of the owners' current state (the last owner update refreshed them unless the state changed since).
+int ensure_poses(deme_ctx* c) {
+    if (c->posesValid) return DEME_OK;
+    DEME_LAUNCH(c, "plane_pose", launch_plane_pose(c->kp, c->anal.p, c->nA, c->own.p, c->pose.p, c->stream));
+    c->posesValid = true;
+    return DEME_OK;
+}
+
 int readback_counters(deme_ctx* c) {
     DEME_HIP(c, hipMemcpyAsync(c->hctr, c->ctr.p, DEV_COUNTERS_HOST_BYTES, hipMemcpyDeviceToHost, c->stream));
     DEME_HIP(c, hipStreamSynchronize(c->stream));
@@ -483,11 +492,11 @@ int deme_ctx_destroy(deme_ctx* c) {
     c->binCount.release(); c->binStart.release(); c->numBins.release(); c->numAnal.release(); c->rec.release();
     c->binEnt.release(); c->pairs.release(); c->rowCount.release(); c->bCnt.release(); c->bRowStart.release();
     c->bPart.release(); c->mirror.release(); c->scanScratch.release(); c->ctr.release();
-    c->aTerm.release(); c->bTerm.release(); c->gTerm.release(); c->aOn.release(); c->bOn.release();
+    c->aTerm.release(); c->bTerm.release(); c->aOn.release(); c->bOn.release();
     for (int k = 0; k < 2; k++) {
         c->rowStart[k].release(); c->idB[k].release(); c->ctype[k].release(); c->hist[k].release();
     }
-    c->idA.release(); c->map.release(); c->frc.release(); c->analPartials.release(); c->analAcc.release();
+    c->idA.release(); c->map.release(); c->frc.release(); c->analPartials.release();
     c->clock.release();
     c->cellCount.release(); c->cellStart.release(); c->cellOf.release(); c->slotOf.release(); c->posOf.release();
     c->survSlab.release(); c->rowSlab.release(); c->mirSlab.release(); c->sorted.release(); c->planeBits.release();
@@ -535,6 +544,7 @@ int deme_sync(deme_ctx* c) {
 }
 
 int deme_set_params(deme_ctx* c, const deme_sim_params* p) {
+    c->posesValid = false;
     c->graphGen++;
     c->candValid = false;  // positions, radii or the margin changed: candidate lists are rebuilt
     c->adjReady = false;  // recorded adjoint checkpoints no longer describe the system
@@ -581,6 +591,7 @@ int deme_upload_templates(deme_ctx* c, uint32_t nS, const uint32_t* sphOwner, co
                           const float* sphRelPos, const uint8_t* sphMat, uint32_t nO, uint32_t nClumps,
                           const float* ownerMass, const float* ownerMoi) {
     c->graphGen++;
+    c->posesValid = false;
     c->candValid = false;  // positions, radii or the margin changed: candidate lists are rebuilt
     c->adjReady = false;  // recorded adjoint checkpoints no longer describe the system
     if (nClumps > nO) return c->fail(DEME_ERR_INVALID_ARGUMENT, "nClumps > nOwners");
@@ -673,6 +684,7 @@ int deme_upload_materials(deme_ctx* c, uint32_t n, const deme_material* m) {
 }
 
 int deme_upload_analytical(deme_ctx* c, uint32_t n, const deme_anal_obj* objs) {
+    c->posesValid = false;
     c->graphGen++;
     c->adjReady = false;  // recorded adjoint checkpoints no longer describe the system
     if (!c->haveTemplates) return c->fail(DEME_ERR_NOT_READY, "upload templates before analytical objects");
@@ -743,6 +755,7 @@ int deme_upload_families(deme_ctx* c, const uint8_t* mask, const deme_family_rul
 }
 
 int deme_upload_state(deme_ctx* c, const deme_owner_state* s) {
+    c->posesValid = false;
     c->candValid = false;  // positions, radii or the margin changed: candidate lists are rebuilt
     c->adjReady = false;  // recorded adjoint checkpoints no longer describe the system
     if (!c->haveTemplates) return c->fail(DEME_ERR_NOT_READY, "upload templates before the owner state");
@@ -844,7 +857,7 @@ int deme_cd_bin_count(deme_ctx* c) {
     DEME_HIP(c, c->binStart.ensure(c->nBins + 1, 1.0));
     DEME_HIP(c, c->scanScratch.ensure(scan_scratch_elems(std::max<uint64_t>({c->nBins, (uint64_t)c->nS, 1u << 22})), 1.0));
     DEME_HIP(c, hipMemsetAsync(c->ctr.p, 0, sizeof(DevCounters), c->stream));
-    DEME_LAUNCH(c, "plane_pose", launch_plane_pose(c->kp, c->anal.p, c->nA, c->own.p, c->pose.p, c->stream));
+    if ((r = ensure_poses(c))) return r;
     // the occupancy histogram must start at zero whatever ran before (an aborted pass leaves counts behind)
     DEME_LAUNCH(c, "fill", launch_fill_u32(c->binCount.p, c->nBins, 0, c->stream));
     DEME_LAUNCH(c, "sphere_bins",
@@ -951,7 +964,6 @@ int deme_cd_sort_remap(deme_ctx* c) {
     DEME_HIP(c, c->bPart.ensure(c->nPairs));
     DEME_HIP(c, c->aTerm.ensure((size_t)6 * C));
     DEME_HIP(c, c->aOn.ensure(C));
-    DEME_HIP(c, c->gTerm.ensure((size_t)6 * C));
     DEME_HIP(c, c->bTerm.ensure((size_t)6 * c->nPairs));
     DEME_HIP(c, c->bOn.ensure(c->nPairs));
     c->termsReady = false;
@@ -1096,7 +1108,7 @@ static int cd_buffers(deme_ctx* c, int* mode) {
 // assignment (bin counts and plane contacts on the way), the cell scan and the counting-sort scatter.
 static int enqueue_cell_pass(deme_ctx* c, int mode) {
     const uint32_t nS = c->nS;
-    DEME_LAUNCH(c, "plane_pose", launch_plane_pose(c->kp, c->anal.p, c->nA, c->own.p, c->pose.p, c->stream));
+    if (int r = ensure_poses(c)) return r;
     // cell counts and the pass's counters cleared by one kernel (a small memset is two fills on this runtime)
     static_assert(sizeof(DevCounters) % 4 == 0, "counters are cleared as 32-bit words");
     DEME_LAUNCH(c, "fill", launch_fill_u32(c->cellCount.p, c->nCells, 0, c->stream,
@@ -1271,6 +1283,7 @@ static int enqueue_skin_pass(deme_ctx* c, int cu) {
     DEME_LAUNCH(c, "plane_pose",
                 launch_pass_start(c->kp, c->anal.p, c->nA, c->own.p, c->pose.p, reinterpret_cast<uint32_t*>(c->ctr.p),
                                   sizeof(DevCounters) / 4, c->stream));
+    c->posesValid = true;
     // (the families for the mask only when a mask is in force; no per-sphere bin counts: this path never reads them)
     DEME_LAUNCH(c, "sphere_pos",
                 launch_sphere_pos(c->kp, c->sph.p, c->own.p, nS, c->pose.p, c->nA, c->maskAny ? c->mask.p : nullptr,
@@ -1428,7 +1441,6 @@ int deme_cd_run(deme_ctx* c) {
     DEME_HIP(c, c->bPart.ensure(nPairs));
     DEME_HIP(c, c->aTerm.ensure((size_t)6 * C));
     DEME_HIP(c, c->aOn.ensure(C));
-    DEME_HIP(c, c->gTerm.ensure((size_t)6 * C));
     DEME_HIP(c, c->bTerm.ensure((size_t)6 * nPairs));
     DEME_HIP(c, c->bOn.ensure(nPairs));
     c->termsReady = false;
@@ -1544,6 +1556,28 @@ static uint8_t* term_flags(deme_ctx* c, bool bSide) {
     return bSide ? c->bOn.p : c->aOn.p;
 }
 
+// The plane owners' partial sums as the force kernel writes them (analPartials sized for the launch beforehand).
+static PlaneSums plane_sums(const deme_ctx* c) {
+    PlaneSums s;
+    s.part = c->analPartials.p;
+    s.first = c->nClumps;
+    s.nOwners = c->nAnalOwners;
+    return s;
+}
+
+static PlaneRefresh plane_refresh(const deme_ctx* c) {
+    PlaneRefresh r;
+    r.anal = c->anal.p;
+    r.pose = c->pose.p;
+    r.nA = c->nA;
+    return r;
+}
+
+// Room for the partial sums of a force launch over nC contacts.
+static hipError_t ensure_partials(deme_ctx* c, uint64_t nC, double grow = 1.25) {
+    return c->analPartials.ensure(std::max<size_t>((size_t)anal_blocks(nC) * MAX_ANAL_OWNERS * 6, 1), grow);
+}
+
 // The force kernel of the context: the specialised one when a model or placeholder values were given, else the
 // ahead-of-time kernel of the built-in model.
 static hipError_t launch_force_ctx(deme_ctx* c, bool full, uint32_t nC, const uint32_t* idB, const uint8_t* ctype,
@@ -1551,30 +1585,29 @@ static hipError_t launch_force_ctx(deme_ctx* c, bool full, uint32_t nC, const ui
                                    ForceRec* out, SpecGuard guard = SpecGuard()) {
     if (c->jitActive)
         return c->jit.launch(full, c->kp, nC, c->idA.p, idB, ctype, c->sph.p, own, c->moi.p, c->anal.p, c->pose.p,
-                             c->mats.p, histIn, map, histOut, c->mirror.p, c->aTerm.p, c->bTerm.p, c->gTerm.p,
+                             c->mats.p, histIn, map, histOut, c->mirror.p, c->aTerm.p, c->bTerm.p, plane_sums(c),
                              term_flags(c, false), term_flags(c, true), out, c->stream, guard);
     return launch_force(c->kp, nC, c->idA.p, idB, ctype, c->sph.p, own, c->moi.p, c->anal.p, c->pose.p, c->mats.p,
-                        histIn, map, histOut, c->mirror.p, c->aTerm.p, c->bTerm.p, c->gTerm.p, term_flags(c, false),
+                        histIn, map, histOut, c->mirror.p, c->aTerm.p, c->bTerm.p, plane_sums(c), term_flags(c, false),
                         term_flags(c, true), out, c->stream, guard);
 }
 
 // The owner update of the context (the specialised kernel when motion strategies or rules were given): owner sums of
 // the list at parity cu, then the integration when `integrate`.
 static hipError_t launch_owner_ctx(deme_ctx* c, int integrate, int cu, SpecGuard guard = SpecGuard()) {
+    PlaneSums sums = plane_sums(c);
+    sums.nPart = guard.ctr ? PART_FROM_COUNTERS : anal_blocks(c->C);
+    const PlaneRefresh planes = plane_refresh(c);
     if (c->ownerJitActive)
-        return c->jitOwner.launch(c->kp, c->nO, c->nClumps, c->nClumps, c->nAnalOwners, c->ownerSphStart.p,
-                                  c->rowStart[cu].p, c->bRowStart.p, c->aTerm.p, c->bTerm.p, term_flags(c, false),
-                                  term_flags(c, true), c->analAcc.p, c->rules.p, c->own.p, c->own.p, c->acc.p,
-                                  integrate, c->clock.p, c->stream, guard);
-    return launch_owner_update(c->kp, c->nO, c->nClumps, c->nClumps, c->nAnalOwners, c->ownerSphStart.p,
-                               c->rowStart[cu].p, c->bRowStart.p, c->aTerm.p, c->bTerm.p, term_flags(c, false),
-                               term_flags(c, true), c->analAcc.p, c->rules.p, c->own.p, c->acc.p, integrate,
-                               c->clock.p, c->stream, nullptr, guard);
+        return c->jitOwner.launch(c->kp, c->nO, c->nClumps, c->ownerSphStart.p, c->rowStart[cu].p, c->bRowStart.p,
+                                  c->aTerm.p, c->bTerm.p, term_flags(c, false), term_flags(c, true), sums, planes,
+                                  c->rules.p, c->own.p, c->own.p, c->acc.p, integrate, c->clock.p, c->stream, guard);
+    return launch_owner_update(c->kp, c->nO, c->nClumps, c->ownerSphStart.p, c->rowStart[cu].p, c->bRowStart.p,
+                               c->aTerm.p, c->bTerm.p, term_flags(c, false), term_flags(c, true), sums, planes,
+                               c->rules.p, c->own.p, c->acc.p, integrate, c->clock.p, c->stream, nullptr, guard);
 }
 
-// poseFresh: a detection pass has just computed the plane poses from the same owner state (the same step), so the
-// force pass reuses them.
-static int force_pass(deme_ctx* c, bool full, bool poseFresh = false) {
+static int force_pass(deme_ctx* c, bool full) {
     int r = check_ready(c);
     if (r) return r;
     if (c->jitActive && c->jitStale && (r = jit_rebuild(c))) return r;
@@ -1583,8 +1616,8 @@ static int force_pass(deme_ctx* c, bool full, bool poseFresh = false) {
     const int cu = c->cur, pv = cu ^ 1;
     const bool remap = c->fresh;
     if (full) DEME_HIP(c, c->frc.ensure(c->C));
-    if (!poseFresh)
-        DEME_LAUNCH(c, "plane_pose", launch_plane_pose(c->kp, c->anal.p, c->nA, c->own.p, c->pose.p, c->stream));
+    if ((r = ensure_poses(c))) return r;
+    DEME_HIP(c, ensure_partials(c, c->C));
     DEME_LAUNCH(c, "force",
                 launch_force_ctx(c, full, (uint32_t)c->C, c->idB[cu].p, c->ctype[cu].p, c->own.p,
                                  remap ? (c->havePrev ? c->hist[pv].p : c->hist[cu].p) : c->hist[cu].p,
@@ -1601,19 +1634,12 @@ int deme_force(deme_ctx* c) { return force_pass(c, true); }
 static int collect_and_update(deme_ctx* c, int integrate, bool capturing = false) {
     if (!c->termsReady) return c->fail(DEME_ERR_NOT_READY, "the force pass must run on the current contact list first");
     const int cu = c->cur;
-    uint32_t nb = 0;
-    DEME_HIP(c, c->analPartials.ensure(std::max<size_t>((size_t)anal_blocks(c->C) * MAX_ANAL_OWNERS * 6, 1)));
-    DEME_HIP(c, c->analAcc.ensure(MAX_ANAL_OWNERS * 6, 1.0));
-    DEME_LAUNCH(c, "anal_collect",
-                launch_anal_collect((uint32_t)c->C, c->idB[cu].p, c->ctype[cu].p, c->gTerm.p, c->anal.p, c->nA,
-                                    c->nClumps, c->nAnalOwners, c->analPartials.p, c->analPartials.cap, &nb,
-                                    c->stream));
-    DEME_LAUNCH(c, "anal_final", launch_anal_final(c->analPartials.p, nb, c->nAnalOwners, c->analAcc.p, c->stream));
     // Motion rules read the time from the device clock; it is written here, before the update, on the stream (a step
     // replayed from a graph gets it from set_step_clock, launched outside the graph)
     if (integrate && c->ownerJitActive && !capturing)
         DEME_LAUNCH(c, "set_clock", launch_set_clock(c->clock.p, c->time, c->stream));
     DEME_LAUNCH(c, integrate ? "owner_update" : "owner_reduce", launch_owner_ctx(c, integrate, cu));
+    if (integrate) c->posesValid = true;
     return DEME_OK;
 }
 
@@ -1637,19 +1663,25 @@ int deme_integrate_owners(deme_ctx* c) {
     // the owner kernel reads nothing of the contact list in this mode
     if (c->ownerJitActive)
         DEME_LAUNCH(c, "set_clock", launch_set_clock(c->clock.p, c->time, c->stream));
+    const PlaneSums sums = plane_sums(c);
+    const PlaneRefresh planes = plane_refresh(c);
     DEME_LAUNCH(c, "owner_integrate",
                 c->ownerJitActive
-                    ? c->jitOwner.launch(c->kp, c->nO, c->nClumps, c->nClumps, c->nAnalOwners, nullptr, nullptr,
-                                         nullptr, nullptr, nullptr, nullptr, nullptr, nullptr, c->rules.p, c->own.p,
-                                         c->own.p, c->acc.p, 2, c->clock.p, c->stream)
-                    : launch_owner_update(c->kp, c->nO, c->nClumps, c->nClumps, c->nAnalOwners, nullptr, nullptr,
-                                          nullptr, nullptr, nullptr, nullptr, nullptr, nullptr, c->rules.p, c->own.p,
-                                          c->acc.p, 2, c->clock.p, c->stream));
+                    ? c->jitOwner.launch(c->kp, c->nO, c->nClumps, nullptr, nullptr, nullptr, nullptr, nullptr,
+                                         nullptr, nullptr, sums, planes, c->rules.p, c->own.p, c->own.p, c->acc.p, 2,
+                                         c->clock.p, c->stream)
+                    : launch_owner_update(c->kp, c->nO, c->nClumps, nullptr, nullptr, nullptr, nullptr, nullptr,
+                                          nullptr, nullptr, sums, planes, c->rules.p, c->own.p, c->acc.p, 2,
+                                          c->clock.p, c->stream));
+    c->posesValid = true;
     return DEME_OK;
 }
 
 // One non-detection step from the captured graph, capturing it first when anything it depends on changed.
 static int step_graph(deme_ctx* c) {
+    // (the captured step reads the poses the owner update before it left)
+    if (int r = ensure_poses(c)) return r;
+    DEME_HIP(c, ensure_partials(c, c->C));
     const bool valid = c->stepExec && c->capturedGen == c->graphGen &&
                        std::memcmp(&c->capturedKp, &c->kp, sizeof(KParams)) == 0;
     if (!valid) {
@@ -1703,7 +1735,7 @@ static std::vector<const void*> cycle_fingerprint(deme_ctx* c, int p) {
             c->scanScratch.p, c->survSlab.p,  c->rowSlab.p,     c->mirSlab.p,     c->rowStart[p].p, c->rowStart[q].p,
             c->bRowStart.p,  c->idA.p,        c->idB[p].p,      c->idB[q].p,      c->ctype[p].p,   c->ctype[q].p,
             c->hist[p].p,    c->hist[q].p,    c->map.p,         c->mirror.p,      c->bPart.p,      c->aTerm.p,
-            c->bTerm.p,      c->gTerm.p,      c->aOn.p,         c->bOn.p,         c->analPartials.p, c->analAcc.p,
+            c->bTerm.p,      c->aOn.p,        c->bOn.p,         c->analPartials.p,
             c->acc.p,        c->clock.p,      c->ctr.p,         c->planeStart.p,
             reinterpret_cast<const void*>(c->jit.full), reinterpret_cast<const void*>(c->jit.terms),
             reinterpret_cast<const void*>(c->jitOwner.fn),
@@ -1727,19 +1759,17 @@ static int cycle_capacity(deme_ctx* c, int p, SpecGuard& g) {
     DEME_HIP(c, c->map.ensure(wantC, 1.0));
     DEME_HIP(c, c->mirror.ensure(wantC, 1.0));
     DEME_HIP(c, c->aTerm.ensure(6 * wantC, 1.0));
-    DEME_HIP(c, c->gTerm.ensure(6 * wantC, 1.0));
     DEME_HIP(c, c->aOn.ensure(wantC, 1.0));
     DEME_HIP(c, c->bPart.ensure(wantP, 1.0));
     DEME_HIP(c, c->bTerm.ensure(6 * wantP, 1.0));
     DEME_HIP(c, c->bOn.ensure(wantP, 1.0));
-    DEME_HIP(c, c->analPartials.ensure((size_t)std::max(anal_blocks(wantC), 1u) * MAX_ANAL_OWNERS * 6, 1.0));
-    DEME_HIP(c, c->analAcc.ensure(MAX_ANAL_OWNERS * 6, 1.0));
+    DEME_HIP(c, ensure_partials(c, wantC, 1.0));
     g = SpecGuard();
     g.ctr = c->ctr.p;
     g.slabCap = c->slabCap;
     const uint64_t analCap = (uint64_t)(c->analPartials.cap / (MAX_ANAL_OWNERS * 6)) * ANAL_TILE;
     g.capC = std::min<uint64_t>({c->idB[p].cap, c->ctype[p].cap, c->hist[p].cap, c->idA.cap, c->map.cap,
-                                 c->mirror.cap, c->aTerm.cap / 6, c->gTerm.cap / 6, c->aOn.cap, analCap,
+                                 c->mirror.cap, c->aTerm.cap / 6, c->aOn.cap, analCap,
                                  0xFFFFFFFFull});
     g.capP = std::min<uint64_t>({c->bPart.cap, c->bTerm.cap / 6, c->bOn.cap});
     return DEME_OK;
@@ -1760,18 +1790,10 @@ static int enqueue_cycle(deme_ctx* c, int f, const SpecGuard& g, int mode) {
     if (r) return r;
     const uint32_t capC = (uint32_t)g.capC;
     for (int s = 0; s < f; s++) {
-        if (s > 0)
-            DEME_LAUNCH(c, "plane_pose", launch_plane_pose(c->kp, c->anal.p, c->nA, c->own.p, c->pose.p, c->stream));
         DEME_LAUNCH(c, "force",
                     launch_force_ctx(c, false, capC, c->idB[p].p, c->ctype[p].p, c->own.p,
                                      s == 0 ? c->hist[q].p : c->hist[p].p, s == 0 ? c->map.p : nullptr, c->hist[p].p,
                                      nullptr, g));
-        uint32_t nb = 0;
-        DEME_LAUNCH(c, "anal_collect",
-                    launch_anal_collect(capC, c->idB[p].p, c->ctype[p].p, c->gTerm.p, c->anal.p, c->nA, c->nClumps,
-                                        c->nAnalOwners, c->analPartials.p, c->analPartials.cap, &nb, c->stream, g));
-        DEME_LAUNCH(c, "anal_final",
-                    launch_anal_final(c->analPartials.p, nb, c->nAnalOwners, c->analAcc.p, c->stream, g));
         DEME_LAUNCH(c, "owner_update", launch_owner_ctx(c, 1, p, g));
         DEME_LAUNCH(c, "advance_clock", launch_advance_clock(c->clock.p, c->sp.h, c->stream));
     }
@@ -1834,6 +1856,8 @@ static int run_cycle(deme_ctx* c, int f, bool* done) {
     // a captured candidate-list pass maps the history through the previous list's candidate indices: they must be
     // the current build's
     if (c->skin() > 0.0 && c->cidxGen[c->cur] != c->candBuilds) return DEME_OK;
+    // (a captured pass over cells reads the poses the owner update before it left)
+    if (int r = ensure_poses(c)) return r;
     const bool valid = cy.exec && cy.gen == c->graphGen && cy.f == f &&
                        std::memcmp(&cy.kp, &c->kp, sizeof(KParams)) == 0 && cy.ptrs == cycle_fingerprint(c, p);
     if (!valid) {
@@ -1873,6 +1897,7 @@ static int run_cycle(deme_ctx* c, int f, bool* done) {
         c->time += (double)c->sp.h;
         c->nSteps++;
     }
+    c->posesValid = true;
     c->cycleReplays++;
     *done = true;
     return DEME_OK;
@@ -1915,7 +1940,7 @@ int deme_step(deme_ctx* c, int nSteps, int updateFreq) {
         if (!detect && !c->fresh && !records && c->useGraphs && !c->timing && !c->jitStale && c->stream) {
             if ((r = step_graph(c))) return r;
         } else {
-            r = force_pass(c, records, detect);
+            r = force_pass(c, records);
             if (r) return r;
             r = collect_and_update(c, 1);
             if (r) return r;
@@ -2171,6 +2196,7 @@ static int adj_save(deme_ctx* c, deme_ctx::AdjCk& k, bool full) {
 }
 
 static int adj_restore(deme_ctx* c, const deme_ctx::AdjCk& k) {
+    c->posesValid = false;
     c->graphGen++;
     c->candValid = false;  // positions, radii or the margin changed: candidate lists are rebuilt
     DEME_HIP(c, hipMemcpyAsync(c->own.p, k.own.p, c->nO * sizeof(OwnerRec), hipMemcpyDeviceToDevice, c->stream));
@@ -2195,7 +2221,6 @@ static int adj_restore(deme_ctx* c, const deme_ctx::AdjCk& k) {
             DEME_HIP(c, c->aTerm.ensure(std::max<uint64_t>((uint64_t)6 * k.C, 1)));
             DEME_HIP(c, c->bOn.ensure(std::max<uint64_t>(k.nPairs, 1)));
             DEME_HIP(c, c->aOn.ensure(std::max<uint64_t>(k.C, 1)));
-            DEME_HIP(c, c->gTerm.ensure(std::max<uint64_t>((uint64_t)6 * k.C, 1)));
             if (k.C) {
                 DEME_HIP(c, hipMemcpyAsync(c->idA.p, k.idA.p, k.C * 4, hipMemcpyDeviceToDevice, c->stream));
                 DEME_HIP(c, hipMemcpyAsync(c->mirror.p, k.mirror.p, k.C * 4, hipMemcpyDeviceToDevice, c->stream));
@@ -2244,9 +2269,11 @@ static int adj_window(deme_ctx* c, int n, bool record) {
         DEME_HIP(c, c->adjHist[k].ensure(std::max<uint64_t>(C, 1)));
         DEME_HIP(c, c->adjAcc[k].ensure((size_t)6 * c->nO));
     }
-    DEME_HIP(c, c->analAcc.ensure(MAX_ANAL_OWNERS * 6, 1.0));
     const int cu = c->cur, pv = cu ^ 1;
-    DEME_LAUNCH(c, "plane_pose", launch_plane_pose(c->kp, c->anal.p, c->nA, c->own.p, c->pose.p, c->stream));
+    if ((r = ensure_poses(c))) return r;
+    DEME_HIP(c, ensure_partials(c, C));
+    PlaneSums sums = plane_sums(c);
+    sums.nPart = anal_blocks(C);
     DEME_LAUNCH(c, "adj_gather", launch_adj_gather_hist((uint32_t)C, c->havePrev ? c->map.p : nullptr,
                                                          (uint32_t)c->Cprev, c->hist[pv].p, c->adjHist[0].p,
                                                          c->stream));
@@ -2256,12 +2283,10 @@ static int adj_window(deme_ctx* c, int n, bool record) {
         DEME_LAUNCH(c, "force", launch_force_ctx(c, false, (uint32_t)C, c->idB[cu].p, c->ctype[cu].p, c->adjOwn[k].p,
                                                  c->adjHist[k].p, nullptr, c->adjHist[k + 1].p, nullptr));
         DEME_LAUNCH(c, "owner_update",
-                    launch_owner_update(c->kp, c->nO, c->nClumps, c->nClumps, c->nAnalOwners, c->ownerSphStart.p,
-                                        c->rowStart[cu].p, c->bRowStart.p, c->aTerm.p, c->bTerm.p,
-                                        term_flags(c, false), term_flags(c, true),
-                                          c->analAcc.p,
-                                        c->rules.p, c->adjOwn[k].p, c->adjAcc[k].p, 1, c->clock.p, c->stream,
-                                        c->adjOwn[k + 1].p));
+                    launch_owner_update(c->kp, c->nO, c->nClumps, c->ownerSphStart.p, c->rowStart[cu].p,
+                                        c->bRowStart.p, c->aTerm.p, c->bTerm.p, term_flags(c, false),
+                                        term_flags(c, true), sums, PlaneRefresh(), c->rules.p, c->adjOwn[k].p,
+                                        c->adjAcc[k].p, 1, c->clock.p, c->stream, c->adjOwn[k + 1].p));
         c->time += (double)c->sp.h;
         c->nSteps++;
     }
@@ -2463,6 +2488,7 @@ int deme_change_family(deme_ctx* c, int from, int to) {
         return c->fail(DEME_ERR_INVALID_ARGUMENT, "family numbers lie in 0..255");
     if (!c->haveState) return c->fail(DEME_ERR_NOT_READY, "no owner state");
     c->adjReady = false;
+    c->posesValid = false;  // (a component's family is part of its pose record)
     DEME_LAUNCH(c, "change_family", launch_change_family(c->own.p, c->nO, (uint8_t)from, (uint8_t)to, c->stream));
     return DEME_OK;
 }
@@ -2551,6 +2577,7 @@ int deme_get_counts(deme_ctx* c, deme_counts* out) {
 int deme_append_clumps(deme_ctx* c, uint32_t nNewSph, const uint32_t* sphOwner, const float* sphRadius,
                        const float* sphRelPos, const uint8_t* sphMat, uint32_t nNew, const float* ownerMass,
                        const float* ownerMoi, const deme_owner_state* s) {
+    c->posesValid = false;
     c->candValid = false;  // positions, radii or the margin changed: candidate lists are rebuilt
     int r = check_ready(c);
     if (r) return r;

@@ -216,6 +216,44 @@ __device__ __forceinline__ CdRec load_cd(const CdRec* __restrict__ p, uint32_t i
     return r;
 }
 
+// World pose of an analytical component from its owner's state.
+__device__ __forceinline__ PlanePose plane_pose_of(const KParams& P, const deme_anal_obj& ob, const OwnerRec& o) {
+    double ox, oy, oz;
+    owner_position(P, o.voxel, o.lx, o.ly, o.lz, ox, oy, oz);
+    float px = ob.relPos[0], py = ob.relPos[1], pz = ob.relPos[2];
+    float nx = ob.rot[0], ny = ob.rot[1], nz = ob.rot[2];
+    rotate(px, py, pz, o.qw, o.qx, o.qy, o.qz);
+    rotate(nx, ny, nz, o.qw, o.qx, o.qy, o.qz);
+    PlanePose pp;
+    pp.px = ox + (double)px;
+    pp.py = oy + (double)py;
+    pp.pz = oz + (double)pz;
+    pp.nx = nx;
+    pp.ny = ny;
+    pp.nz = nz;
+    pp.owner = ob.owner;
+    pp.fam = o.fam;
+    pp.type = ob.type;
+    return pp;
+}
+
+// Sums over the sphere-plane contacts per analytical owner, passed from the force kernel to the owner update. Each
+// force workgroup (ANAL_TILE contacts) writes nOwners x 6 partial sums at part[block * nOwners * 6]; the owner update
+// folds nPart of them (PART_FROM_COUNTERS: the number of blocks of the guard's contact count).
+constexpr uint32_t PART_FROM_COUNTERS = 0xFFFFFFFFu;
+constexpr uint32_t MAX_ANAL_OWNERS = 8;
+struct PlaneSums {
+    float* part = nullptr;
+    uint32_t first = 0, nOwners = 0;  // owner numbers first .. first + nOwners - 1
+    uint32_t nPart = 0;
+};
+// What the owner update refreshes after moving the analytical owners: the poses of all nA components (pose null: none).
+struct PlaneRefresh {
+    const deme_anal_obj* anal = nullptr;
+    PlanePose* pose = nullptr;
+    uint32_t nA = 0;
+};
+
 // Device-side counters read back by the host after a detection pass.
 struct DevCounters {
     uint32_t pairCount;

@@ -54,10 +54,13 @@ constexpr uint64_t SCAN2_SMALL_N = 65536;
 constexpr uint64_t scan2_sums_elems(uint64_t n) {
     return 2 * ((n <= SCAN2_SMALL_N ? (n + SCAN_BLOCK - 1) / SCAN_BLOCK : (n + SCAN2_TILE - 1) / SCAN2_TILE) + 1);
 }
-constexpr uint32_t MAX_ANAL_OWNERS = 8;
-// Plane-owner sums: each workgroup of k_anal_collect folds one tile of ANAL_TILE contacts (256 lanes x ANAL_ITEMS)
-// into nAnalOwners x 6 partials, so the partials buffer holds anal_blocks(nC) x nAnalOwners x 6 floats.
-constexpr uint32_t ANAL_ITEMS = 4;
+using deme_dev::MAX_ANAL_OWNERS;
+using deme_dev::PART_FROM_COUNTERS;
+using deme_dev::PlaneRefresh;
+using deme_dev::PlaneSums;
+// Plane-owner sums: each workgroup of the force kernel folds its ANAL_TILE contacts (256 lanes x ANAL_ITEMS) into
+// nAnalOwners x 6 partials, so the partials buffer holds anal_blocks(nC) x nAnalOwners x 6 floats.
+constexpr uint32_t ANAL_ITEMS = 1;
 constexpr uint32_t ANAL_TILE = 256 * ANAL_ITEMS;
 inline uint32_t anal_blocks(uint64_t nC) { return (uint32_t)((nC + ANAL_TILE - 1) / ANAL_TILE); }
 
@@ -214,27 +217,20 @@ hipError_t launch_cand_tscatter(uint32_t nK, const uint32_t* candB, const uint32
 hipError_t launch_cand_tsort(uint32_t nS, const uint32_t* tStart, uint32_t* tC, uint32_t* tPos, hipStream_t st);
 
 // dyn.hip
-// aTerm / gTerm: 6 floats per contact; bTerm: 6 floats per mirror entry; out (optional): full contact records
+// aTerm: 6 floats per contact; bTerm: 6 floats per mirror entry; sums: the plane owners' partial sums, one set per
+// workgroup (anal_blocks(nC) of them); out (optional): full contact records
 hipError_t launch_force(const KParams& P, uint32_t nC, const uint32_t* idA, const uint32_t* idB, const uint8_t* ctype,
                         const SphereRec* sph, const OwnerRec* own, const float4* moi, const deme_anal_obj* anal,
                         const PlanePose* pose, const deme_material* mats, const float4* histIn, const uint32_t* map,
-                        float4* histOut, const uint32_t* mirror, float* aTerm, float* bTerm, float* gTerm,
-                        uint8_t* aOn, uint8_t* bOn,
+                        float4* histOut, const uint32_t* mirror, float* aTerm, float* bTerm,
+                        const PlaneSums& sums, uint8_t* aOn, uint8_t* bOn,
                         ForceRec* out, hipStream_t st, SpecGuard guard = SpecGuard());
-// blockPartials holds partialCap floats; a launch that would need more (anal_blocks(nC) * nAnalOwners * 6) returns
-// hipErrorInvalidValue and writes nothing. With a guard (a step captured with its detection pass) nC is the capacity
-// the grid covers and the kernels take the count from the pass's counters.
-hipError_t launch_anal_collect(uint32_t nC, const uint32_t* idB, const uint8_t* ctype, const float* gTerm,
-                               const deme_anal_obj* anal, uint32_t nA, uint32_t firstAnalOwner, uint32_t nAnalOwners,
-                               float* blockPartials, uint64_t partialCap, uint32_t* nBlocksOut, hipStream_t st,
-                               SpecGuard guard = SpecGuard());
-hipError_t launch_anal_final(const float* blockPartials, uint32_t nBlocks, uint32_t nAnalOwners, float* analAcc,
-                             hipStream_t st, SpecGuard guard = SpecGuard());
-hipError_t launch_owner_update(const KParams& P, uint32_t nO, uint32_t nClumps, uint32_t firstAnalOwner,
-                               uint32_t nAnalOwners, const uint32_t* ownerSphStart, const uint32_t* rowStart,
-                               const uint32_t* bRowStart, const float* aTerm, const float* bTerm,
-                               const uint8_t* aOn, const uint8_t* bOn,
-                               const float* analAcc, const deme_family_rule* rules, OwnerRec* own,
+// The owner update: nClumps clump owners and sums.nOwners analytical owners (numbered from sums.first). The first
+// workgroup folds the force kernel's partial sums, moves the analytical owners and refreshes the plane poses.
+hipError_t launch_owner_update(const KParams& P, uint32_t nO, uint32_t nClumps, const uint32_t* ownerSphStart,
+                               const uint32_t* rowStart, const uint32_t* bRowStart, const float* aTerm,
+                               const float* bTerm, const uint8_t* aOn, const uint8_t* bOn, const PlaneSums& sums,
+                               const PlaneRefresh& planes, const deme_family_rule* rules, OwnerRec* own,
                                float* acc /* 6 x nO SoA: aX aY aZ alX alY alZ */, int doIntegrate,
                                const double* clock /* device: the simulation time the motion rules read */,
                                hipStream_t st, OwnerRec* ownOut = nullptr /* integrated records; null: in place */,
@@ -249,6 +245,10 @@ hipError_t launch_fill_u32(uint32_t* p, uint64_t n, uint32_t v, hipStream_t st, 
 hipError_t launch_change_family(OwnerRec* own, uint32_t nO, uint8_t from, uint8_t to, hipStream_t st);
 
 // jit_rt.cpp: the force kernel specialised at run time by hipRTC
+// workgroups of the owner update: one for the analytical owners (when there are any), then 256 clumps each
+inline uint32_t owner_blocks(uint32_t nClumps, uint32_t nAnalOwners) {
+    return (nAnalOwners ? 1u : 0u) + (nClumps + 255) / 256;
+}
 struct JitForce {
     hipModule_t mod = nullptr;
     hipFunction_t full = nullptr, terms = nullptr;
@@ -258,7 +258,7 @@ struct JitForce {
                       const uint8_t* ctype, const SphereRec* sph, const OwnerRec* own, const float4* moi,
                       const deme_anal_obj* anal, const PlanePose* pose, const deme_material* mats,
                       const float4* histIn, const uint32_t* map, float4* histOut, const uint32_t* mirror,
-                      float* aTerm, float* bTerm, float* gTerm, uint8_t* aOn, uint8_t* bOn, ForceRec* out,
+                      float* aTerm, float* bTerm, const PlaneSums& sums, uint8_t* aOn, uint8_t* bOn, ForceRec* out,
                       hipStream_t st, SpecGuard guard = SpecGuard()) const;
 };
 // the owner update kernel specialised with motion strategies / family change rules
@@ -267,11 +267,10 @@ struct JitOwner {
     hipFunction_t fn = nullptr;
     void release();
     hipError_t load(const std::vector<char>& code);
-    hipError_t launch(const KParams& P, uint32_t nO, uint32_t nClumps, uint32_t firstAnal, uint32_t nAnalOwners,
-                      const uint32_t* ownerSphStart, const uint32_t* rowStart, const uint32_t* bRowStart,
-                      const float* aTerm, const float* bTerm, const uint8_t* aOn, const uint8_t* bOn,
-                      const float* analAcc, const deme_family_rule* rules,
-                      const OwnerRec* own, OwnerRec* ownOut, float* acc, int doIntegrate, const double* clock,
+    hipError_t launch(const KParams& P, uint32_t nO, uint32_t nClumps, const uint32_t* ownerSphStart,
+                      const uint32_t* rowStart, const uint32_t* bRowStart, const float* aTerm, const float* bTerm,
+                      const uint8_t* aOn, const uint8_t* bOn, const PlaneSums& sums, const PlaneRefresh& planes,
+                      const deme_family_rule* rules, const OwnerRec* own, OwnerRec* ownOut, float* acc, int doIntegrate, const double* clock,
                       hipStream_t st, SpecGuard guard = SpecGuard()) const;
 };
 std::string jit_owner_source(const std::vector<std::pair<std::string, std::string>>& values);

@@ -28,9 +28,9 @@ SPHERE_PLANE = 3
 NULL_MAP = 0xFFFFFFFF
 NUM_MASK_ENTRIES = 256 * 257 // 2
 NUM_FAMILIES = 256
-# contacts per workgroup tile of the plane-owner sums (ANAL_TILE in csrc/deme_internal.h): the sums write one set of
-# partials per tile
-ANAL_TILE = 1024
+# contacts per workgroup of the force kernel (ANAL_TILE in csrc/deme_internal.h): it writes one set of the plane
+# owners' partial sums
+ANAL_TILE = 256
 INTEGRATOR = {"forward_euler": 0, "centered_difference": 1, "extended_taylor": 2}
 
 

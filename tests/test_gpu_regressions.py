@@ -147,3 +147,47 @@ def test_prefix_scan_every_path_against_numpy():
             _scan_case(lib, h, n, rng)
     finally:
         lib.deme_ctx_destroy(h)
+
+
+@pytest.mark.parametrize("n", [1, 63, 255, 256, 257, 70_000])
+def test_plane_owner_sums_at_workgroup_edges(n):
+    """Spheres pressed into a floor and a slanted plane of two owners: the force kernel's partial sums (one set per 256
+    contacts) and the owner update's fold of them, at the edges of a workgroup and of the fold's 256 lanes, against the
+    oracle; a moved plane is seen by the next detection (the owner update refreshes the poses)."""
+    import pyoracle
+
+    side = int(np.ceil(np.sqrt(n)))
+    r = 0.002
+    k = np.arange(n)
+    xyz = np.stack([(k % side) * 2.2 * r, (k // side) * 2.2 * r, np.zeros(n)], 1)
+    L = max(side * 2.2 * r + 8 * r, 0.05)
+    xyz += np.array([-L / 2 + 4 * r, -L / 2 + 4 * r, -L / 2 + 0.95 * r])
+    sc = scenes.spheres_scene(xyz, r, (L, L, L))
+    extra = np.zeros(1, ANAL_DTYPE)
+    extra[0]["owner"] = n + 1
+    extra[0]["relPos"] = (0.0, 0.0, -L / 2 + 0.03 * r)
+    extra[0]["rot"] = (0.0, 0.0, 1.0)
+    extra[0]["mass"] = 1e15
+    sc.anal = np.concatenate([sc.anal, extra])
+    sc.state = {q: np.concatenate([v, v[n:n + 1]]) for q, v in sc.state.items()}
+    sc.state["family"][n + 1] = 0  # the second plane moves freely
+    sc.state["vZ"][n + 1] = -0.01
+    sc.n_owners = n + 2
+    sc.owner_mass = np.append(sc.owner_mass, np.float32(1e15))
+    sc.owner_moi = np.ascontiguousarray(np.append(sc.owner_moi, np.full((1, 3), 1e15, np.float32), 0))
+    dev, ora = DeviceSystem(sc), pyoracle.OracleSystem(sc)
+    for _ in range(3):
+        dev.step(1, 1)
+        ora.step(1, 1)
+        sd, so = dev.get_state(), ora.get_state()
+        for q in ("aX", "aY", "aZ", "alphaX", "alphaY"):
+            d, o = sd[q][n:].astype(np.float64), so[q][n:].astype(np.float64)
+            # sums of n float terms in another order: n ulps of the largest partial sum
+            bound = 1e-5 * np.abs(so["aZ"][n:]) * (L if q.startswith("alpha") else 1.0) + 1e-30
+            assert np.all(np.abs(d - o) <= bound), (q, d, o)
+        for q in ("voxelID", "locX", "locY", "locZ"):
+            assert np.array_equal(sd[q][n:], so[q][n:]), q
+    a, b = dev.contacts(), ora.contacts()
+    assert len(a[0]) >= 2 * n
+    for x, y in zip(a[:3], b[:3]):
+        assert np.array_equal(x, y)
