@@ -19,36 +19,10 @@ namespace deme_int {
 using namespace deme_dev;
 namespace {
 
-struct BinRange {
-    uint32_t x0, x1, y0, y1, z0, z1;
-};
-
-// DEMBinSphereKernels.cu:52-64 (double position and radius span, truncating conversions)
-__device__ __forceinline__ BinRange bin_range(const KParams& P, double X, double Y, double Z, double rCD) {
-    const double bx = X / P.binSize, by = Y / P.binSize, bz = Z / P.binSize, span = rCD / P.binSize;
-    BinRange r;
-    r.x0 = sat_u32(bx - span);
-    r.x1 = sat_u32(bx + span);
-    r.y0 = sat_u32(by - span);
-    r.y1 = sat_u32(by + span);
-    r.z0 = sat_u32(bz - span);
-    r.z1 = sat_u32(bz + span);
-    return r;
-}
-
 // getPointBinID<binID_t> (DEMHelperKernels.cu:266-273)
 __device__ __forceinline__ uint32_t point_bin(const KParams& P, double X, double Y, double Z) {
     const uint32_t ix = sat_u32(X / P.binSize), iy = sat_u32(Y / P.binSize), iz = sat_u32(Z / P.binSize);
     return ix + iy * P.nbX + iz * P.nbX * P.nbY;
-}
-
-// checkSphereEntityOverlap<double> without contact point (DEMHelperKernels.cu:356-391); rCD already holds r + beta.
-__device__ __forceinline__ bool plane_cd(const KParams& P, const PlanePose& pp, double X, double Y, double Z,
-                                         double rCD) {
-    if (pp.type != DEME_ANAL_OBJ_TYPE_PLANE) return false;
-    const double dx = X - pp.px, dy = Y - pp.py, dz = Z - pp.pz;
-    const double dist = dx * (double)pp.nx + dy * (double)pp.ny + dz * (double)pp.nz;
-    return !(dist > rCD + (double)P.beta);
 }
 
 __global__ __launch_bounds__(64) void k_plane_pose(KParams P, const deme_anal_obj* __restrict__ anal, uint32_t nA,

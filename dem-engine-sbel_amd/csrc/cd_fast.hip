@@ -17,46 +17,6 @@ namespace deme_int {
 using namespace deme_dev;
 namespace {
 
-struct BinRange {
-    uint32_t x0, x1, y0, y1, z0, z1;
-};
-
-__device__ __forceinline__ BinRange bin_range(const KParams& P, double X, double Y, double Z, double rCD) {
-    const double bx = X / P.binSize, by = Y / P.binSize, bz = Z / P.binSize, span = rCD / P.binSize;
-    BinRange r;
-    r.x0 = sat_u32(bx - span);
-    r.x1 = sat_u32(bx + span);
-    r.y0 = sat_u32(by - span);
-    r.y1 = sat_u32(by + span);
-    r.z0 = sat_u32(bz - span);
-    r.z1 = sat_u32(bz + span);
-    return r;
-}
-
-__device__ __forceinline__ bool plane_cd(const KParams& P, const PlanePose& pp, double X, double Y, double Z,
-                                         double rCD) {
-    if (pp.type != DEME_ANAL_OBJ_TYPE_PLANE) return false;
-    const double dx = X - pp.px, dy = Y - pp.py, dz = Z - pp.pz;
-    const double dist = dx * (double)pp.nx + dy * (double)pp.ny + dz * (double)pp.nz;
-    return !(dist > rCD + (double)P.beta);
-}
-
-__device__ __forceinline__ bool range_in_grid(const KParams& P, const BinRange& r) {
-    return r.x1 < P.nbX && r.y1 < P.nbY && r.z1 < P.nbZ;
-}
-
-// Membership of a linear bin id in the linear ids of a range (the reference's bins may alias when a range crosses
-// the grid's upper faces; this enumerates exactly the ids the reference would form).
-// (Out of line: the rare path. Arguments by value, so the caller's ranges stay in registers.)
-__device__ __noinline__ bool range_has_linear(uint32_t nbX, uint32_t nbY, BinRange r, uint32_t lin) {
-    const uint32_t nbXY = nbX * nbY;
-    for (uint32_t k = 0; k <= r.z1 - r.z0; k++)
-        for (uint32_t j = 0; j <= r.y1 - r.y0; j++)
-            for (uint32_t i = 0; i <= r.x1 - r.x0; i++)
-                if ((r.x0 + i) + (r.y0 + j) * nbX + (r.z0 + k) * nbXY == lin) return true;
-    return false;
-}
-
 // Cell of a position, clamped to the cell grid (positions outside the world collapse onto edge cells, which only
 // adds candidates).
 __device__ __forceinline__ void cell_of(const CellGrid& G, double X, double Y, double Z, int& cx, int& cy, int& cz) {
@@ -104,23 +64,8 @@ __device__ __forceinline__ void sphere_detect(const KParams& P, const SphereRec&
     const BinRange r = bin_range(P, X, Y, Z, rCD);
     const uint32_t nx = r.x1 - r.x0 + 1, ny = r.y1 - r.y0 + 1, nz = r.z1 - r.z0 + 1;
     if (numBins) numBins[s] = (uint16_t)((int)(uint16_t)nx * (int)(uint16_t)ny * (int)(uint16_t)nz);
-    if ((uint64_t)nx * ny * nz > 65535u) {
-        atomicOr(&ctr->err, ERRBIT_CAPACITY);
-    } else {
-        // The linear id grows with each of i, j, k, so without 32-bit wrap the range's largest id is its last corner.
-        const uint32_t nbXY = P.nbX * P.nbY;
-        const uint64_t last = (uint64_t)r.x1 + (uint64_t)r.y1 * P.nbX + (uint64_t)r.z1 * nbXY;
-        bool outside = last >= P.nBins;
-        if (last > 0xFFFFFFFFull) {
-            // ids wrap: enumerate them as the reference forms them
-            outside = false;
-            for (uint32_t dk = 0; dk < nz; dk++)
-                for (uint32_t dj = 0; dj < ny; dj++)
-                    for (uint32_t di = 0; di < nx; di++)
-                        outside |= ((r.x0 + di) + (r.y0 + dj) * P.nbX + (r.z0 + dk) * nbXY) >= P.nBins;
-        }
-        if (outside) atomicOr(&ctr->err, ERRBIT_OUTSIDE);
-    }
+    const uint32_t bad = bin_range_err(P, r);
+    if (bad) atomicOr(&ctr->err, bad);
     uint32_t cnt = 0;
     unsigned long long bits = 0;  // bit k: component a0 + k of the sphere's scene
     uint32_t a0, a1;
@@ -258,134 +203,6 @@ __global__ __launch_bounds__(256) void k_cell_scatter(KParams P, const SphereRec
         rf += beta;
         sortedF[pos] = make_float4((float)cr.x, (float)cr.y, (float)cr.z, rf);
     }
-}
-
-// Expanded radius as the reference's detection kernel forms it: float(r + beta), widened to double.
-__device__ __forceinline__ double expanded_radius(const KParams& P, float r) {
-    float rf = r;
-    rf += P.beta;
-    return (double)rf;
-}
-
-// First half of the reference's sphere-pair test (checkSpheresOverlap<double>, DEMHelperKernels.cu:195-205): the
-// expanded spheres overlap.
-__device__ __forceinline__ bool expanded_overlap(double ra, const CdRec& A, double rb, const CdRec& B) {
-    const double dx = A.x - B.x, dy = A.y - B.y, dz = A.z - B.z;
-    const double d2 = dx * dx + dy * dy + dz * dz;
-    return !(d2 > (ra + rb) * (ra + rb));
-}
-
-// Second half, for a pair that overlaps: the contact point (DEMHelperKernels.cu:206-222) computed with A the lower id,
-// and its bin inside both spheres' AABB bin ranges.
-struct RuleBins {
-    uint32_t ix, iy, iz;
-    BinRange ga, gb;
-};
-
-__device__ __forceinline__ void contact_point(const KParams& P, const CdRec& A, const CdRec& B, double& cx, double& cy,
-                                              double& cz) {
-    const double ra = expanded_radius(P, A.r), rb = expanded_radius(P, B.r);
-    const double dx = A.x - B.x, dy = A.y - B.y, dz = A.z - B.z;
-    const double d2 = dx * dx + dy * dy + dz * dz;
-    float nX = (float)dx, nY = (float)dy, nZ = (float)dz;
-    const float mag = sqrtf(nX * nX + nY * nY + nZ * nZ);
-    nX /= mag;
-    nY /= mag;
-    nZ /= mag;
-    const double half = (ra + rb - sqrt(d2)) / 2.0;
-    cx = B.x + (rb - half) * (double)nX;
-    cy = B.y + (rb - half) * (double)nY;
-    cz = B.z + (rb - half) * (double)nZ;
-}
-
-__device__ __forceinline__ double cd_radius(const KParams& P, float r) {
-    double v = (double)r;
-    v += (double)P.beta;
-    return v;
-}
-
-// The reference's bin indices, with its divisions by binSize.
-__device__ __forceinline__ void rule_bins_exact(const KParams& P, const CdRec& A, const CdRec& B, double cx, double cy,
-                                                double cz, RuleBins& R) {
-    R.ix = sat_u32(cx / P.binSize);
-    R.iy = sat_u32(cy / P.binSize);
-    R.iz = sat_u32(cz / P.binSize);
-    R.ga = bin_range(P, A.x, A.y, A.z, cd_radius(P, A.r));
-    R.gb = bin_range(P, B.x, B.y, B.z, cd_radius(P, B.r));
-}
-
-// The same bin indices from multiplications by the reciprocal of the bin size, used when every floor input lies
-// farther from an integer than the product and the quotient can differ (a few ulps; the margin is 2^-40 relative):
-// then each floor, and so the rule, equals the division's. Returns false when a value is too close to call.
-__device__ __forceinline__ bool far_from_int(double t, double scale) {
-    const double f = t - floor(t);
-    const double eps = 0x1p-40 * (scale + 1.0);
-    return f > eps && f < 1.0 - eps;
-}
-
-__device__ __forceinline__ bool range_fast(const KParams& P, double inv, double X, double Y, double Z, double rCD,
-                                           BinRange& r) {
-    const double bx = X * inv, by = Y * inv, bz = Z * inv, span = rCD * inv;
-    const double ax = fabs(bx) + span, ay = fabs(by) + span, az = fabs(bz) + span;
-    const double x0 = bx - span, x1 = bx + span, y0 = by - span, y1 = by + span, z0 = bz - span, z1 = bz + span;
-    if (!(far_from_int(x0, ax) && far_from_int(x1, ax) && far_from_int(y0, ay) && far_from_int(y1, ay) &&
-          far_from_int(z0, az) && far_from_int(z1, az)))
-        return false;
-    r.x0 = sat_u32(x0);
-    r.x1 = sat_u32(x1);
-    r.y0 = sat_u32(y0);
-    r.y1 = sat_u32(y1);
-    r.z0 = sat_u32(z0);
-    r.z1 = sat_u32(z1);
-    return true;
-}
-
-__device__ __forceinline__ bool rule_bins_fast(const KParams& P, double inv, const CdRec& A, const CdRec& B, double cx,
-                                               double cy, double cz, RuleBins& R) {
-    const double qx = cx * inv, qy = cy * inv, qz = cz * inv;
-    if (!(far_from_int(qx, fabs(qx)) && far_from_int(qy, fabs(qy)) && far_from_int(qz, fabs(qz)))) return false;
-    R.ix = sat_u32(qx);
-    R.iy = sat_u32(qy);
-    R.iz = sat_u32(qz);
-    return range_fast(P, inv, A.x, A.y, A.z, cd_radius(P, A.r), R.ga) &&
-           range_fast(P, inv, B.x, B.y, B.z, cd_radius(P, B.r), R.gb);
-}
-
-__device__ __forceinline__ bool rule_member(const KParams& P, const RuleBins& R) {
-    if (range_in_grid(P, R.ga) && range_in_grid(P, R.gb)) {
-        // no aliasing: a linear id is one (i, j, k) -- unless the point itself lies past the grid, where the
-        // reference's linear id aliases; fall through to the exact enumeration then
-        if (R.ix < P.nbX && R.iy < P.nbY && R.iz < P.nbZ)
-            return R.ix >= R.ga.x0 && R.ix <= R.ga.x1 && R.iy >= R.ga.y0 && R.iy <= R.ga.y1 && R.iz >= R.ga.z0 &&
-                   R.iz <= R.ga.z1 && R.ix >= R.gb.x0 && R.ix <= R.gb.x1 && R.iy >= R.gb.y0 && R.iy <= R.gb.y1 &&
-                   R.iz >= R.gb.z0 && R.iz <= R.gb.z1;
-    }
-    const uint32_t lin = R.ix + R.iy * P.nbX + R.iz * P.nbX * P.nbY;
-    return range_has_linear(P.nbX, P.nbY, R.ga, lin) && range_has_linear(P.nbX, P.nbY, R.gb, lin);
-}
-
-// True only when the bin rule of an overlapping pair must hold. The exact contact point lies inside both expanded
-// spheres, ra - half from A's centre and rb - half from B's (half: half the overlap, at most the smaller radius), so its
-// bin lies in both spheres' bin ranges as soon as half exceeds what rounding can move: the float-rounded direction
-// moves the point by under 6e-7 (ra + rb), float(r + beta) differs from r + beta by under 6e-8 (ra + rb), and the
-// double positions and quotients add a few 2^-52 of the coordinates. Floors and saturation are monotone, and a triple
-// inside both ranges is among the linear ids of both, so the aliasing cases agree. Everything else (grazing pairs,
-// near-coincident centres, one sphere deep inside another, NaN) answers false and takes the full rule.
-__device__ __forceinline__ bool bin_rule_certain(double ra, const CdRec& A, double rb, const CdRec& B) {
-    const double dx = A.x - B.x, dy = A.y - B.y, dz = A.z - B.z;
-    const double sum = ra + rb, dist = sqrt(dx * dx + dy * dy + dz * dz), half = 0.5 * (sum - dist);
-    const double reach = fabs(A.x) + fabs(A.y) + fabs(A.z) + sum;
-    return half > 1e-6 * sum + 0x1p-46 * reach && half <= fmin(ra, rb) && dist > 1e-3 * sum && sum > 1e-12;
-}
-
-// A: the lower id of an overlapping pair. inv: 1 / binSize.
-__device__ __forceinline__ bool bin_rule_point(const KParams& P, double inv, const CdRec& A, const CdRec& B) {
-    if (bin_rule_certain(expanded_radius(P, A.r), A, expanded_radius(P, B.r), B)) return true;
-    double cx, cy, cz;
-    contact_point(P, A, B, cx, cy, cz);
-    RuleBins R;
-    if (!rule_bins_fast(P, inv, A, B, cx, cy, cz, R)) rule_bins_exact(P, A, B, cx, cy, cz, R);
-    return rule_member(P, R);
 }
 
 // One lane per sphere in cell order, half-shell: each lane pairs its sphere with the later spheres of its own cell

@@ -169,6 +169,21 @@ struct deme_ctx {
         // every pass stale: the cell sweep runs instead
         return 0.5 * s > SKIN_SLACK + 4.0 * posUnit ? s : 0.0;
     }
+    // Stepping on the candidates (direct.hip): the status, the candidates' histories and the plane candidates with their
+    // rows, flags, histories and terms; the old build's during a rebuild. The pairs' flags are candAcc[cur].
+    // planesGen: the build (candBuilds) the plane candidates go with. directSkip: calls of deme_step that do not try
+    // (after a state near the grid's end, doubling up to 64 while that repeats).
+    DBuf<DirectState> dstate;
+    DirectState* hdstate = nullptr;  // pinned mirror
+    DBuf<float4> dHist, dHistOld, dPHist, dPHistOld;
+    DBuf<uint8_t> dPOn, dPOnOld, dOnOld;
+    DBuf<uint32_t> pStart, pStartOld, pSph, pPlane, pPlaneOld, candStartOld, candBOld;
+    DBuf<float> pTerm;
+    DBuf<unsigned long long> nearBits;
+    DBuf<PlanePose> pose0;
+    uint32_t nPlane = 0;
+    uint64_t planesGen = 0;
+    uint32_t directSkip = 0, directBackoff = 0;
     int pairMode = -1;  // pair sweep mode (launch_cell_pairs); -1: chosen from the radius spread
     uint32_t pairBlock = 256;  // pair sweep workgroup size
     double cycleHeadroom = 1.25;  // capacity of a captured interval: headroom x the current counts + slack
@@ -464,8 +479,10 @@ int deme_ctx_create(int device, void* stream, deme_ctx** out) {
         c->ownStream = true;
     }
     if (c->ctr.ensure(1, 1.0) != hipSuccess || c->clock.ensure(1, 1.0) != hipSuccess ||
-        hipHostMalloc((void**)&c->hctr, sizeof(DevCounters), hipHostMallocDefault) != hipSuccess) {
-        delete c;
+        c->dstate.ensure(1, 1.0) != hipSuccess ||
+        hipHostMalloc((void**)&c->hctr, sizeof(DevCounters), hipHostMallocDefault) != hipSuccess ||
+        hipHostMalloc((void**)&c->hdstate, sizeof(DirectState), hipHostMallocDefault) != hipSuccess) {
+        deme_ctx_destroy(c);
         return DEME_ERR_HIP;
     }
     std::memset(c->hctr, 0, sizeof(DevCounters));
@@ -524,6 +541,11 @@ int deme_ctx_destroy(deme_ctx* c) {
     if (c->stepExec) (void)hipGraphExecDestroy(c->stepExec);
     for (auto& cy : c->cycle)
         if (cy.exec) (void)hipGraphExecDestroy(cy.exec);
+    c->dstate.release(); c->dHist.release(); c->dHistOld.release(); c->dPHist.release(); c->dPHistOld.release();
+    c->dPOn.release(); c->dPOnOld.release(); c->dOnOld.release(); c->pStart.release(); c->pStartOld.release();
+    c->pSph.release(); c->pPlane.release(); c->pPlaneOld.release(); c->candStartOld.release(); c->candBOld.release();
+    c->pTerm.release(); c->nearBits.release(); c->pose0.release();
+    if (c->hdstate) (void)hipHostFree(c->hdstate);
     if (c->hctr) (void)hipHostFree(c->hctr);
     if (c->evCounts) (void)hipEventDestroy(c->evCounts);
     if (c->ownStream) (void)hipStreamDestroy(c->stream);
@@ -684,6 +706,7 @@ int deme_upload_materials(deme_ctx* c, uint32_t n, const deme_material* m) {
 }
 
 int deme_upload_analytical(deme_ctx* c, uint32_t n, const deme_anal_obj* objs) {
+    c->planesGen = 0;
     c->posesValid = false;
     c->graphGen++;
     c->adjReady = false;  // recorded adjoint checkpoints no longer describe the system
@@ -1274,6 +1297,30 @@ static int skin_buffers(deme_ctx* c) {
     return DEME_OK;
 }
 
+// The row and mirror-row scans of the touching candidates (candAcc[cu]) and plane contacts (numAnal), totals in the
+// device counters.
+static int enqueue_row_scans(deme_ctx* c, int cu) {
+    const uint32_t nS = c->nS;
+    if ((uint64_t)nS <= SCAN2_TILE * SCAN_TILE) {
+        // the row counts formed inside the scan's first pass
+        DEME_LAUNCH(c, "scan_rows",
+                    scan2_cand_rows(c->candStart.p, c->tStart.p, c->tC.p, c->candAcc[cu].p, c->numAnal.p, nS,
+                                    c->tRank.p, c->rowStart[cu].p, c->bRowStart.p, &c->ctr.p->total[1], &c->ctr.p->total[2],
+                                    c->scanTmp.p, c->scan2Sums.p, c->ctr.p, c->stream));
+    } else {
+        DEME_LAUNCH(c, "cand_count",
+                    launch_cand_count(nS, c->candStart.p, c->tStart.p, c->tC.p, c->candAcc[cu].p, c->aCnt.p,
+                                      c->bCnt.p, c->tRank.p, c->ctr.p, c->stream));
+        DEME_LAUNCH(c, "scan_rows",
+                    scan_u32(c->aCnt.p, c->numAnal.p, nS, c->rowStart[cu].p, &c->ctr.p->total[1], c->scanScratch.p,
+                             c->stream));
+        DEME_LAUNCH(c, "scan_brows",
+                    scan_u32(c->bCnt.p, nullptr, nS, c->bRowStart.p, &c->ctr.p->total[2], c->scanScratch.p,
+                             c->stream));
+    }
+    return DEME_OK;
+}
+
 // One candidate-list pass up to the row scans: plane poses, counters cleared, per-sphere positions (with the
 // displacement since the build), the predicate on the candidates (touching flags, row counts), the mirror-row
 // counts, the row and mirror-row scans.
@@ -1294,24 +1341,7 @@ static int enqueue_skin_pass(deme_ctx* c, int cu) {
                 launch_cand_flags(c->kp, (uint32_t)c->nCand, c->pos.p, c->meta.p, c->candA.p, c->candB.p,
                                   c->maskAny ? c->mask.p : nullptr, stale_limit2(c), c->candAcc[cu].p, c->ctr.p,
                                   c->dispRef.p + 3 * cu, c->stream));
-    if ((uint64_t)nS <= SCAN2_TILE * SCAN_TILE) {
-        // the row counts formed inside the scan's first pass
-        DEME_LAUNCH(c, "scan_rows",
-                    scan2_cand_rows(c->candStart.p, c->tStart.p, c->tC.p, c->candAcc[cu].p, c->numAnal.p, nS,
-                                    c->tRank.p, c->rowStart[cu].p, c->bRowStart.p, &c->ctr.p->total[1], &c->ctr.p->total[2],
-                                    c->scanTmp.p, c->scan2Sums.p, c->ctr.p, c->stream));
-    } else {
-        DEME_LAUNCH(c, "cand_count",
-                    launch_cand_count(nS, c->candStart.p, c->tStart.p, c->tC.p, c->candAcc[cu].p, c->aCnt.p,
-                                      c->bCnt.p, c->tRank.p, c->ctr.p, c->stream));
-        DEME_LAUNCH(c, "scan_rows",
-                    scan_u32(c->aCnt.p, c->numAnal.p, nS, c->rowStart[cu].p, &c->ctr.p->total[1], c->scanScratch.p,
-                             c->stream));
-        DEME_LAUNCH(c, "scan_brows",
-                    scan_u32(c->bCnt.p, nullptr, nS, c->bRowStart.p, &c->ctr.p->total[2], c->scanScratch.p,
-                             c->stream));
-    }
-    return DEME_OK;
+    return enqueue_row_scans(c, cu);
 }
 
 // Bookkeeping at the end of a detection pass (candidate-list or cell sweep; disp2: the largest squared displacement
@@ -1903,12 +1933,319 @@ static int run_cycle(deme_ctx* c, int f, bool* done) {
     return DEME_OK;
 }
 
+// ---- stepping on the candidates (direct.hip) ----
+static DirectList direct_list(const deme_ctx* c) {
+    DirectList d{};
+    d.nPair = (uint32_t)c->nCand;
+    d.nPlane = c->nPlane;
+    d.candA = c->candA.p;
+    d.candB = c->candB.p;
+    d.tPos = c->tPos.p;
+    d.pSph = c->pSph.p;
+    d.pPlane = c->pPlane.p;
+    d.pStart = c->pStart.p;
+    d.on = c->candAcc[c->cur].p;
+    d.pOn = c->dPOn.p;
+    d.bOn = c->bOn.p;
+    d.hist = c->dHist.p;
+    d.pHist = c->dPHist.p;
+    d.pTerm = c->pTerm.p;
+    d.mask = c->maskAny ? c->mask.p : nullptr;
+    d.st = c->dstate.p;
+    return d;
+}
+
+// Spheres are listed for a plane within 1.5 skins of it. Both now and later their displacement since the build stays
+// within half a skin, so they moved at most one skin in between; the planes themselves may move by the rest (less a
+// tenth for rounding).
+constexpr double PLANE_MARGIN = 1.5, PLANE_MOTION = 0.45;
+
+static DirectCheck direct_check(const deme_ctx* c) {
+    DirectCheck k{};
+    k.sph = c->sph.p;
+    k.pos0 = c->pos0.p;
+    k.unit = c->posUnit;
+    k.limit2 = stale_limit2(c);
+    const double rmax = (double)c->maxRadius, bs = c->sp.binSize;
+    // a contact point strays from its spheres by under 1e-6 of the radii: limits a hundred times that below the end
+    auto hi = [&](uint32_t nb) { return (double)nb * bs * (1.0 - 1e-12) - 1e-4 * rmax; };
+    const double span = 2.0 * (rmax + (double)c->sp.beta) / bs + 2.0;
+    const bool fits = span * span * span <= 65535.0;
+    k.hiX = fits ? hi(c->sp.nbX) : -INFINITY;
+    k.hiY = fits ? hi(c->sp.nbY) : -INFINITY;
+    k.hiZ = fits ? hi(c->sp.nbZ) : -INFINITY;
+    k.pose0 = c->pose0.p;
+    k.planeLimit = PLANE_MOTION * c->skin();
+    k.reach = ((double)c->sp.nbX + c->sp.nbY + c->sp.nbZ) * bs;
+    return k;
+}
+
+static int direct_clear_state(deme_ctx* c) {
+    static_assert(sizeof(DirectState) % 4 == 0, "the status is cleared as 32-bit words");
+    DEME_LAUNCH(c, "fill", launch_fill_u32(reinterpret_cast<uint32_t*>(c->dstate.p), sizeof(DirectState) / 4, 0,
+                                           c->stream));
+    return DEME_OK;
+}
+
+// The plane candidates of the current state and the buffers of both kinds of candidates.
+static int direct_planes(deme_ctx* c) {
+    const uint32_t nS = c->nS;
+    int r = ensure_poses(c);
+    if (r) return r;
+    if (c->planesGen != c->candBuilds) {
+        DEME_HIP(c, c->nearBits.ensure(nS));
+        DEME_HIP(c, c->aCnt.ensure(nS));
+        DEME_HIP(c, c->pStart.ensure((size_t)nS + 1));
+        DEME_HIP(c, c->pose0.ensure(std::max<uint32_t>(c->nA, 1)));
+        DEME_LAUNCH(c, "direct_near", launch_direct_near(c->kp, c->sph.p, c->own.p, nS, c->pose.p, c->nA,
+                                                         PLANE_MARGIN * c->skin(), c->nearBits.p, c->aCnt.p, c->stream));
+        DEME_LAUNCH(c, "direct_scan", scan_u32(c->aCnt.p, nullptr, nS, c->pStart.p, &c->ctr.p->total[2],
+                                               c->scanScratch.p, c->stream));
+        if ((r = readback_counters(c))) return r;
+        const uint64_t n = c->hctr->total[2];
+        if (n > 0xFFFFFFFFull) return c->fail(DEME_ERR_CAPACITY, "plane candidate count exceeds 2^32 - 1");
+        c->nPlane = (uint32_t)n;
+        const size_t np = std::max<size_t>(n, 1);
+        DEME_HIP(c, c->pSph.ensure(np));
+        DEME_HIP(c, c->pPlane.ensure(np));
+        DEME_LAUNCH(c, "direct_plane_rows",
+                    launch_direct_plane_rows(c->kp, c->sph.p, c->own.p, nS, c->nearBits.p, c->pStart.p, c->pSph.p,
+                                             c->pPlane.p, c->pose.p, c->nA, c->pose0.p, c->stream));
+        c->planesGen = c->candBuilds;
+    }
+    const size_t nK = std::max<size_t>(c->nCand, 1), nP = std::max<size_t>(c->nPlane, 1);
+    DEME_HIP(c, c->dPOn.ensure(nP));
+    DEME_HIP(c, c->dPHist.ensure(nP));
+    DEME_HIP(c, c->pTerm.ensure(6 * nP));
+    DEME_HIP(c, c->dHist.ensure(nK));
+    DEME_HIP(c, c->aTerm.ensure(6 * nK));
+    DEME_HIP(c, c->bTerm.ensure(6 * nK));
+    DEME_HIP(c, c->bOn.ensure(nK));
+    DEME_HIP(c, ensure_partials(c, nP));
+    return DEME_OK;
+}
+
+// The contact list's histories to the candidates, and the check of the current state.
+static int direct_enter(deme_ctx* c) {
+    int r = direct_planes(c);
+    if (r) return r;
+    if ((r = direct_clear_state(c))) return r;
+    const int cu = c->cur;
+    DEME_LAUNCH(c, "direct_enter", launch_direct_enter(direct_list(c), c->cidx[cu].p, c->rowStart[cu].p, c->idB[cu].p,
+                                                       c->ctype[cu].p, c->hist[cu].p, c->stream));
+    DEME_LAUNCH(c, "direct_check", launch_direct_check(c->kp, direct_check(c), c->own.p, c->nS, c->pose.p, c->nA,
+                                                       c->dstate.p, c->stream));
+    return DEME_OK;
+}
+
+// New candidates from the current state, with the flags and histories of the old ones carried over.
+static int direct_rebuild(deme_ctx* c) {
+    const DirectList old = direct_list(c);
+    const int cu = c->cur;
+    std::swap(c->candStart, c->candStartOld);
+    std::swap(c->candB, c->candBOld);
+    std::swap(c->candAcc[cu], c->dOnOld);
+    std::swap(c->dHist, c->dHistOld);
+    std::swap(c->pStart, c->pStartOld);
+    std::swap(c->pPlane, c->pPlaneOld);
+    std::swap(c->dPOn, c->dPOnOld);
+    std::swap(c->dPHist, c->dPHistOld);
+    int r = build_candidates(c);
+    if (r) return r;
+    c->builtThisPass = false;  // (no pass's)
+    if ((r = direct_planes(c))) return r;
+    DEME_LAUNCH(c, "direct_join",
+                launch_direct_join(c->nS, c->candStartOld.p, c->candBOld.p, c->candStart.p, c->candB.p, c->pStartOld.p,
+                                   c->pPlaneOld.p, old, direct_list(c), c->stream));
+    return direct_clear_state(c);
+}
+
+// The contact list of the last step taken on the candidates, in place of the list it was entered with: the rows of the
+// touching candidates with their histories, as that step's own pass would have left them (the next pass maps against
+// it; the map of this list itself is not formed, since a pass always follows).
+static int direct_leave(deme_ctx* c) {
+    const DirectList d = direct_list(c);
+    const int cu = c->cur;
+    const uint32_t nS = c->nS;
+    int r = skin_buffers(c);
+    if (r) return r;
+    SpecGuard g;
+    for (int attempt = 0;; attempt++) {
+        DEME_LAUNCH(c, "direct_plane_bits",
+                    launch_direct_plane_bits(c->kp, c->sph.p, c->own.p, nS, d, c->numAnal.p, c->planeBits.p,
+                                             reinterpret_cast<uint32_t*>(c->ctr.p), sizeof(DevCounters) / 4,
+                                             c->stream));
+        if ((r = enqueue_row_scans(c, cu))) return r;
+        DEME_HIP(c, hipMemcpyAsync(c->hctr, c->ctr.p, DEV_COUNTERS_HOST_BYTES, hipMemcpyDeviceToHost, c->stream));
+        DEME_HIP(c, hipEventRecord(c->evCounts, c->stream));
+        // (enqueued before the totals are known, and skipped on the device if they outgrow the buffers)
+        g.ctr = c->ctr.p;
+        g.slabCap = c->slabCap;
+        g.capC = std::min({c->idB[cu].cap, c->ctype[cu].cap, c->hist[cu].cap, c->idA.cap, c->map.cap, c->mirror.cap});
+        g.capP = ~0ull;
+        DEME_LAUNCH(c, "cand_fill",
+                    launch_cand_fill(d.nPair, c->candA.p, c->candB.p, c->candStart.p, d.on, c->rowStart[cu].p,
+                                     c->numAnal.p, c->tPos.p, c->tRank.p, c->bRowStart.p, nullptr, nullptr,
+                                     c->cidx[cu].p, c->idA.p, c->idB[cu].p, c->ctype[cu].p, c->map.p, c->mirror.p,
+                                     c->stream, g));
+        DEME_LAUNCH(c, "cand_planes",
+                    launch_cand_planes(c->kp, c->sph.p, c->own.p, nS, c->rowStart[cu].p, c->planeBits.p, nullptr,
+                                       nullptr, nullptr, false, c->idA.p, c->idB[cu].p, c->ctype[cu].p, c->map.p,
+                                       c->mirror.p, c->stream, g));
+        DEME_LAUNCH(c, "direct_leave",
+                    launch_direct_leave(d, c->cidx[cu].p, c->rowStart[cu].p, c->hist[cu].p, c->stream, g));
+        DEME_HIP(c, hipEventSynchronize(c->evCounts));
+        const uint64_t C = c->hctr->total[1], nPairs = c->hctr->total[2];
+        if (C > 0xFFFFFFFFull) return c->fail(DEME_ERR_CAPACITY, "contact count exceeds contactPairs_t (2^32 - 1)");
+        if (nPairs > C) return c->fail(DEME_ERR_HIP, "inconsistent contact and mirror-row counts");
+        c->C = C;
+        c->nPairs = nPairs;
+        c->nGeo = C - nPairs;
+        if (C <= g.capC) break;
+        if (attempt) return c->fail(DEME_ERR_CAPACITY, "contact list could not be sized");
+        DEME_HIP(c, c->idB[cu].ensure(C));
+        DEME_HIP(c, c->ctype[cu].ensure(C));
+        DEME_HIP(c, c->hist[cu].ensure(C));
+        DEME_HIP(c, c->idA.ensure(C));
+        DEME_HIP(c, c->map.ensure(C));
+        DEME_HIP(c, c->mirror.ensure(C));
+    }
+    c->cidxGen[cu] = c->candBuilds;
+    c->contactsReady = true;
+    c->fresh = c->forcesFull = c->termsReady = false;
+    return DEME_OK;
+}
+
+// Whether the next steps may run on the candidates: detection every step, no drift margin (a list with a margin holds
+// pairs that do not touch, which only a pass lists), and the current list and its histories index the lists in force.
+static bool direct_ready(const deme_ctx* c) {
+    return !(c->sp.beta > 0.f) && c->contactsReady && !c->fresh && !c->needDetect && c->nS > 0 && c->skin() > 0.0 &&
+           c->candValid && c->cidxGen[c->cur] == c->candBuilds;
+}
+
+// Up to n steps on the candidates, in batches the host enqueues without waiting: a batch whose state fails the check
+// part-way leaves the rest of its kernels skipped, and the count of steps done comes back with its status. *done: steps
+// taken; *again: the lists were kept or rebuilt to the end (else the caller goes on with passes).
+static int run_direct(deme_ctx* c, int n, int* done, bool* again) {
+    *done = 0;
+    *again = true;
+    int r = 0;
+    if (c->jitActive && c->jitStale && (r = jit_rebuild(c))) return r;
+    if ((r = direct_enter(c))) return r;
+    bool rebuilt = false, giveUp = false;
+    double dispMax2 = 0.0;
+    uint32_t counted = 0;
+    while (*done < n) {
+        // steps expected before the lists go stale: by the displacement so far, else by the last lists' lifetime
+        const DirectCheck check = direct_check(c);
+        const double m = (double)c->passesSinceBuild, frac = std::max(std::sqrt(dispMax2 / check.limit2), 0.125);
+        double expect = m > 0 ? m / frac - m : (c->lastLifetime < 1000 ? (double)c->lastLifetime : 8.0);
+        const int batch = std::min(n - *done, (int)std::min(std::max(0.9 * expect, 2.0), 32.0));
+        const DirectList d = direct_list(c);
+        PlaneSums sums = plane_sums(c);
+        sums.nPart = (c->nPlane + 255) / 256;
+        const PlaneRefresh planes = plane_refresh(c);
+        double t = c->time;
+        for (int k = 0; k < batch; k++) {
+            DEME_LAUNCH(c, "force",
+                        c->jitActive
+                            ? c->jit.launch_direct(c->kp, d, c->sph.p, c->own.p, c->moi.p, c->anal.p, c->pose.p,
+                                                   c->mats.p, c->aTerm.p, c->bTerm.p, sums, c->stream)
+                            : launch_force_direct(c->kp, d, c->sph.p, c->own.p, c->moi.p, c->anal.p, c->pose.p,
+                                                  c->mats.p, c->aTerm.p, c->bTerm.p, sums, c->stream));
+            if (c->ownerJitActive) DEME_LAUNCH(c, "set_clock", launch_set_clock(c->clock.p, t, c->stream));
+            t += (double)c->sp.h;
+            DEME_LAUNCH(c, "owner_update",
+                        c->ownerJitActive
+                            ? c->jitOwner.launch(c->kp, c->nO, c->nClumps, c->ownerSphStart.p, c->candStart.p,
+                                                 c->tStart.p, c->aTerm.p, c->bTerm.p, d.on, d.bOn, sums, planes,
+                                                 c->rules.p, c->own.p, c->own.p, c->acc.p, 1, c->clock.p, c->stream,
+                                                 SpecGuard(), d, check)
+                            : launch_owner_update(c->kp, c->nO, c->nClumps, c->ownerSphStart.p, c->candStart.p,
+                                                  c->tStart.p, c->aTerm.p, c->bTerm.p, d.on, d.bOn, sums, planes,
+                                                  c->rules.p, c->own.p, c->acc.p, 1, c->clock.p, c->stream, nullptr,
+                                                  SpecGuard(), d, check));
+        }
+        DEME_HIP(c, hipMemcpyAsync(c->hdstate, c->dstate.p, sizeof(DirectState), hipMemcpyDeviceToHost, c->stream));
+        DEME_HIP(c, hipStreamSynchronize(c->stream));
+        const uint32_t steps = c->hdstate->steps - counted, err = c->hdstate->err;
+        counted = c->hdstate->steps;
+        for (uint32_t k = 0; k < steps; k++) {
+            c->time += (double)c->sp.h;
+            c->nSteps++;
+        }
+        *done += (int)steps;
+        c->passesSinceBuild += steps;
+        if (c->passesSinceBuild >= 4) c->cellBackoff = 0;
+        dispMax2 = 0.0;
+        for (unsigned long long b : c->hdstate->disp2) {
+            double v;
+            std::memcpy(&v, &b, sizeof(v));
+            dispMax2 = std::max(dispMax2, v);
+        }
+        if (err & ERRBIT_STALE) c->rebuildNext = true;
+        if (err & ~(uint32_t)ERRBIT_STALE) {
+            c->directBackoff = std::min<uint32_t>(std::max<uint32_t>(2 * c->directBackoff, 1), 64);
+            c->directSkip = c->directBackoff;
+            *again = false;
+            break;
+        }
+        if (!err) {
+            c->directBackoff = 0;
+            rebuilt = false;
+            continue;
+        }
+        if (*done >= n) break;  // the pass that follows rebuilds
+        // lists that die within 4 steps at the widest automatic skin give way to the cell sweep for a while, lists stale
+        // right after a build to the pass (which reports why)
+        giveUp = c->skinSet < 0.0 && c->passesSinceBuild < 4 &&
+                 c->skinAuto >= 0.8 * (double)c->meanRadius * (1.0 - 1e-9);
+        if (giveUp || (rebuilt && steps == 0)) {
+            *again = false;
+            break;
+        }
+        if ((r = direct_rebuild(c))) {
+            // (out of memory in the build) the candidates and their histories are gone
+            c->contactsReady = c->havePrev = c->candValid = false;
+            return r;
+        }
+        rebuilt = true;
+        dispMax2 = 0.0;
+        counted = 0;
+    }
+    if (*done > 0 || rebuilt) {
+        if ((r = direct_leave(c))) return r;
+    }
+    if (giveUp) {
+        c->cellBackoff = std::min<uint32_t>(c->cellBackoff ? 2 * c->cellBackoff : 64, 4096);
+        c->cellPassesLeft = c->cellBackoff;
+        c->candValid = false;
+        c->graphGen++;
+    }
+    return DEME_OK;
+}
+
+// Steps on the candidates pay once a call holds this many: entering and leaving cost about two passes.
+constexpr int DIRECT_MIN_STEPS = 6;
+
 int deme_step(deme_ctx* c, int nSteps, int updateFreq) {
     c->adjReady = false;  // recorded adjoint checkpoints no longer describe the system
     int r = check_ready(c);
     if (r) return r;
     const uint64_t f = updateFreq > 0 ? (uint64_t)updateFreq : 1;
+    bool direct = f == 1 && !c->useGraphs;
+    if (direct && c->directSkip > 0) {
+        c->directSkip--;
+        direct = false;
+    }
     for (int k = 0; k < nSteps; k++) {
+        // detecting every step, all but the last step of the call may run on the candidates; the last one runs its own
+        // pass, so the call leaves the contact list, its map and its records as every step would
+        if (direct && nSteps - k >= DIRECT_MIN_STEPS && direct_ready(c)) {
+            int done = 0;
+            if ((r = run_direct(c, nSteps - k - 1, &done, &direct))) return r;
+            k += done;
+        }
         const bool detect = c->nSteps % f == 0 || !c->contactsReady || c->needDetect;
         // a whole interval from its graph: due for detection, a current list to carry the history over, all f steps
         // within this call, and no per-contact records wanted on its last step

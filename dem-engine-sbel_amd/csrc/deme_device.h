@@ -216,6 +216,231 @@ __device__ __forceinline__ CdRec load_cd(const CdRec* __restrict__ p, uint32_t i
     return r;
 }
 
+// ERRBIT_STALE: a sphere moved too far since the candidate lists were built; they must be rebuilt and the pass redone
+// ERRBIT_EDGE: a sphere too near the bin grid's upper ends for stepping on the candidates
+enum : uint32_t {
+    ERRBIT_CAPACITY = 1u,
+    ERRBIT_PAIR_OVERFLOW = 2u,
+    ERRBIT_OUTSIDE = 4u,
+    ERRBIT_STALE = 8u,
+    ERRBIT_EDGE = 16u
+};
+
+// --------------------------------------------------------------------------------------------------------------
+// The contact predicate of detection: expanded overlap, plane distance, and the contact-point bin rule.
+// --------------------------------------------------------------------------------------------------------------
+struct BinRange {
+    uint32_t x0, x1, y0, y1, z0, z1;
+};
+
+// DEMBinSphereKernels.cu:52-64 (double position and radius span, truncating conversions)
+__device__ __forceinline__ BinRange bin_range(const KParams& P, double X, double Y, double Z, double rCD) {
+    const double bx = X / P.binSize, by = Y / P.binSize, bz = Z / P.binSize, span = rCD / P.binSize;
+    BinRange r;
+    r.x0 = sat_u32(bx - span);
+    r.x1 = sat_u32(bx + span);
+    r.y0 = sat_u32(by - span);
+    r.y1 = sat_u32(by + span);
+    r.z0 = sat_u32(bz - span);
+    r.z1 = sat_u32(bz + span);
+    return r;
+}
+
+// checkSphereEntityOverlap<double> without contact point (DEMHelperKernels.cu:356-391); rCD already holds r + beta.
+__device__ __forceinline__ bool plane_cd(const KParams& P, const PlanePose& pp, double X, double Y, double Z,
+                                         double rCD) {
+    if (pp.type != DEME_ANAL_OBJ_TYPE_PLANE) return false;
+    const double dx = X - pp.px, dy = Y - pp.py, dz = Z - pp.pz;
+    const double dist = dx * (double)pp.nx + dy * (double)pp.ny + dz * (double)pp.nz;
+    return !(dist > rCD + (double)P.beta);
+}
+
+__device__ __forceinline__ bool range_in_grid(const KParams& P, const BinRange& r) {
+    return r.x1 < P.nbX && r.y1 < P.nbY && r.z1 < P.nbZ;
+}
+
+// Membership of a linear bin id in the linear ids of a range (the reference's bins may alias when a range crosses
+// the grid's upper faces; this enumerates exactly the ids the reference would form).
+// (Out of line: the rare path. Arguments by value, so the caller's ranges stay in registers.)
+static __device__ __noinline__ bool range_has_linear(uint32_t nbX, uint32_t nbY, BinRange r, uint32_t lin) {
+    const uint32_t nbXY = nbX * nbY;
+    for (uint32_t k = 0; k <= r.z1 - r.z0; k++)
+        for (uint32_t j = 0; j <= r.y1 - r.y0; j++)
+            for (uint32_t i = 0; i <= r.x1 - r.x0; i++)
+                if ((r.x0 + i) + (r.y0 + j) * nbX + (r.z0 + k) * nbXY == lin) return true;
+    return false;
+}
+
+// Expanded radius as the reference's detection kernel forms it: float(r + beta), widened to double.
+__device__ __forceinline__ double expanded_radius(const KParams& P, float r) {
+    float rf = r;
+    rf += P.beta;
+    return (double)rf;
+}
+
+// First half of the reference's sphere-pair test (checkSpheresOverlap<double>, DEMHelperKernels.cu:195-205): the
+// expanded spheres overlap.
+__device__ __forceinline__ bool expanded_overlap(double ra, const CdRec& A, double rb, const CdRec& B) {
+    const double dx = A.x - B.x, dy = A.y - B.y, dz = A.z - B.z;
+    const double d2 = dx * dx + dy * dy + dz * dz;
+    return !(d2 > (ra + rb) * (ra + rb));
+}
+
+// Second half, for a pair that overlaps: the contact point (DEMHelperKernels.cu:206-222) computed with A the lower id,
+// and its bin inside both spheres' AABB bin ranges.
+struct RuleBins {
+    uint32_t ix, iy, iz;
+    BinRange ga, gb;
+};
+
+__device__ __forceinline__ void contact_point(const KParams& P, const CdRec& A, const CdRec& B, double& cx, double& cy,
+                                              double& cz) {
+    const double ra = expanded_radius(P, A.r), rb = expanded_radius(P, B.r);
+    const double dx = A.x - B.x, dy = A.y - B.y, dz = A.z - B.z;
+    const double d2 = dx * dx + dy * dy + dz * dz;
+    float nX = (float)dx, nY = (float)dy, nZ = (float)dz;
+    const float mag = sqrtf(nX * nX + nY * nY + nZ * nZ);
+    nX /= mag;
+    nY /= mag;
+    nZ /= mag;
+    const double half = (ra + rb - sqrt(d2)) / 2.0;
+    cx = B.x + (rb - half) * (double)nX;
+    cy = B.y + (rb - half) * (double)nY;
+    cz = B.z + (rb - half) * (double)nZ;
+}
+
+__device__ __forceinline__ double cd_radius(const KParams& P, float r) {
+    double v = (double)r;
+    v += (double)P.beta;
+    return v;
+}
+
+// The reference's bin indices, with its divisions by binSize.
+__device__ __forceinline__ void rule_bins_exact(const KParams& P, const CdRec& A, const CdRec& B, double cx, double cy,
+                                                double cz, RuleBins& R) {
+    R.ix = sat_u32(cx / P.binSize);
+    R.iy = sat_u32(cy / P.binSize);
+    R.iz = sat_u32(cz / P.binSize);
+    R.ga = bin_range(P, A.x, A.y, A.z, cd_radius(P, A.r));
+    R.gb = bin_range(P, B.x, B.y, B.z, cd_radius(P, B.r));
+}
+
+// The same bin indices from multiplications by the reciprocal of the bin size, used when every floor input lies
+// farther from an integer than the product and the quotient can differ (a few ulps; the margin is 2^-40 relative):
+// then each floor, and so the rule, equals the division's. Returns false when a value is too close to call.
+__device__ __forceinline__ bool far_from_int(double t, double scale) {
+    const double f = t - floor(t);
+    const double eps = 0x1p-40 * (scale + 1.0);
+    return f > eps && f < 1.0 - eps;
+}
+
+__device__ __forceinline__ bool range_fast(const KParams& P, double inv, double X, double Y, double Z, double rCD,
+                                           BinRange& r) {
+    const double bx = X * inv, by = Y * inv, bz = Z * inv, span = rCD * inv;
+    const double ax = fabs(bx) + span, ay = fabs(by) + span, az = fabs(bz) + span;
+    const double x0 = bx - span, x1 = bx + span, y0 = by - span, y1 = by + span, z0 = bz - span, z1 = bz + span;
+    if (!(far_from_int(x0, ax) && far_from_int(x1, ax) && far_from_int(y0, ay) && far_from_int(y1, ay) &&
+          far_from_int(z0, az) && far_from_int(z1, az)))
+        return false;
+    r.x0 = sat_u32(x0);
+    r.x1 = sat_u32(x1);
+    r.y0 = sat_u32(y0);
+    r.y1 = sat_u32(y1);
+    r.z0 = sat_u32(z0);
+    r.z1 = sat_u32(z1);
+    return true;
+}
+
+__device__ __forceinline__ bool rule_bins_fast(const KParams& P, double inv, const CdRec& A, const CdRec& B, double cx,
+                                               double cy, double cz, RuleBins& R) {
+    const double qx = cx * inv, qy = cy * inv, qz = cz * inv;
+    if (!(far_from_int(qx, fabs(qx)) && far_from_int(qy, fabs(qy)) && far_from_int(qz, fabs(qz)))) return false;
+    R.ix = sat_u32(qx);
+    R.iy = sat_u32(qy);
+    R.iz = sat_u32(qz);
+    return range_fast(P, inv, A.x, A.y, A.z, cd_radius(P, A.r), R.ga) &&
+           range_fast(P, inv, B.x, B.y, B.z, cd_radius(P, B.r), R.gb);
+}
+
+__device__ __forceinline__ bool rule_member(const KParams& P, const RuleBins& R) {
+    if (range_in_grid(P, R.ga) && range_in_grid(P, R.gb)) {
+        // no aliasing: a linear id is one (i, j, k) -- unless the point itself lies past the grid, where the
+        // reference's linear id aliases; fall through to the exact enumeration then
+        if (R.ix < P.nbX && R.iy < P.nbY && R.iz < P.nbZ)
+            return R.ix >= R.ga.x0 && R.ix <= R.ga.x1 && R.iy >= R.ga.y0 && R.iy <= R.ga.y1 && R.iz >= R.ga.z0 &&
+                   R.iz <= R.ga.z1 && R.ix >= R.gb.x0 && R.ix <= R.gb.x1 && R.iy >= R.gb.y0 && R.iy <= R.gb.y1 &&
+                   R.iz >= R.gb.z0 && R.iz <= R.gb.z1;
+    }
+    const uint32_t lin = R.ix + R.iy * P.nbX + R.iz * P.nbX * P.nbY;
+    return range_has_linear(P.nbX, P.nbY, R.ga, lin) && range_has_linear(P.nbX, P.nbY, R.gb, lin);
+}
+
+// True only when the bin rule of an overlapping pair must hold. The exact contact point lies inside both expanded
+// spheres, ra - half from A's centre and rb - half from B's (half: half the overlap, at most the smaller radius), so its
+// bin lies in both spheres' bin ranges as soon as half exceeds what rounding can move: the float-rounded direction
+// moves the point by under 6e-7 (ra + rb), float(r + beta) differs from r + beta by under 6e-8 (ra + rb), and the
+// double positions and quotients add a few 2^-52 of the coordinates. Floors and saturation are monotone, and a triple
+// inside both ranges is among the linear ids of both, so the aliasing cases agree. Everything else (grazing pairs,
+// near-coincident centres, one sphere deep inside another, NaN) answers false and takes the full rule.
+__device__ __forceinline__ bool bin_rule_certain(double ra, const CdRec& A, double rb, const CdRec& B) {
+    const double dx = A.x - B.x, dy = A.y - B.y, dz = A.z - B.z;
+    const double sum = ra + rb, dist = sqrt(dx * dx + dy * dy + dz * dz), half = 0.5 * (sum - dist);
+    const double reach = fabs(A.x) + fabs(A.y) + fabs(A.z) + sum;
+    return half > 1e-6 * sum + 0x1p-46 * reach && half <= fmin(ra, rb) && dist > 1e-3 * sum && sum > 1e-12;
+}
+
+// A: the lower id of an overlapping pair. inv: 1 / binSize.
+__device__ __forceinline__ bool bin_rule_point(const KParams& P, double inv, const CdRec& A, const CdRec& B) {
+    if (bin_rule_certain(expanded_radius(P, A.r), A, expanded_radius(P, B.r), B)) return true;
+    double cx, cy, cz;
+    contact_point(P, A, B, cx, cy, cz);
+    RuleBins R;
+    if (!rule_bins_fast(P, inv, A, B, cx, cy, cz, R)) rule_bins_exact(P, A, B, cx, cy, cz, R);
+    return rule_member(P, R);
+}
+
+// The rule for pairs whose spheres' ranges lie inside the grid on every axis, the contact point with them (no linear id
+// aliases then, so membership is per axis), one axis at a time: the force kernel's registers are taken, and the general
+// form inlined there costs it a wave per SIMD (140 registers; out of line, 150). A: the lower id.
+__device__ __forceinline__ bool axis_in_ranges(double binSize, double c, double xa, double ra, double xb, double rb) {
+    const uint32_t i = sat_u32(c / binSize);
+    const double ba = xa / binSize, sa = ra / binSize;
+    if (i < sat_u32(ba - sa) || i > sat_u32(ba + sa)) return false;
+    const double bb = xb / binSize, sb = rb / binSize;
+    return !(i < sat_u32(bb - sb) || i > sat_u32(bb + sb));
+}
+__device__ __forceinline__ bool bin_rule_inside(const KParams& P, const CdRec& A, const CdRec& B) {
+    if (bin_rule_certain(expanded_radius(P, A.r), A, expanded_radius(P, B.r), B)) return true;
+    double cx, cy, cz;
+    contact_point(P, A, B, cx, cy, cz);
+    const double ra = cd_radius(P, A.r), rb = cd_radius(P, B.r);
+    if (!axis_in_ranges(P.binSize, cx, A.x, ra, B.x, rb)) return false;
+    __builtin_amdgcn_sched_barrier(0);
+    if (!axis_in_ranges(P.binSize, cy, A.y, ra, B.y, rb)) return false;
+    __builtin_amdgcn_sched_barrier(0);
+    return axis_in_ranges(P.binSize, cz, A.z, ra, B.z, rb);
+}
+
+// The bin-range check of a sphere's detection record: ERRBIT_CAPACITY when it touches more bins than the reference can
+// count, ERRBIT_OUTSIDE when a bin of its range lies past the grid, 0 when neither.
+__device__ __forceinline__ uint32_t bin_range_err(const KParams& P, const BinRange& r) {
+    const uint32_t nx = r.x1 - r.x0 + 1, ny = r.y1 - r.y0 + 1, nz = r.z1 - r.z0 + 1;
+    if ((uint64_t)nx * ny * nz > 65535u) return ERRBIT_CAPACITY;
+    // The linear id grows with each of i, j, k, so without 32-bit wrap the range's largest id is its last corner.
+    const uint32_t nbXY = P.nbX * P.nbY;
+    const uint64_t last = (uint64_t)r.x1 + (uint64_t)r.y1 * P.nbX + (uint64_t)r.z1 * nbXY;
+    bool outside = last >= P.nBins;
+    if (last > 0xFFFFFFFFull) {
+        // ids wrap: enumerate them as the reference forms them
+        outside = false;
+        for (uint32_t dk = 0; dk < nz; dk++)
+            for (uint32_t dj = 0; dj < ny; dj++)
+                for (uint32_t di = 0; di < nx; di++)
+                    outside |= ((r.x0 + di) + (r.y0 + dj) * P.nbX + (r.z0 + dk) * nbXY) >= P.nBins;
+    }
+    return outside ? ERRBIT_OUTSIDE : 0u;
+}
+
 // World pose of an analytical component from its owner's state.
 __device__ __forceinline__ PlanePose plane_pose_of(const KParams& P, const deme_anal_obj& ob, const OwnerRec& o) {
     double ox, oy, oz;
@@ -295,9 +520,6 @@ __host__ __device__ inline double max_disp2(const DevCounters& c) {
     return d;
 }
 
-// ERRBIT_STALE: a sphere moved too far since the candidate lists were built; they must be rebuilt and the pass redone
-enum : uint32_t { ERRBIT_CAPACITY = 1u, ERRBIT_PAIR_OVERFLOW = 2u, ERRBIT_OUTSIDE = 4u, ERRBIT_STALE = 8u };
-
 // Kernels enqueued before the host has read a detection pass's counters (so the GPU does not wait for the host, or
 // the whole step sits in a captured graph) exit at once, writing nothing, when the pass failed, a slab row
 // overflowed, or the contact / mirror-row totals exceed the buffers they were given; the host then redoes them.
@@ -309,6 +531,93 @@ struct SpecGuard {
 };
 __device__ __forceinline__ bool spec_skip(const SpecGuard& g) {
     return g.ctr && (g.ctr->err || g.ctr->maxOcc > g.slabCap || g.ctr->total[1] > g.capC || g.ctr->total[2] > g.capP);
+}
+
+// --------------------------------------------------------------------------------------------------------------
+// Stepping on the candidates: between list builds, the force kernel takes the build's candidates themselves (one lane
+// each: the predicate, then the force of those that touch), with histories and owner terms kept by candidate, and the
+// owner update sums over the candidate rows. No contact list is formed in between.
+// --------------------------------------------------------------------------------------------------------------
+// err: set by the checks of a state (ERRBIT_*), sticky; the force kernel copies it to skip, which the owner update of
+// the same step obeys (that kernel itself checks the state it leaves, so it cannot read err); steps: owner updates
+// done; disp2: as in DevCounters.
+struct DirectState {
+    uint32_t err, skip, steps, pad;
+    unsigned long long disp2[64];
+};
+// The candidates: pairs c < nPair (candA < candB, tPos: slot of c in the transposed rows) and planes q < nPlane (sphere
+// pSph, component pPlane; rows pStart by sphere). on / pOn: touched in the last step, whose history then stands in hist /
+// pHist; bOn: on by transposed slot. aTerm, pTerm: A's owner terms; bTerm: B's, by transposed slot.
+struct DirectList {
+    uint32_t nPair, nPlane;
+    const uint32_t *candA, *candB, *tPos, *pSph, *pPlane, *pStart;
+    uint8_t *on, *pOn, *bOn;
+    float4 *hist, *pHist;
+    float* pTerm;
+    const uint8_t* mask;  // family mask, null when every pair is allowed
+    DirectState* st;      // null: not stepping on candidates
+};
+// What the owner update checks of the state it leaves: no sphere farther than sqrt(limit2) from its position at the
+// build (pos0, in units of unit), every sphere clear of the bin grid's upper ends (its upper corner below hiX, hiY,
+// hiZ: its bin range, and the contact point of any pair, then lie inside the grid; the hosts' limits are minus infinity
+// where a sphere could touch too many bins), and no component moved by more than planeLimit since the plane candidates
+// were made (pose0; reach bounds a sphere's distance from the origin). A state that fails is left to the contact-list
+// path: its pass reports an error, or goes on.
+struct DirectCheck {
+    const SphereRec* sph;
+    const BuildPos* pos0;
+    double unit, limit2;
+    double hiX, hiY, hiZ;
+    const PlanePose* pose0;
+    double planeLimit, reach;
+};
+
+// One sphere's part of the check: ERRBIT_* bits, d2 raised to its squared displacement.
+__device__ __forceinline__ uint32_t direct_check_sphere(const KParams& P, const DirectCheck& C, const OwnerRec& o,
+                                                        uint32_t s, double& d2) {
+    const SphereRec sr = load_sphere(C.sph, s);
+    const BuildPos b = C.pos0[s];
+    double X, Y, Z;
+    sphere_position(P, o, sr, X, Y, Z);
+    const double rCD = (double)sr.r + (double)P.beta;
+    uint32_t bad = 0;
+    if (!(X + rCD < C.hiX && Y + rCD < C.hiY && Z + rCD < C.hiZ)) bad = ERRBIT_EDGE;
+    constexpr int32_t unfit = -2147483647 - 1;  // INT32_MIN (hipRTC has no limits)
+    const double inf = __builtin_huge_val();
+    if (b.x == unfit || b.y == unfit || b.z == unfit) {
+        d2 = inf;
+    } else {
+        const double dx = X - (double)b.x * C.unit, dy = Y - (double)b.y * C.unit, dz = Z - (double)b.z * C.unit;
+        const double q = dx * dx + dy * dy + dz * dz;
+        const double v = q == q ? q : inf;
+        d2 = v > d2 ? v : d2;
+    }
+    return bad;
+}
+
+// Whether component a's plane moved too far since its near spheres were listed: the signed distance of any point within
+// reach of the origin changes by at most |n.p - n0.p0| + |n - n0| reach.
+__device__ __forceinline__ bool direct_plane_moved(const DirectCheck& C, const PlanePose& a, const PlanePose& b) {
+    const double oa = a.px * (double)a.nx + a.py * (double)a.ny + a.pz * (double)a.nz;
+    const double ob = b.px * (double)b.nx + b.py * (double)b.ny + b.pz * (double)b.nz;
+    const double dx = (double)a.nx - (double)b.nx, dy = (double)a.ny - (double)b.ny, dz = (double)a.nz - (double)b.nz;
+    return !(fabs(oa - ob) + sqrt(dx * dx + dy * dy + dz * dz) * C.reach <= C.planeLimit);
+}
+
+// A workgroup's (256 lanes) displacements and error bits into the state; every lane calls it.
+__device__ __forceinline__ void direct_report(DirectState* st, double limit2, double d2, uint32_t bad) {
+    if (d2 > limit2) bad |= ERRBIT_STALE;
+#pragma unroll
+    for (int off = 32; off > 0; off >>= 1) {
+        d2 = fmax(d2, __shfl_xor(d2, off, 64));
+        bad |= (uint32_t)__shfl_xor((int)bad, off, 64);
+    }
+    if ((threadIdx.x & 63u) == 0) {
+        if (bad) atomicOr(&st->err, bad);
+        if (d2 > limit2 * 0x1p-6)  // (smaller ones do not decide anything: no atomic for them)
+            atomicMax(&st->disp2[(blockIdx.x * 4u + (threadIdx.x >> 6)) % DISP_SLOTS],
+                      (unsigned long long)__double_as_longlong(d2));
+    }
 }
 
 }  // namespace deme_dev

@@ -55,6 +55,9 @@ constexpr uint64_t scan2_sums_elems(uint64_t n) {
     return 2 * ((n <= SCAN2_SMALL_N ? (n + SCAN_BLOCK - 1) / SCAN_BLOCK : (n + SCAN2_TILE - 1) / SCAN2_TILE) + 1);
 }
 using deme_dev::MAX_ANAL_OWNERS;
+using deme_dev::DirectCheck;
+using deme_dev::DirectList;
+using deme_dev::DirectState;
 using deme_dev::PART_FROM_COUNTERS;
 using deme_dev::PlaneRefresh;
 using deme_dev::PlaneSums;
@@ -234,7 +237,39 @@ hipError_t launch_owner_update(const KParams& P, uint32_t nO, uint32_t nClumps, 
                                float* acc /* 6 x nO SoA: aX aY aZ alX alY alZ */, int doIntegrate,
                                const double* clock /* device: the simulation time the motion rules read */,
                                hipStream_t st, OwnerRec* ownOut = nullptr /* integrated records; null: in place */,
-                               SpecGuard guard = SpecGuard());
+                               SpecGuard guard = SpecGuard(), const DirectList& direct = DirectList(),
+                               const DirectCheck& check = DirectCheck());
+// The force kernel over the candidates D (the predicate, then the force of those that touch; D's flags, histories and
+// terms in place). The partial sums cover the plane candidates' workgroups: (D.nPlane + 255) / 256 of them.
+hipError_t launch_force_direct(const KParams& P, const DirectList& D, const SphereRec* sph, const OwnerRec* own,
+                               const float4* moi, const deme_anal_obj* anal, const PlanePose* pose,
+                               const deme_material* mats, float* aTerm, float* bTerm, const PlaneSums& sums,
+                               hipStream_t st);
+inline uint32_t direct_force_blocks(const DirectList& D) {
+    const uint32_t b = (D.nPlane + 255u) / 256u + (D.nPair + 255u) / 256u;
+    return b ? b : 1u;  // (the skip flag is passed on even when there is no candidate)
+}
+
+// direct.hip: what connects the candidates to the contact list (see there)
+hipError_t launch_direct_near(const KParams& P, const SphereRec* sph, const OwnerRec* own, uint32_t nS,
+                              const PlanePose* pose, uint32_t nA, double margin, unsigned long long* nearBits,
+                              uint32_t* nearCnt, hipStream_t st);
+hipError_t launch_direct_plane_rows(const KParams& P, const SphereRec* sph, const OwnerRec* own, uint32_t nS,
+                                    const unsigned long long* nearBits, const uint32_t* pStart, uint32_t* pSph,
+                                    uint32_t* pPlane, const PlanePose* pose, uint32_t nA, PlanePose* pose0,
+                                    hipStream_t st);
+hipError_t launch_direct_enter(const DirectList& D, const uint32_t* cidx, const uint32_t* rowStart, const uint32_t* idB,
+                               const uint8_t* ctype, const float4* listHist, hipStream_t st);
+hipError_t launch_direct_join(uint32_t nS, const uint32_t* oldStart, const uint32_t* oldB, const uint32_t* newStart,
+                              const uint32_t* newB, const uint32_t* oldPStart, const uint32_t* oldPlane,
+                              const DirectList& O, const DirectList& D, hipStream_t st);
+hipError_t launch_direct_check(const KParams& P, const DirectCheck& C, const OwnerRec* own, uint32_t nS,
+                               const PlanePose* pose, uint32_t nA, DirectState* state, hipStream_t st);
+hipError_t launch_direct_plane_bits(const KParams& P, const SphereRec* sph, const OwnerRec* own, uint32_t nS,
+                                    const DirectList& D, uint32_t* numAnal, unsigned long long* planeBits,
+                                    uint32_t* clear, uint32_t nClear, hipStream_t st);
+hipError_t launch_direct_leave(const DirectList& D, const uint32_t* cidx, const uint32_t* rowStart, float4* listHist,
+                               hipStream_t st, SpecGuard guard);
 // clock[0] = t (one lane; the time the owner update's motion rules read, written on the stream before the update)
 hipError_t launch_set_clock(double* clock, double t, hipStream_t st);
 // clock[0] += (double)h: the time step the host adds after each step, done on the device inside a captured step
@@ -251,7 +286,7 @@ inline uint32_t owner_blocks(uint32_t nClumps, uint32_t nAnalOwners) {
 }
 struct JitForce {
     hipModule_t mod = nullptr;
-    hipFunction_t full = nullptr, terms = nullptr;
+    hipFunction_t full = nullptr, terms = nullptr, direct = nullptr;
     void release();
     hipError_t load(const std::vector<char>& code);
     hipError_t launch(bool wantFull, const KParams& P, uint32_t nC, const uint32_t* idA, const uint32_t* idB,
@@ -260,6 +295,10 @@ struct JitForce {
                       const float4* histIn, const uint32_t* map, float4* histOut, const uint32_t* mirror,
                       float* aTerm, float* bTerm, const PlaneSums& sums, uint8_t* aOn, uint8_t* bOn, ForceRec* out,
                       hipStream_t st, SpecGuard guard = SpecGuard()) const;
+    hipError_t launch_direct(const KParams& P, const DirectList& D, const SphereRec* sph, const OwnerRec* own,
+                             const float4* moi, const deme_anal_obj* anal, const PlanePose* pose,
+                             const deme_material* mats, float* aTerm, float* bTerm, const PlaneSums& sums,
+                             hipStream_t st) const;
 };
 // the owner update kernel specialised with motion strategies / family change rules
 struct JitOwner {
@@ -271,7 +310,8 @@ struct JitOwner {
                       const uint32_t* rowStart, const uint32_t* bRowStart, const float* aTerm, const float* bTerm,
                       const uint8_t* aOn, const uint8_t* bOn, const PlaneSums& sums, const PlaneRefresh& planes,
                       const deme_family_rule* rules, const OwnerRec* own, OwnerRec* ownOut, float* acc, int doIntegrate, const double* clock,
-                      hipStream_t st, SpecGuard guard = SpecGuard()) const;
+                      hipStream_t st, SpecGuard guard = SpecGuard(), const DirectList& direct = DirectList(),
+                      const DirectCheck& check = DirectCheck()) const;
 };
 std::string jit_owner_source(const std::vector<std::pair<std::string, std::string>>& values);
 

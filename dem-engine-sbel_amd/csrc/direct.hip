@@ -1,0 +1,261 @@
+// Stepping on the candidates of a list build (deme_step with detection every step and no drift margin).
+//
+// Detecting every step, the passes of the contact-list path mostly renumber: of 1M clumps' 2.97M candidates all but a
+// few touch from one step to the next, yet each pass forms flags, row counts, two scans, the rows, the mirror links and
+// the history map (220 of 400 us a step), and small systems pay the launches. Between builds the candidates' own order
+// already is the canonical order, so the force kernel can take them directly: history and owner terms live in the
+// candidate's slots, a flag says whether it touched, and the owner update sums the flagged terms of the candidate rows
+// -- the same terms in the same order, bit for bit. A step is then two kernels (force, owner update), and the host reads
+// one status per batch of steps.
+//
+// This file holds what connects the two forms: the plane candidates (spheres near a plane, which the pair lists do not
+// hold), histories carried from the contact list to the candidates and back, and from one build's candidates to the
+// next.
+#include "deme_internal.h"
+
+namespace deme_int {
+using namespace deme_dev;
+namespace {
+
+// Planes within `margin` of touching each sphere (no family mask: families may change from step to step).
+__global__ __launch_bounds__(256) void k_direct_near(KParams P, const SphereRec* __restrict__ sph,
+                                                     const OwnerRec* __restrict__ own, uint32_t nS,
+                                                     const PlanePose* __restrict__ pose, uint32_t nA, double margin,
+                                                     unsigned long long* __restrict__ nearBits,
+                                                     uint32_t* __restrict__ nearCnt) {
+    const uint32_t s = blockIdx.x * blockDim.x + threadIdx.x;
+    if (s >= nS) return;
+    const SphereRec sr = load_sphere(sph, s);
+    const OwnerRec o = load_owner(own, sr.owner);
+    double X, Y, Z;
+    sphere_position(P, o, sr, X, Y, Z);
+    const double reach = (double)sr.r + (double)P.beta + margin;
+    unsigned long long bits = 0;
+    uint32_t a0, a1;
+    scene_planes(P, o.scene, a0, a1);
+    for (uint32_t a = a0; a < a1 && a < nA && a - a0 < 64; a++)
+        if (plane_cd(P, pose[a], X, Y, Z, reach)) bits |= 1ull << (a - a0);
+    nearBits[s] = bits;
+    nearCnt[s] = (uint32_t)__popcll(bits);
+}
+
+__global__ __launch_bounds__(256) void k_direct_plane_rows(KParams P, const SphereRec* __restrict__ sph,
+                                                           const OwnerRec* __restrict__ own, uint32_t nS,
+                                                           const unsigned long long* __restrict__ nearBits,
+                                                           const uint32_t* __restrict__ pStart,
+                                                           uint32_t* __restrict__ pSph, uint32_t* __restrict__ pPlane,
+                                                           const PlanePose* __restrict__ pose, uint32_t nA,
+                                                           PlanePose* __restrict__ pose0) {
+    const uint32_t s = blockIdx.x * blockDim.x + threadIdx.x;
+    if (blockIdx.x == 0)
+        for (uint32_t a = threadIdx.x; a < nA; a += 256) pose0[a] = pose[a];
+    if (s >= nS) return;
+    unsigned long long bits = nearBits[s];
+    if (!bits) return;
+    uint32_t a0 = 0, a1 = 0;
+    scene_planes(P, own[sph[s].owner].scene, a0, a1);
+    for (uint32_t q = pStart[s]; bits; q++) {
+        pSph[q] = s;
+        pPlane[q] = a0 + (uint32_t)(__ffsll(bits) - 1);
+        bits &= bits - 1;
+    }
+}
+
+// The contact list's histories to the candidates: pairs through their contact index (cidx, valid where on), planes by
+// looking their component up at the head of the sphere's row. One lane per candidate, planes after the pairs.
+__global__ __launch_bounds__(256) void k_direct_enter(DirectList D, uint32_t pairBlocks,
+                                                      const uint32_t* __restrict__ cidx,
+                                                      const uint32_t* __restrict__ rowStart,
+                                                      const uint32_t* __restrict__ idB,
+                                                      const uint8_t* __restrict__ ctype,
+                                                      const float4* __restrict__ listHist) {
+    if (blockIdx.x < pairBlocks) {
+        const uint32_t c = blockIdx.x * 256u + threadIdx.x;
+        if (c >= D.nPair) return;
+        const uint8_t f = D.on[c];
+        D.bOn[D.tPos[c]] = f;
+        if (f) D.hist[c] = listHist[cidx[c]];
+        return;
+    }
+    const uint32_t q = (blockIdx.x - pairBlocks) * 256u + threadIdx.x;
+    if (q >= D.nPlane) return;
+    const uint32_t s = D.pSph[q], p = D.pPlane[q], e = rowStart[s + 1];
+    uint8_t f = 0;
+    for (uint32_t i = rowStart[s]; i < e && ctype[i] == DEME_SPHERE_PLANE_CONTACT && idB[i] <= p; i++)
+        if (idB[i] == p) {
+            f = 1;
+            D.pHist[q] = listHist[i];
+        }
+    D.pOn[q] = f;
+}
+
+// One sphere's row of new candidates matched against its old row (both ascending in partner): flags and histories of
+// the partners found. Rows are short: the old row's first entries are held in registers.
+constexpr uint32_t JOIN_REG = 8;
+__device__ __forceinline__ void join_row(uint32_t o0, uint32_t o1, const uint32_t* __restrict__ oldB,
+                                         const uint8_t* __restrict__ oldOn, const float4* __restrict__ oldHist,
+                                         uint32_t n0, uint32_t n1, const uint32_t* __restrict__ newB,
+                                         const uint32_t* __restrict__ tPos, uint8_t* __restrict__ on,
+                                         uint8_t* __restrict__ bOn, float4* __restrict__ hist) {
+    const uint32_t no = o1 - o0;
+    uint32_t ob[JOIN_REG];
+    uint8_t of[JOIN_REG];
+#pragma unroll
+    for (uint32_t k = 0; k < JOIN_REG; k++) {
+        ob[k] = k < no ? oldB[o0 + k] : 0xFFFFFFFFu;
+        of[k] = k < no ? oldOn[o0 + k] : (uint8_t)0;
+    }
+    for (uint32_t c = n0; c < n1; c++) {
+        const uint32_t b = newB[c];
+        uint32_t m = 0xFFFFFFFFu;
+        uint8_t f = 0;
+#pragma unroll
+        for (uint32_t k = 0; k < JOIN_REG; k++)
+            if (k < no && ob[k] == b) {
+                m = o0 + k;
+                f = of[k];
+            }
+        for (uint32_t j = o0 + JOIN_REG; j < o1 && m == 0xFFFFFFFFu; j++)
+            if (oldB[j] == b) {
+                m = j;
+                f = oldOn[j];
+            }
+        on[c] = f;
+        if (bOn) bOn[tPos[c]] = f;
+        if (f) hist[c] = oldHist[m];
+    }
+}
+
+__global__ __launch_bounds__(256) void k_direct_join(uint32_t nS, const uint32_t* __restrict__ oldStart,
+                                                     const uint32_t* __restrict__ oldB,
+                                                     const uint32_t* __restrict__ newStart,
+                                                     const uint32_t* __restrict__ newB,
+                                                     const uint32_t* __restrict__ oldPStart,
+                                                     const uint32_t* __restrict__ oldPlane, DirectList O, DirectList D) {
+    const uint32_t s = blockIdx.x * blockDim.x + threadIdx.x;
+    if (s >= nS) return;
+    join_row(oldStart[s], oldStart[s + 1], oldB, O.on, O.hist, newStart[s], newStart[s + 1], newB, D.tPos, D.on, D.bOn,
+             D.hist);
+    const uint32_t p0 = D.pStart[s], p1 = D.pStart[s + 1];
+    if (p0 < p1)
+        join_row(oldPStart[s], oldPStart[s + 1], oldPlane, O.pOn, O.pHist, p0, p1, D.pPlane, nullptr, D.pOn, nullptr,
+                 D.pHist);
+}
+
+// The check of a state the owner update did not leave itself (a call's first step on the candidates).
+__global__ __launch_bounds__(256) void k_direct_check(KParams P, DirectCheck C, const OwnerRec* __restrict__ own,
+                                                      uint32_t nS, const PlanePose* __restrict__ pose, uint32_t nA,
+                                                      DirectState* st) {
+    const uint32_t s = blockIdx.x * blockDim.x + threadIdx.x;
+    double d2 = 0.0;
+    uint32_t bad = 0;
+    if (s < nS) bad = direct_check_sphere(P, C, load_owner(own, C.sph[s].owner), s, d2);
+    if (blockIdx.x == 0)
+        for (uint32_t a = threadIdx.x; a < nA; a += 256)
+            if (direct_plane_moved(C, pose[a], C.pose0[a])) bad |= ERRBIT_STALE;
+    direct_report(st, C.limit2, d2, bad);
+}
+
+// Back to the contact list, first: the plane contacts of the last step per sphere (count and bits within the scene's
+// components), and the pass's counters cleared.
+__global__ __launch_bounds__(256) void k_direct_plane_bits(KParams P, const SphereRec* __restrict__ sph,
+                                                           const OwnerRec* __restrict__ own, uint32_t nS, DirectList D,
+                                                           uint32_t* __restrict__ numAnal,
+                                                           unsigned long long* __restrict__ planeBits,
+                                                           uint32_t* __restrict__ clear, uint32_t nClear) {
+    if (blockIdx.x == 0)
+        for (uint32_t k = threadIdx.x; k < nClear; k += 256) clear[k] = 0u;
+    const uint32_t s = blockIdx.x * blockDim.x + threadIdx.x;
+    if (s >= nS) return;
+    unsigned long long bits = 0;
+    const uint32_t q0 = D.pStart[s], q1 = D.pStart[s + 1];
+    if (q0 < q1) {
+        uint32_t a0 = 0, a1 = 0;
+        scene_planes(P, own[sph[s].owner].scene, a0, a1);
+        for (uint32_t q = q0; q < q1; q++)
+            if (D.pOn[q]) bits |= 1ull << (D.pPlane[q] - a0);
+    }
+    planeBits[s] = bits;
+    numAnal[s] = (uint32_t)__popcll(bits);
+}
+
+// ... last: the candidates' histories to the list (contact indices in cidx; a sphere's plane contacts head its row).
+__global__ __launch_bounds__(256) void k_direct_leave(DirectList D, uint32_t pairBlocks,
+                                                      const uint32_t* __restrict__ cidx,
+                                                      const uint32_t* __restrict__ rowStart,
+                                                      float4* __restrict__ listHist, SpecGuard guard) {
+    if (spec_skip(guard)) return;
+    if (blockIdx.x < pairBlocks) {
+        const uint32_t c = blockIdx.x * 256u + threadIdx.x;
+        if (c < D.nPair && D.on[c]) listHist[cidx[c]] = D.hist[c];
+        return;
+    }
+    const uint32_t q = (blockIdx.x - pairBlocks) * 256u + threadIdx.x;
+    if (q >= D.nPlane || !D.pOn[q]) return;
+    const uint32_t s = D.pSph[q];
+    uint32_t k = 0;
+    for (uint32_t j = D.pStart[s]; j < q; j++) k += D.pOn[j];
+    listHist[rowStart[s] + k] = D.pHist[q];
+}
+
+inline uint32_t blocks(uint64_t n) { return (uint32_t)((n + 255) / 256); }
+
+}  // namespace
+
+hipError_t launch_direct_near(const KParams& P, const SphereRec* sph, const OwnerRec* own, uint32_t nS,
+                              const PlanePose* pose, uint32_t nA, double margin, unsigned long long* nearBits,
+                              uint32_t* nearCnt, hipStream_t st) {
+    if (nS == 0) return hipSuccess;
+    k_direct_near<<<blocks(nS), 256, 0, st>>>(P, sph, own, nS, pose, nA, margin, nearBits, nearCnt);
+    return hipGetLastError();
+}
+
+hipError_t launch_direct_plane_rows(const KParams& P, const SphereRec* sph, const OwnerRec* own, uint32_t nS,
+                                    const unsigned long long* nearBits, const uint32_t* pStart, uint32_t* pSph,
+                                    uint32_t* pPlane, const PlanePose* pose, uint32_t nA, PlanePose* pose0,
+                                    hipStream_t st) {
+    if (nS == 0) return hipSuccess;
+    k_direct_plane_rows<<<blocks(nS), 256, 0, st>>>(P, sph, own, nS, nearBits, pStart, pSph, pPlane, pose, nA, pose0);
+    return hipGetLastError();
+}
+
+hipError_t launch_direct_enter(const DirectList& D, const uint32_t* cidx, const uint32_t* rowStart, const uint32_t* idB,
+                               const uint8_t* ctype, const float4* listHist, hipStream_t st) {
+    const uint32_t pb = blocks(D.nPair), g = pb + blocks(D.nPlane);
+    if (g == 0) return hipSuccess;
+    k_direct_enter<<<g, 256, 0, st>>>(D, pb, cidx, rowStart, idB, ctype, listHist);
+    return hipGetLastError();
+}
+
+hipError_t launch_direct_join(uint32_t nS, const uint32_t* oldStart, const uint32_t* oldB, const uint32_t* newStart,
+                              const uint32_t* newB, const uint32_t* oldPStart, const uint32_t* oldPlane,
+                              const DirectList& O, const DirectList& D, hipStream_t st) {
+    if (nS == 0) return hipSuccess;
+    k_direct_join<<<blocks(nS), 256, 0, st>>>(nS, oldStart, oldB, newStart, newB, oldPStart, oldPlane, O, D);
+    return hipGetLastError();
+}
+
+hipError_t launch_direct_check(const KParams& P, const DirectCheck& C, const OwnerRec* own, uint32_t nS,
+                               const PlanePose* pose, uint32_t nA, DirectState* state, hipStream_t st) {
+    if (nS == 0) return hipSuccess;
+    k_direct_check<<<blocks(nS), 256, 0, st>>>(P, C, own, nS, pose, nA, state);
+    return hipGetLastError();
+}
+
+hipError_t launch_direct_plane_bits(const KParams& P, const SphereRec* sph, const OwnerRec* own, uint32_t nS,
+                                    const DirectList& D, uint32_t* numAnal, unsigned long long* planeBits,
+                                    uint32_t* clear, uint32_t nClear, hipStream_t st) {
+    if (nS == 0) return hipSuccess;
+    k_direct_plane_bits<<<blocks(nS), 256, 0, st>>>(P, sph, own, nS, D, numAnal, planeBits, clear, nClear);
+    return hipGetLastError();
+}
+
+hipError_t launch_direct_leave(const DirectList& D, const uint32_t* cidx, const uint32_t* rowStart, float4* listHist,
+                               hipStream_t st, SpecGuard guard) {
+    const uint32_t pb = blocks(D.nPair), g = pb + blocks(D.nPlane);
+    if (g == 0) return hipSuccess;
+    k_direct_leave<<<g, 256, 0, st>>>(D, pb, cidx, rowStart, listHist, guard);
+    return hipGetLastError();
+}
+
+}  // namespace deme_int

@@ -56,17 +56,25 @@ hipError_t launch_force(const KParams& P, uint32_t nC, const uint32_t* idA, cons
     return hipGetLastError();
 }
 
+hipError_t launch_force_direct(const KParams& P, const DirectList& D, const SphereRec* sph, const OwnerRec* own,
+                               const float4* moi, const deme_anal_obj* anal, const PlanePose* pose,
+                               const deme_material* mats, float* aTerm, float* bTerm, const PlaneSums& sums,
+                               hipStream_t st) {
+    deme_force_direct<<<direct_force_blocks(D), 256, 0, st>>>(P, D, sph, own, moi, anal, pose, mats, aTerm, bTerm, sums);
+    return hipGetLastError();
+}
+
 hipError_t launch_owner_update(const KParams& P, uint32_t nO, uint32_t nClumps, const uint32_t* ownerSphStart,
                                const uint32_t* rowStart, const uint32_t* bRowStart, const float* aTerm,
                                const float* bTerm, const uint8_t* aOn, const uint8_t* bOn, const PlaneSums& sums,
                                const PlaneRefresh& planes, const deme_family_rule* rules, OwnerRec* own, float* acc,
                                int doIntegrate, const double* clock, hipStream_t st, OwnerRec* ownOut,
-                               SpecGuard guard) {
+                               SpecGuard guard, const DirectList& direct, const DirectCheck& check) {
     if (nO == 0) return hipSuccess;
     if (sums.nOwners > MAX_ANAL_OWNERS) return hipErrorInvalidValue;
     deme_owner_update<<<owner_blocks(nClumps, sums.nOwners), 256, 0, st>>>(
         P, nO, nClumps, ownerSphStart, rowStart, bRowStart, aTerm, bTerm, aOn, bOn, sums, planes, rules, own,
-        ownOut ? ownOut : own, acc, doIntegrate, clock, guard);
+        ownOut ? ownOut : own, acc, doIntegrate, clock, guard, direct, check);
     return hipGetLastError();
 }
 

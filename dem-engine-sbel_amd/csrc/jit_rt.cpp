@@ -123,7 +123,7 @@ int jit_compile(const std::string& src, const std::string& arch, std::vector<cha
 void JitForce::release() {
     if (mod) (void)hipModuleUnload(mod);
     mod = nullptr;
-    full = terms = nullptr;
+    full = terms = direct = nullptr;
 }
 
 hipError_t JitForce::load(const std::vector<char>& code) {
@@ -134,7 +134,19 @@ hipError_t JitForce::load(const std::vector<char>& code) {
         return e;
     }
     if ((e = hipModuleGetFunction(&full, mod, "deme_force_full")) != hipSuccess) return e;
-    return hipModuleGetFunction(&terms, mod, "deme_force_terms");
+    if ((e = hipModuleGetFunction(&terms, mod, "deme_force_terms")) != hipSuccess) return e;
+    return hipModuleGetFunction(&direct, mod, "deme_force_direct");
+}
+
+hipError_t JitForce::launch_direct(const KParams& P, const DirectList& D, const SphereRec* sph, const OwnerRec* own,
+                                   const float4* moi, const deme_anal_obj* anal, const PlanePose* pose,
+                                   const deme_material* mats, float* aTerm, float* bTerm, const PlaneSums& sums,
+                                   hipStream_t st) const {
+    KParams p = P;
+    DirectList d = D;
+    PlaneSums ps = sums;
+    void* args[] = {&p, &d, &sph, &own, &moi, &anal, &pose, &mats, &aTerm, &bTerm, &ps};
+    return hipModuleLaunchKernel(direct, direct_force_blocks(D), 1, 1, 256, 1, 1, 0, st, args, nullptr);
 }
 
 hipError_t JitForce::launch(bool wantFull, const KParams& P, uint32_t nC, const uint32_t* idA, const uint32_t* idB,
@@ -174,14 +186,18 @@ hipError_t JitOwner::launch(const KParams& P, uint32_t nO, uint32_t nClumps, con
                             const float* bTerm, const uint8_t* aOn, const uint8_t* bOn, const PlaneSums& sums,
                             const PlaneRefresh& planes, const deme_family_rule* rules, const OwnerRec* own,
                             OwnerRec* ownOut, float* acc, int doIntegrate, const double* clock,
-                            hipStream_t st, SpecGuard guard) const {
+                            hipStream_t st, SpecGuard guard, const DirectList& direct,
+                            const DirectCheck& check) const {
     if (nO == 0) return hipSuccess;
     if (sums.nOwners > MAX_ANAL_OWNERS) return hipErrorInvalidValue;
     KParams p = P;
     PlaneSums ps = sums;
     PlaneRefresh pr = planes;
+    DirectList d = direct;
+    DirectCheck ck = check;
     void* args[] = {&p,   &nO,  &nClumps, &ownerSphStart, &rowStart, &bRowStart, &aTerm,       &bTerm, &aOn,  &bOn,
-                    &ps,  &pr,  &rules,   &own,           &ownOut,   &acc,       &doIntegrate, &clock, &guard};
+                    &ps,  &pr,  &rules,   &own,           &ownOut,   &acc,       &doIntegrate, &clock, &guard,
+                    &d,   &ck};
     return hipModuleLaunchKernel(fn, owner_blocks(nClumps, sums.nOwners), 1, 1, 256, 1, 1, 0, st, args, nullptr);
 }
 

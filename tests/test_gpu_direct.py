@@ -1,0 +1,169 @@
+"""Steps taken on the candidates between list builds (deme_step with detection every step and no drift margin) against
+the contact-list path (the cell sweep every pass): states, contact lists, persistent maps, histories and records bit for
+bit, over what a candidate may meet -- planes that move, masks and families that change on the way, scenes of a batch,
+user force models, spheres at the end of the bin grid, lists that go stale or die at once, empty systems -- and over
+calls too short to use them."""
+import numpy as np
+import pytest
+
+from deme_amd import scenes
+from deme_amd.abi import ANAL_DTYPE, RULE_DTYPE, DemeError, DeviceSystem
+
+pytestmark = pytest.mark.gpu
+
+LINEAR = """
+    const float vn = dot(ALinVel - BLinVel, B2A);
+    force = (float)(2e3 * overlapDepth) * B2A - (1.0f * vn) * B2A;
+    contact_age += ts;
+"""
+
+
+def _same(a, b):
+    sa, sb = a.get_state(), b.get_state()
+    for k in sa:
+        assert np.array_equal(sa[k], sb[k]), k
+    ca, cb = a.counts(), b.counts()
+    for k in ("nContacts", "nPrevContacts", "nSphereGeoContacts", "nSteps", "time"):
+        assert getattr(ca, k) == getattr(cb, k), k
+    for x, y in zip(a.contacts(), b.contacts()):
+        assert np.array_equal(x, y)
+    assert np.array_equal(a.wildcards(), b.wildcards())
+
+
+def _pair(sc, setup=None):
+    a, b = DeviceSystem(sc), DeviceSystem(sc)
+    b.set_skin(0.0)
+    for d in (a, b):
+        if setup:
+            setup(d)
+    return a, b
+
+
+def _clumps_masked():
+    sc = scenes.clump_settling(n_clumps=3001, box=(0.1, 0.1, 0.2), velocity_sigma=0.3, omega_sigma=20.0, seed=51)
+    fam = np.random.default_rng(1).integers(0, 3, sc.n_clumps)
+    sc.state["family"][:sc.n_clumps] = fam
+    sc.mask[1 * 2 // 2 + 0] = 1  # families 0 and 1 do not touch
+    sc.mask[2 * 3 // 2 + 2] = 1  # nor family 2 among itself
+    rule = "if (family_code == 1 && t > 2.4e-4f) newFamily = 2; else if (family_code == 2 && vel.z < -0.4f) newFamily = 0;"
+    return sc, lambda d: d.set_motion_rules(family_change_rules=rule)
+
+
+def _bed_fast_plate():
+    sc = scenes.polydisperse_bed(n=9001, seed=52, relax_iters=4, plate_speed=30.0, h=2e-6)
+    sc.state["vX"][:sc.n_clumps] = np.random.default_rng(2).normal(0, 0.3, sc.n_clumps)
+    return sc, None
+
+
+def _batch():
+    return scenes.batched_columns(n_scenes=7, total_scale=0.02, pitch_scale=0.8, seed=53), None
+
+
+def _model():
+    sc = scenes.sphere_settling(n=4003, spacing=1.98, velocity_sigma=0.3, omega_sigma=5.0, seed=54)
+
+    def setup(d):
+        d.set_force_model(LINEAR, ["contact_age"])
+        d.keep_contact_records(True)
+
+    return sc, setup
+
+
+def _rolling():
+    return scenes.sphere_settling(n=2500, spacing=1.98, velocity_sigma=0.5, omega_sigma=30.0, Crr=0.05, seed=55), None
+
+
+def _fast_gas():
+    # lists die within a few steps even at the widest automatic skin
+    return scenes.sphere_settling(n=2000, spacing=3.0, velocity_sigma=60.0, seed=56), None
+
+
+def _at_the_grid_end():
+    # a box an exact multiple of the bin size, spheres pressed into its upper walls: bin ranges end at the grid's end
+    r = 0.005
+    L = 0.16
+    g = np.stack(np.meshgrid(*[np.arange(15)] * 3, indexing="ij"), -1).reshape(-1, 3) * (2 * r * 0.995)
+    g = g - g.max(0) + (L / 2 - 0.98 * r)
+    vel = np.random.default_rng(3).normal(0, 0.1, g.shape)
+    return scenes.spheres_scene(g, r, (L, L, L), vel=vel), None
+
+
+def _apart():
+    # nothing in contact, no candidates: a grid of distant spheres without planes
+    g = np.stack(np.meshgrid(*[np.arange(4)] * 3, indexing="ij"), -1).reshape(-1, 3) * 0.05
+    return scenes.spheres_scene(g - g.mean(0), 0.002, (0.4, 0.4, 0.4), planes=False), None
+
+
+SCENES = {f.__name__[1:]: f for f in (_clumps_masked, _bed_fast_plate, _batch, _model, _rolling, _fast_gas,
+                                      _at_the_grid_end, _apart)}
+
+
+@pytest.mark.parametrize("skin", [None, 3e-5])
+@pytest.mark.parametrize("name", sorted(SCENES))
+def test_steps_on_the_candidates_equal_the_contact_list_path(name, skin):
+    sc, setup = SCENES[name]()
+    a, b = _pair(sc, setup)
+    if skin is not None:
+        a.set_skin(skin)
+    for chunk in (1, 5, 6, 7, 40, 1, 70):
+        a.step(chunk, 1)
+        b.step(chunk, 1)
+        _same(a, b)
+        if name == "model":
+            for x, y in zip(a.forces(), b.forces()):
+                assert np.array_equal(x, y)
+    if name not in ("apart",):
+        assert a.counts().nContacts > 20
+
+
+def test_a_plane_turned_into_the_bed_is_met():
+    """A fixed plane far from every sphere, rotated between calls by a new state: its spheres are listed anew."""
+    sc = scenes.sphere_settling(n=3000, spacing=1.99, velocity_sigma=0.2, seed=57)
+    nc = sc.n_clumps
+    extra = np.zeros(1, ANAL_DTYPE)
+    extra[0]["owner"] = nc + 1
+    extra[0]["relPos"] = (0.0, 0.0, -0.29)
+    extra[0]["rot"] = (0.0, 0.0, 1.0)
+    extra[0]["mass"] = 1e15
+    sc.anal = np.concatenate([sc.anal, extra])
+    sc.state = {q: np.concatenate([v, v[nc:nc + 1]]) for q, v in sc.state.items()}
+    sc.state["family"][nc + 1] = 9
+    rule = np.zeros(1, RULE_DTYPE)[0]
+    rule["used"] = rule["linVelPrescribed"] = rule["rotVelPrescribed"] = 1
+    rule["velSet"] = 0x3F
+    rule["vel"][:] = (0.0, 0.0, 0.0, 0.0, 400.0, 0.0)  # turns by 4 mrad a step
+    sc.rules[9] = rule
+    sc.n_owners = nc + 2
+    sc.owner_mass = np.append(sc.owner_mass, np.float32(1e15))
+    sc.owner_moi = np.ascontiguousarray(np.append(sc.owner_moi, np.full((1, 3), 1e15, np.float32), 0))
+    a, b = _pair(sc)
+    for chunk in (10, 30, 25):
+        a.step(chunk, 1)
+        b.step(chunk, 1)
+        _same(a, b)
+    st = a.get_state()
+    st["oriQw"][nc + 1], st["oriQx"][nc + 1] = np.float32(0.9), np.float32(np.sqrt(1 - 0.81))
+    for d in (a, b):
+        d.set_state(st)
+        d.step(20, 1)
+    _same(a, b)
+
+
+def test_a_sphere_leaving_the_world_fails_at_the_same_step():
+    g = np.stack(np.meshgrid(np.arange(6), np.arange(6), np.arange(3), indexing="ij"), -1).reshape(-1, 3) * 0.0098
+    xyz = np.concatenate([g - g.mean(0), [[0.0, 0.0, 0.04]]])
+    vel = np.zeros_like(xyz)
+    vel[-1] = (0.0, 0.0, 100.0)
+    sc = scenes.spheres_scene(xyz, 0.005, (0.1295, 0.1295, 0.1295), planes=False, vel=vel)
+    a, b = _pair(sc)
+    errors = []
+    for d in (a, b):
+        d.step(3, 1)
+        with pytest.raises(DemeError) as e:
+            d.step(400, 1)
+        errors.append(str(e.value))
+    assert errors[0] == errors[1]
+    assert a.counts().nSteps == b.counts().nSteps
+    sa, sb = a.get_state(), b.get_state()
+    for k in sa:
+        assert np.array_equal(sa[k], sb[k]), k
