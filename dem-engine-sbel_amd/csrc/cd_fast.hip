@@ -549,13 +549,6 @@ __global__ __launch_bounds__(256) void k_cell_rows(KParams P, const SphereRec* _
     for (uint32_t q = st; q < en; q++) idA[q] = s;
 }
 
-// A build position coordinate in fixed point (scale = 1 / unit): rounded to the nearest unit, INT32_MIN when it does
-// not fit in (-2^31, 2^31) units (a NaN fails both comparisons).
-__device__ __forceinline__ int32_t build_fix(double x, double scale) {
-    const double v = rint(x * scale);
-    return (v > -2147483648.0 && v < 2147483648.0) ? (int32_t)v : INT32_MIN;
-}
-
 // Candidate lists from a candidate build: sphere s's row of higher-id partners within the skin (ascending), copied
 // from its slab column at its sorted position; the sphere's position at the build is kept (in fixed point) for the
 // displacement test.

@@ -174,13 +174,22 @@ struct deme_ctx {
     // planesGen: the build (candBuilds) the plane candidates go with. directSkip: calls of deme_step that do not try
     // (after a state near the grid's end, doubling up to 64 while that repeats).
     DBuf<DirectState> dstate;
-    DirectState* hdstate = nullptr;  // pinned mirror
+    struct HostStatus {
+        DirectState d;
+        SkinStats stats;
+    };
+    HostStatus* hdstate = nullptr;  // pinned mirrors
     DBuf<float4> dHist, dHistOld, dPHist, dPHistOld;
     DBuf<uint8_t> dPOn, dPOnOld, dOnOld;
     DBuf<uint32_t> pStart, pStartOld, pSph, pPlane, pPlaneOld, candStartOld, candBOld;
     DBuf<float> pTerm;
     DBuf<unsigned long long> nearBits;
     DBuf<PlanePose> pose0;
+    DBuf<OwnerBuild> own0;  // the owners' poses at the build
+    DBuf<SkinStats> skinStats;
+    // the automatic skin chosen from a build's statistics for the next build (0: none chosen), and the largest
+    // displacement per step seen lately (0: unknown)
+    double skinNext = 0.0, skinNextRatio = 1.0, stepMove = 0.0;  // (its candidates over the current lists')
     uint32_t nPlane = 0;
     uint64_t planesGen = 0;
     uint32_t directSkip = 0, directBackoff = 0;
@@ -285,6 +294,7 @@ struct deme_ctx {
     CellGrid grid{};
     uint64_t nCells = 0;
     float maxRadius = 0.f, meanRadius = 0.f;
+    float maxRel = 0.f;  // largest distance of a sphere's centre from its owner
     uint32_t slabCap = 32;
     double cellScale = 1.0;  // cell edge = cellScale x the largest interaction distance (>= 1)
     DBuf<uint32_t> cellCount, cellStart, cellOf, slotOf, posOf, aCnt, survSlab, rowSlab, mirSlab;
@@ -481,7 +491,7 @@ int deme_ctx_create(int device, void* stream, deme_ctx** out) {
     if (c->ctr.ensure(1, 1.0) != hipSuccess || c->clock.ensure(1, 1.0) != hipSuccess ||
         c->dstate.ensure(1, 1.0) != hipSuccess ||
         hipHostMalloc((void**)&c->hctr, sizeof(DevCounters), hipHostMallocDefault) != hipSuccess ||
-        hipHostMalloc((void**)&c->hdstate, sizeof(DirectState), hipHostMallocDefault) != hipSuccess) {
+        hipHostMalloc((void**)&c->hdstate, sizeof(deme_ctx::HostStatus), hipHostMallocDefault) != hipSuccess) {
         deme_ctx_destroy(c);
         return DEME_ERR_HIP;
     }
@@ -544,7 +554,8 @@ int deme_ctx_destroy(deme_ctx* c) {
     c->dstate.release(); c->dHist.release(); c->dHistOld.release(); c->dPHist.release(); c->dPHistOld.release();
     c->dPOn.release(); c->dPOnOld.release(); c->dOnOld.release(); c->pStart.release(); c->pStartOld.release();
     c->pSph.release(); c->pPlane.release(); c->pPlaneOld.release(); c->candStartOld.release(); c->candBOld.release();
-    c->pTerm.release(); c->nearBits.release(); c->pose0.release();
+    c->pTerm.release(); c->nearBits.release(); c->pose0.release(); c->own0.release();
+    c->skinStats.release();
     if (c->hdstate) (void)hipHostFree(c->hdstate);
     if (c->hctr) (void)hipHostFree(c->hctr);
     if (c->evCounts) (void)hipEventDestroy(c->evCounts);
@@ -622,7 +633,7 @@ int deme_upload_templates(deme_ctx* c, uint32_t nS, const uint32_t* sphOwner, co
     std::vector<SphereRec> hs(nS);
     std::vector<uint32_t> start(nClumps + 1, 0);
     uint32_t maxMat = 0;
-    float maxR = 0.f;
+    float maxR = 0.f, maxRel = 0.f;
     for (uint32_t s = 0; s < nS; s++) {
         maxMat = std::max<uint32_t>(maxMat, sphMat[s]);
         if (sphOwner[s] >= nClumps) return c->fail(DEME_ERR_INVALID_ARGUMENT, "sphere owner is not a clump");
@@ -637,6 +648,7 @@ int deme_upload_templates(deme_ctx* c, uint32_t nS, const uint32_t* sphOwner, co
         hs[s].ry = sphRelPos[3 * s + 1];
         hs[s].rz = sphRelPos[3 * s + 2];
         hs[s].mat = sphMat[s];
+        maxRel = std::max(maxRel, std::hypot(std::hypot(hs[s].rx, hs[s].ry), hs[s].rz));
         hs[s].pad0 = hs[s].pad1 = 0;
         start[sphOwner[s] + 1]++;
     }
@@ -682,6 +694,7 @@ int deme_upload_templates(deme_ctx* c, uint32_t nS, const uint32_t* sphOwner, co
     c->maxMatSph = maxMat;
     c->maxMat = std::max(c->maxMatSph, c->maxMatAnal);
     c->maxRadius = maxR;
+    c->maxRel = maxRel;
     c->hostRadius.assign(sphRadius, sphRadius + nS);
     c->meanRadius = mean_radius(c->hostRadius);
     c->needDetect = false;
@@ -1188,7 +1201,11 @@ static double stale_limit2(const deme_ctx* c) {
 // Candidate lists from the current state: the cell sweep in its build mode (pairs of different owners within the
 // skin of touching), rows of higher-id partners in id order (candStart / candB) and the build positions (pos0).
 static int build_candidates(deme_ctx* c) {
-    if (c->skinSet < 0.0 && c->candBuilds > 0 && c->candValid) {
+    if (c->skinSet < 0.0 && c->skinNext > 0.0) {
+        c->skinAuto = c->skinNext;  // (chosen from the statistics of the lists being retired)
+        c->skinCostPrev = -1.0;
+        c->skinDir = 0;
+    } else if (c->skinSet < 0.0 && c->candBuilds > 0 && c->candValid) {
         // the retiring lists' lifetime and size judge their skin (lists dropped for other reasons -- a host change,
         // a return from the cell sweep -- do not)
         constexpr double BUILD_PASSES = 2.7;
@@ -1216,6 +1233,7 @@ static int build_candidates(deme_ctx* c) {
         c->skinCostPrev = cost;
         c->skinAuto = std::min(std::max(next, 0.05 * m), 0.8 * m);
     }
+    c->skinNext = 0.0;
     c->lastLifetime = c->candBuilds > 0 ? c->passesSinceBuild : ~0ull;
     c->builtThisPass = true;
     c->passesSinceBuild = 0;
@@ -1265,7 +1283,9 @@ static int build_candidates(deme_ctx* c) {
         DEME_HIP(c, c->cidx[k].ensure(nK));
     }
     // the build positions (in fixed point, posUnit) are the reference: no displacement, no common translation yet
-    DEME_LAUNCH(c, "fill", launch_fill_u32(reinterpret_cast<uint32_t*>(c->dispRef.p), 12, 0, c->stream));
+    DEME_HIP(c, c->skinStats.ensure(1, 1.0));
+    DEME_LAUNCH(c, "fill", launch_fill_u32(reinterpret_cast<uint32_t*>(c->dispRef.p), 12, 0, c->stream,
+                                           reinterpret_cast<uint32_t*>(c->skinStats.p), sizeof(SkinStats) / 4));
     DEME_LAUNCH(c, "cand_rows",
                 launch_cand_rows(nS, c->rowSlab.p, c->candStart.p, c->candA.p, c->candB.p, c->sorted.p, c->pos0.p,
                                  1.0 / c->posUnit, c->stream));
@@ -1278,6 +1298,9 @@ static int build_candidates(deme_ctx* c) {
     DEME_LAUNCH(c, "cand_tscatter",
                 launch_cand_tscatter(nK32, c->candB.p, c->cidx[0].p, c->tStart.p, c->tC.p, c->stream));
     DEME_LAUNCH(c, "cand_tsort", launch_cand_tsort(nS, c->tStart.p, c->tC.p, c->tPos.p, c->stream));
+    DEME_HIP(c, c->own0.ensure(std::max<uint32_t>(c->nClumps, 1)));
+    DEME_LAUNCH(c, "owner_build", launch_owner_build(c->kp, c->sph.p, c->own.p, c->ownerSphStart.p, c->nClumps,
+                                                     1.0 / c->posUnit, c->own0.p, c->skinStats.p, c->stream));
     c->candValid = true;
     c->rebuildNext = false;
     c->candBuilds++;
@@ -1962,13 +1985,14 @@ constexpr double PLANE_MARGIN = 1.5, PLANE_MOTION = 0.45;
 
 static DirectCheck direct_check(const deme_ctx* c) {
     DirectCheck k{};
-    k.sph = c->sph.p;
-    k.pos0 = c->pos0.p;
+    k.own0 = c->own0.p;
     k.unit = c->posUnit;
-    k.limit2 = stale_limit2(c);
+    k.limit = std::sqrt(stale_limit2(c));
     const double rmax = (double)c->maxRadius, bs = c->sp.binSize;
-    // a contact point strays from its spheres by under 1e-6 of the radii: limits a hundred times that below the end
-    auto hi = [&](uint32_t nb) { return (double)nb * bs * (1.0 - 1e-12) - 1e-4 * rmax; };
+    // an owner's spheres reach maxRel + r past it; a contact point strays from its spheres by under 1e-6 of the radii
+    // (the limits leave a hundred times that)
+    const double past = (double)c->maxRel * 1.00001 + rmax * 1.0001 + (double)c->sp.beta;
+    auto hi = [&](uint32_t nb) { return (double)nb * bs * (1.0 - 1e-12) - past; };
     const double span = 2.0 * (rmax + (double)c->sp.beta) / bs + 2.0;
     const bool fits = span * span * span <= 65535.0;
     k.hiX = fits ? hi(c->sp.nbX) : -INFINITY;
@@ -1987,7 +2011,55 @@ static int direct_clear_state(deme_ctx* c) {
     return DEME_OK;
 }
 
-// The plane candidates of the current state and the buffers of both kinds of candidates.
+// Seconds of a step on k candidates and of a build, fitted to 600 spheres to 1M clumps: the launches, then 70 ps a
+// candidate; a build some 25 launches and three waits, then about three steps over its candidates.
+static double direct_step_s(double k) { return 14e-6 + 70e-12 * k; }
+static double direct_build_s(double k) { return 300e-6 + 3.0 * 70e-12 * k; }
+
+// The automatic skin the statistics of the lists in force ask for: the smallest time per step, builds included, among
+// sixteenths of their skin and 1.25 and 1.5 times it, a build coming every time the fastest sphere moves half the skin.
+// *candRatio: its candidates over the current lists'. (1M clumps moving at 0.02 m/s: 0.2 r lists 4.98M candidates, 352 us
+// a step; the skin chosen 4.40M, 269 us.)
+static double choose_skin(const deme_ctx* c, const SkinStats& st, double* candRatio) {
+    const double s = c->skin(), m = (double)c->meanRadius;
+    float speed;
+    std::memcpy(&speed, &st.speedBits, sizeof(speed));
+    const double move = std::max({(double)speed * (double)c->sp.h, c->stepMove, 1e-30});
+    double total = 0.0;
+    for (uint32_t g : st.gaps) total += g;
+    *candRatio = 1.0;
+    if (!(total > 0.0) || !std::isfinite(move)) return s;
+    const double nK = (double)c->nCand;
+    auto cost = [&](double k, double skin) {
+        return direct_step_s(k * nK) + direct_build_s(k * nK) / std::max(0.5 * skin / move, 1.0);
+    };
+    double best = cost(1.0, s), bestSkin = s, below = 0.0;
+    for (uint32_t j = 1; j < SKIN_BUCKETS; j++) {
+        below += st.gaps[j - 1] / total;
+        const double skin = s * j / SKIN_BUCKETS;
+        if (skin < 0.01 * m) continue;
+        if (cost(below, skin) < best) {
+            best = cost(below, skin);
+            bestSkin = skin;
+            *candRatio = below;
+        }
+    }
+    // beyond the skin the lists say nothing: the count grows on as over their last quarter, somewhat faster
+    double last = 0.0;
+    for (uint32_t j = SKIN_BUCKETS - SKIN_BUCKETS / 4; j < SKIN_BUCKETS; j++) last += st.gaps[j] / total;
+    for (int q = 1; q <= 2; q++) {
+        const double skin = s * (1.0 + 0.25 * q), k = 1.0 + 1.2 * last * q;
+        if (skin <= 0.8 * m && cost(k, skin) < best) {
+            best = cost(k, skin);
+            bestSkin = skin;
+            *candRatio = k;
+        }
+    }
+    return bestSkin;
+}
+
+// The plane candidates of the current state and the buffers of both kinds of candidates; with a new build also the skin
+// the next one should take (skinNext).
 static int direct_planes(deme_ctx* c) {
     const uint32_t nS = c->nS;
     int r = ensure_poses(c);
@@ -2001,7 +2073,18 @@ static int direct_planes(deme_ctx* c) {
                                                          PLANE_MARGIN * c->skin(), c->nearBits.p, c->aCnt.p, c->stream));
         DEME_LAUNCH(c, "direct_scan", scan_u32(c->aCnt.p, nullptr, nS, c->pStart.p, &c->ctr.p->total[2],
                                                c->scanScratch.p, c->stream));
+        const bool choose = c->skinSet < 0.0;
+        if (choose) {
+            DEME_LAUNCH(c, "gap_hist", launch_gap_hist(c->kp, c->sph.p, c->own.p, c->candA.p, c->candB.p,
+                                                       (uint32_t)c->nCand, c->skin(), c->skinStats.p, c->stream));
+            DEME_HIP(c, hipMemcpyAsync(&c->hdstate->stats, c->skinStats.p, sizeof(SkinStats), hipMemcpyDeviceToHost,
+                                       c->stream));
+        }
         if ((r = readback_counters(c))) return r;
+        if (choose) {
+            const double s = choose_skin(c, c->hdstate->stats, &c->skinNextRatio);
+            c->skinNext = s != c->skin() ? s : 0.0;
+        }
         const uint64_t n = c->hctr->total[2];
         if (n > 0xFFFFFFFFull) return c->fail(DEME_ERR_CAPACITY, "plane candidate count exceeds 2^32 - 1");
         c->nPlane = (uint32_t)n;
@@ -2033,7 +2116,7 @@ static int direct_enter(deme_ctx* c) {
     const int cu = c->cur;
     DEME_LAUNCH(c, "direct_enter", launch_direct_enter(direct_list(c), c->cidx[cu].p, c->rowStart[cu].p, c->idB[cu].p,
                                                        c->ctype[cu].p, c->hist[cu].p, c->stream));
-    DEME_LAUNCH(c, "direct_check", launch_direct_check(c->kp, direct_check(c), c->own.p, c->nS, c->pose.p, c->nA,
+    DEME_LAUNCH(c, "direct_check", launch_direct_check(c->kp, direct_check(c), c->own.p, c->nClumps, c->pose.p, c->nA,
                                                        c->dstate.p, c->stream));
     return DEME_OK;
 }
@@ -2133,12 +2216,27 @@ static int run_direct(deme_ctx* c, int n, int* done, bool* again) {
     if (c->jitActive && c->jitStale && (r = jit_rebuild(c))) return r;
     if ((r = direct_enter(c))) return r;
     bool rebuilt = false, giveUp = false;
-    double dispMax2 = 0.0;
+    double dispMax = 0.0;
     uint32_t counted = 0;
     while (*done < n) {
+        // a skin with clearly fewer candidates is taken at once when it pays for the build within its lifetime or the
+        // rest of the call
+        if (c->skinNext > 0.0 && c->skinNext < c->skin() && !rebuilt) {
+            const double life = 0.5 * c->skinNext / std::max(c->stepMove, 1e-30), nK = (double)c->nCand;
+            const double gain = direct_step_s(nK) - direct_step_s(nK * c->skinNextRatio);
+            if (gain * std::min((double)(n - *done), life) > 1.5 * direct_build_s(nK * c->skinNextRatio)) {
+                if ((r = direct_rebuild(c))) {
+                    c->contactsReady = c->havePrev = c->candValid = false;
+                    return r;
+                }
+                rebuilt = true;
+                dispMax = 0.0;
+                counted = 0;
+            }
+        }
         // steps expected before the lists go stale: by the displacement so far, else by the last lists' lifetime
         const DirectCheck check = direct_check(c);
-        const double m = (double)c->passesSinceBuild, frac = std::max(std::sqrt(dispMax2 / check.limit2), 0.125);
+        const double m = (double)c->passesSinceBuild, frac = std::max(dispMax / check.limit, 0.125);
         double expect = m > 0 ? m / frac - m : (c->lastLifetime < 1000 ? (double)c->lastLifetime : 8.0);
         const int batch = std::min(n - *done, (int)std::min(std::max(0.9 * expect, 2.0), 32.0));
         const DirectList d = direct_list(c);
@@ -2166,10 +2264,10 @@ static int run_direct(deme_ctx* c, int n, int* done, bool* again) {
                                                   c->rules.p, c->own.p, c->acc.p, 1, c->clock.p, c->stream, nullptr,
                                                   SpecGuard(), d, check));
         }
-        DEME_HIP(c, hipMemcpyAsync(c->hdstate, c->dstate.p, sizeof(DirectState), hipMemcpyDeviceToHost, c->stream));
+        DEME_HIP(c, hipMemcpyAsync(&c->hdstate->d, c->dstate.p, sizeof(DirectState), hipMemcpyDeviceToHost, c->stream));
         DEME_HIP(c, hipStreamSynchronize(c->stream));
-        const uint32_t steps = c->hdstate->steps - counted, err = c->hdstate->err;
-        counted = c->hdstate->steps;
+        const uint32_t steps = c->hdstate->d.steps - counted, err = c->hdstate->d.err;
+        counted = c->hdstate->d.steps;
         for (uint32_t k = 0; k < steps; k++) {
             c->time += (double)c->sp.h;
             c->nSteps++;
@@ -2177,12 +2275,14 @@ static int run_direct(deme_ctx* c, int n, int* done, bool* again) {
         *done += (int)steps;
         c->passesSinceBuild += steps;
         if (c->passesSinceBuild >= 4) c->cellBackoff = 0;
-        dispMax2 = 0.0;
-        for (unsigned long long b : c->hdstate->disp2) {
+        dispMax = 0.0;
+        for (unsigned long long b : c->hdstate->d.disp) {
             double v;
             std::memcpy(&v, &b, sizeof(v));
-            dispMax2 = std::max(dispMax2, v);
+            dispMax = std::max(dispMax, v);
         }
+        if (c->passesSinceBuild >= 4)
+            c->stepMove = std::max(dispMax, 0.125 * check.limit) / (double)c->passesSinceBuild;
         if (err & ERRBIT_STALE) c->rebuildNext = true;
         if (err & ~(uint32_t)ERRBIT_STALE) {
             c->directBackoff = std::min<uint32_t>(std::max<uint32_t>(2 * c->directBackoff, 1), 64);
@@ -2210,7 +2310,7 @@ static int run_direct(deme_ctx* c, int n, int* done, bool* again) {
             return r;
         }
         rebuilt = true;
-        dispMax2 = 0.0;
+        dispMax = 0.0;
         counted = 0;
     }
     if (*done > 0 || rebuilt) {
@@ -2314,6 +2414,7 @@ int deme_set_skin(deme_ctx* c, double skin) {
     c->skinSet = skin < 0.0 ? -1.0 : skin;
     c->skinAuto = 0.0;
     c->skinCostPrev = -1.0;
+    c->skinNext = c->stepMove = 0.0;
     c->skinDir = 0;
     c->cellPassesLeft = 0;
     c->cellBackoff = 0;
@@ -2930,7 +3031,7 @@ int deme_append_clumps(deme_ctx* c, uint32_t nNewSph, const uint32_t* sphOwner, 
     std::vector<SphereRec> hs(nNewSph);
     std::vector<uint32_t> cnt(nNew, 0);
     uint32_t maxMat = c->maxMatSph;
-    float maxR = c->maxRadius;
+    float maxR = c->maxRadius, maxRel = c->maxRel;
     for (uint32_t k = 0; k < nNewSph; k++) {
         if (sphOwner[k] >= nNew) return c->fail(DEME_ERR_INVALID_ARGUMENT, "sphere owner is not an appended clump");
         if (k > 0 && sphOwner[k] < sphOwner[k - 1])
@@ -2946,6 +3047,7 @@ int deme_append_clumps(deme_ctx* c, uint32_t nNewSph, const uint32_t* sphOwner, 
         h.rz = sphRelPos[3 * k + 2];
         h.mat = sphMat[k];
         h.pad0 = h.pad1 = 0;
+        maxRel = std::max(maxRel, std::hypot(std::hypot(h.rx, h.ry), h.rz));
         cnt[sphOwner[k]]++;
         maxMat = std::max<uint32_t>(maxMat, sphMat[k]);
         maxR = std::max(maxR, sphRadius[k]);
@@ -3051,6 +3153,7 @@ int deme_append_clumps(deme_ctx* c, uint32_t nNewSph, const uint32_t* sphOwner, 
     c->nClumps = nC;
     c->maxMatSph = maxMat;
     c->maxMat = std::max(c->maxMatSph, c->maxMatAnal);
+    c->maxRel = maxRel;
     if (maxR > c->maxRadius) c->nCells = 0;  // re-derive the cell grid for the larger spheres
     c->maxRadius = maxR;
     c->scenesDirty = true;
@@ -3102,6 +3205,7 @@ int deme_change_clump_sizes(deme_ctx* c, uint32_t n, const uint32_t* ids, const 
         if (mark[owner[i]]) c->hostRadius[i] *= f[owner[i]];
         maxR = std::max(maxR, c->hostRadius[i]);
     }
+    c->maxRel *= std::max(1.f, *std::max_element(f.begin(), f.end()));  // (a bound)
     if (maxR != c->maxRadius) c->nCells = 0;
     c->maxRadius = maxR;
     c->meanRadius = mean_radius(c->hostRadius);

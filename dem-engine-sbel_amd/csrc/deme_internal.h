@@ -35,6 +35,20 @@ using deme_dev::INSPECT_MAX;
 using deme_dev::INSPECT_MIN;
 using deme_dev::INSPECT_SUM;
 
+// A build position coordinate in fixed point (scale = 1 / unit): rounded to the nearest unit, INT32_MIN when it does
+// not fit in (-2^31, 2^31) units (a NaN fails both comparisons).
+__device__ __forceinline__ int32_t build_fix(double x, double scale) {
+    const double v = rint(x * scale);
+    return (v > -2147483648.0 && v < 2147483648.0) ? (int32_t)v : INT32_MIN;
+}
+
+constexpr uint32_t SKIN_BUCKETS = 16, SKIN_SAMPLES = 65536;
+struct SkinStats {
+    uint32_t gaps[SKIN_BUCKETS];
+    uint32_t speedBits;
+    uint32_t pad[3];
+};
+
 // Uniform cell grid over the simulation world used to generate candidate pairs (edge >= largest interaction
 // distance, so partners lie in the 27 neighbouring cells).
 struct CellGrid {
@@ -58,6 +72,7 @@ using deme_dev::MAX_ANAL_OWNERS;
 using deme_dev::DirectCheck;
 using deme_dev::DirectList;
 using deme_dev::DirectState;
+using deme_dev::OwnerBuild;
 using deme_dev::PART_FROM_COUNTERS;
 using deme_dev::PlaneRefresh;
 using deme_dev::PlaneSums;
@@ -263,7 +278,14 @@ hipError_t launch_direct_enter(const DirectList& D, const uint32_t* cidx, const 
 hipError_t launch_direct_join(uint32_t nS, const uint32_t* oldStart, const uint32_t* oldB, const uint32_t* newStart,
                               const uint32_t* newB, const uint32_t* oldPStart, const uint32_t* oldPlane,
                               const DirectList& O, const DirectList& D, hipStream_t st);
-hipError_t launch_direct_check(const KParams& P, const DirectCheck& C, const OwnerRec* own, uint32_t nS,
+hipError_t launch_owner_build(const KParams& P, const SphereRec* sph, const OwnerRec* own,
+                              const uint32_t* ownerSphStart, uint32_t nClumps, double scale, OwnerBuild* own0,
+                              SkinStats* stats, hipStream_t st);
+// What the choice of a skin reads of a build: the candidates' gaps in sixteenths of the skin (a sample of at most
+// SKIN_SAMPLES) and the largest speed of a sphere (bits of a float).
+hipError_t launch_gap_hist(const KParams& P, const SphereRec* sph, const OwnerRec* own, const uint32_t* candA,
+                           const uint32_t* candB, uint32_t nK, double skin, SkinStats* stats, hipStream_t st);
+hipError_t launch_direct_check(const KParams& P, const DirectCheck& C, const OwnerRec* own, uint32_t nClumps,
                                const PlanePose* pose, uint32_t nA, DirectState* state, hipStream_t st);
 hipError_t launch_direct_plane_bits(const KParams& P, const SphereRec* sph, const OwnerRec* own, uint32_t nS,
                                     const DirectList& D, uint32_t* numAnal, unsigned long long* planeBits,

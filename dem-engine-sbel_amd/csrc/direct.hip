@@ -142,18 +142,91 @@ __global__ __launch_bounds__(256) void k_direct_join(uint32_t nS, const uint32_t
                  D.pHist);
 }
 
+// An owner's pose at a candidate build (coordinates in fixed point as the spheres' build positions); returns a bound of
+// its spheres' speed.
+__device__ __forceinline__ float owner_build(const KParams& P, const SphereRec* __restrict__ sph,
+                                             const OwnerRec* __restrict__ own,
+                                             const uint32_t* __restrict__ ownerSphStart, uint32_t o, double scale,
+                                             OwnerBuild* __restrict__ own0) {
+    const OwnerRec r = load_owner(own, o);
+    double X, Y, Z;
+    owner_position(P, r.voxel, r.lx, r.ly, r.lz, X, Y, Z);
+    float rel2 = 0.f;
+    for (uint32_t s = ownerSphStart[o]; s < ownerSphStart[o + 1]; s++) {
+        const SphereRec sr = load_sphere(sph, s);
+        rel2 = fmaxf(rel2, sr.rx * sr.rx + sr.ry * sr.ry + sr.rz * sr.rz);
+    }
+    OwnerBuild b;
+    b.x = build_fix(X, scale);
+    b.y = build_fix(Y, scale);
+    b.z = build_fix(Z, scale);
+    b.relMax = rel2 > 0.f ? sqrtf(rel2) * 1.000001f : 0.f;  // (rounded up)
+    b.qw = r.qw;
+    b.qx = r.qx;
+    b.qy = r.qy;
+    b.qz = r.qz;
+    uint4* dst = reinterpret_cast<uint4*>(own0 + o);
+    const uint4* src = reinterpret_cast<const uint4*>(&b);
+    dst[0] = src[0];
+    dst[1] = src[1];
+    const float v = sqrtf(r.vx * r.vx + r.vy * r.vy + r.vz * r.vz);
+    const float w = sqrtf(r.wx * r.wx + r.wy * r.wy + r.wz * r.wz);
+    return v + w * b.relMax;
+}
+
+__global__ __launch_bounds__(256) void k_owner_build(KParams P, const SphereRec* __restrict__ sph,
+                                                     const OwnerRec* __restrict__ own,
+                                                     const uint32_t* __restrict__ ownerSphStart, uint32_t nClumps,
+                                                     double scale, OwnerBuild* __restrict__ own0,
+                                                     SkinStats* __restrict__ stats) {
+    const uint32_t o = blockIdx.x * blockDim.x + threadIdx.x;
+    // the largest speed of a sphere (bounded by |v| + |w| relMax), for the choice of the skin
+    float speed = 0.f;
+    if (o < nClumps) speed = owner_build(P, sph, own, ownerSphStart, o, scale, own0);
+#pragma unroll
+    for (int off = 32; off > 0; off >>= 1) speed = fmaxf(speed, __shfl_xor(speed, off, 64));
+    // (only a wave above what stands there already goes to the one address: every wave of 1M owners did, 274 us)
+    const uint32_t bits = __float_as_uint(speed);
+    if ((threadIdx.x & 63u) == 0 && bits > __hip_atomic_load(&stats->speedBits, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT))
+        atomicMax(&stats->speedBits, bits);
+}
+
+// How the candidates' gaps are spread over the skin: a sample of them (every stride-th), gaps in sixteenths of the skin.
+__global__ __launch_bounds__(256) void k_gap_hist(KParams P, const SphereRec* __restrict__ sph,
+                                                  const OwnerRec* __restrict__ own, const uint32_t* __restrict__ candA,
+                                                  const uint32_t* __restrict__ candB, uint32_t nK, uint32_t stride,
+                                                  double skin, SkinStats* __restrict__ stats) {
+    __shared__ uint32_t h[SKIN_BUCKETS];
+    if (threadIdx.x < SKIN_BUCKETS) h[threadIdx.x] = 0;
+    __syncthreads();
+    const uint64_t c = ((uint64_t)blockIdx.x * 256u + threadIdx.x) * stride;
+    if (c < nK) {
+        const SphereRec a = load_sphere(sph, candA[c]), b = load_sphere(sph, candB[c]);
+        const OwnerRec oa = load_owner(own, a.owner), ob = load_owner(own, b.owner);
+        double ax, ay, az, bx, by, bz;
+        sphere_position(P, oa, a, ax, ay, az);
+        sphere_position(P, ob, b, bx, by, bz);
+        const double dx = ax - bx, dy = ay - by, dz = az - bz;
+        const double gap = sqrt(dx * dx + dy * dy + dz * dz) - ((double)a.r + (double)b.r + 2.0 * (double)P.beta);
+        const double k = gap / skin * SKIN_BUCKETS;
+        atomicAdd(&h[k > 0.0 ? (k < SKIN_BUCKETS ? (uint32_t)k : SKIN_BUCKETS - 1) : 0u], 1u);
+    }
+    __syncthreads();
+    if (threadIdx.x < SKIN_BUCKETS && h[threadIdx.x]) atomicAdd(&stats->gaps[threadIdx.x], h[threadIdx.x]);
+}
+
 // The check of a state the owner update did not leave itself (a call's first step on the candidates).
 __global__ __launch_bounds__(256) void k_direct_check(KParams P, DirectCheck C, const OwnerRec* __restrict__ own,
-                                                      uint32_t nS, const PlanePose* __restrict__ pose, uint32_t nA,
+                                                      uint32_t nClumps, const PlanePose* __restrict__ pose, uint32_t nA,
                                                       DirectState* st) {
-    const uint32_t s = blockIdx.x * blockDim.x + threadIdx.x;
-    double d2 = 0.0;
+    const uint32_t o = blockIdx.x * blockDim.x + threadIdx.x;
+    double disp = 0.0;
     uint32_t bad = 0;
-    if (s < nS) bad = direct_check_sphere(P, C, load_owner(own, C.sph[s].owner), s, d2);
+    if (o < nClumps) bad = direct_check_owner(P, C, load_owner(own, o), o, disp);
     if (blockIdx.x == 0)
         for (uint32_t a = threadIdx.x; a < nA; a += 256)
             if (direct_plane_moved(C, pose[a], C.pose0[a])) bad |= ERRBIT_STALE;
-    direct_report(st, C.limit2, d2, bad);
+    direct_report(st, C.limit, disp, bad);
 }
 
 // Back to the contact list, first: the plane contacts of the last step per sphere (count and bits within the scene's
@@ -235,10 +308,26 @@ hipError_t launch_direct_join(uint32_t nS, const uint32_t* oldStart, const uint3
     return hipGetLastError();
 }
 
-hipError_t launch_direct_check(const KParams& P, const DirectCheck& C, const OwnerRec* own, uint32_t nS,
+hipError_t launch_owner_build(const KParams& P, const SphereRec* sph, const OwnerRec* own,
+                              const uint32_t* ownerSphStart, uint32_t nClumps, double scale, OwnerBuild* own0,
+                              SkinStats* stats, hipStream_t st) {
+    if (nClumps == 0) return hipSuccess;
+    k_owner_build<<<blocks(nClumps), 256, 0, st>>>(P, sph, own, ownerSphStart, nClumps, scale, own0, stats);
+    return hipGetLastError();
+}
+
+hipError_t launch_gap_hist(const KParams& P, const SphereRec* sph, const OwnerRec* own, const uint32_t* candA,
+                           const uint32_t* candB, uint32_t nK, double skin, SkinStats* stats, hipStream_t st) {
+    if (nK == 0) return hipSuccess;
+    const uint32_t stride = (nK + SKIN_SAMPLES - 1) / SKIN_SAMPLES;
+    k_gap_hist<<<blocks((nK + stride - 1) / stride), 256, 0, st>>>(P, sph, own, candA, candB, nK, stride, skin, stats);
+    return hipGetLastError();
+}
+
+hipError_t launch_direct_check(const KParams& P, const DirectCheck& C, const OwnerRec* own, uint32_t nClumps,
                                const PlanePose* pose, uint32_t nA, DirectState* state, hipStream_t st) {
-    if (nS == 0) return hipSuccess;
-    k_direct_check<<<blocks(nS), 256, 0, st>>>(P, C, own, nS, pose, nA, state);
+    if (nClumps == 0) return hipSuccess;
+    k_direct_check<<<blocks(nClumps), 256, 0, st>>>(P, C, own, nClumps, pose, nA, state);
     return hipGetLastError();
 }
 
