@@ -9,6 +9,7 @@
 #include <map>
 #include <new>
 #include <string>
+#include <thread>
 #include <unordered_map>
 #include <vector>
 
@@ -215,6 +216,11 @@ struct deme_ctx {
     uint32_t nS = 0, nO = 0, nClumps = 0, nA = 0, nM = 0, nAnalOwners = 0;
     uint32_t maxMatSph = 0, maxMatAnal = 0, maxMat = 0;
     uint64_t nBins = 0;
+    // caller arrays on their way to or from the device: packed there, through pinned slots here (move_packed)
+    DBuf<uint8_t> pack;
+    uint8_t* stage = nullptr;
+    size_t stageBytes = 0;
+    hipEvent_t stageEv[8] = {};
     std::vector<float> hostMass;
     std::vector<float> hostRadius;  // sphere radii (the host's copy, for the cell grid after size changes)
     bool needDetect = false;        // clumps were appended: the next step starts with a detection pass
@@ -448,6 +454,86 @@ int ensure_poses(deme_ctx* c) {
     return DEME_OK;
 }
 
+// ---- caller arrays: packed on the device, moved through pinned slots ----
+// One array of the caller at byte `off` of the packed buffer.
+struct PackedArray {
+    size_t off, bytes;
+    char* host;
+};
+
+// A packed device buffer's layout while it is filled: arrays one after another, 16-byte aligned; null arrays take no
+// room.
+struct Packing {
+    std::vector<PackedArray> arrays;
+    size_t total = 0;
+    static constexpr size_t NONE = ~(size_t)0;
+    size_t add(const void* host, size_t bytes) {
+        if (!host || !bytes) return NONE;
+        const size_t off = total;
+        arrays.push_back({off, bytes, static_cast<char*>(const_cast<void*>(host))});
+        total = (total + bytes + 15) & ~(size_t)15;
+        return off;
+    }
+};
+
+// The packed buffer c->pack to the caller's arrays (down) or the other way, in chunks of one pinned slot per worker:
+// while one chunk is on the link, the workers copy others to or from the caller's pageable memory, whose first touch
+// (page by page) costs more than the transfer itself and spreads over the workers. Measured for 1M owners (85 MB, fresh
+// arrays): 23 ms by the runtime's own pageable copies and one host loop over the records.
+constexpr size_t STAGE_SLOT = 2u << 20;
+constexpr int STAGE_WORKERS = 8;
+int move_packed(deme_ctx* c, const Packing& k, bool down) {
+    if (!k.total) return DEME_OK;
+    const size_t slot = std::min(STAGE_SLOT, (k.total + 65535) & ~(size_t)65535);
+    const size_t chunks = (k.total + slot - 1) / slot;
+    const int workers = (int)std::min<size_t>(chunks, STAGE_WORKERS);
+    if (c->stageBytes < slot * workers) {
+        if (c->stage) DEME_HIP(c, hipHostFree(c->stage));
+        c->stage = nullptr;
+        c->stageBytes = 0;
+        DEME_HIP(c, hipHostMalloc((void**)&c->stage, slot * workers, hipHostMallocDefault));
+        c->stageBytes = slot * workers;
+    }
+    for (int w = 0; w < workers; w++)
+        if (!c->stageEv[w]) DEME_HIP(c, hipEventCreateWithFlags(&c->stageEv[w], hipEventDisableTiming));
+    hipError_t err[STAGE_WORKERS] = {};
+    auto work = [&](int w) {
+        uint8_t* s = c->stage + slot * w;
+        hipError_t e = hipSetDevice(c->device);
+        for (size_t j = w; j < chunks && e == hipSuccess; j += workers) {
+            const size_t lo = j * slot, hi = std::min(lo + slot, k.total);
+            auto touch = [&] {  // the chunk's part of every array that overlaps it
+                for (const PackedArray& a : k.arrays) {
+                    const size_t b = std::max(lo, a.off), f = std::min(hi, a.off + a.bytes);
+                    if (b >= f) continue;
+                    if (down) std::memcpy(a.host + (b - a.off), s + (b - lo), f - b);
+                    else std::memcpy(s + (b - lo), a.host + (b - a.off), f - b);
+                }
+            };
+            if (!down) touch();
+            e = down ? hipMemcpyAsync(s, c->pack.p + lo, hi - lo, hipMemcpyDeviceToHost, c->stream)
+                     : hipMemcpyAsync(c->pack.p + lo, s, hi - lo, hipMemcpyHostToDevice, c->stream);
+            if (e == hipSuccess) e = hipEventRecord(c->stageEv[w], c->stream);
+            if (e == hipSuccess) e = hipEventSynchronize(c->stageEv[w]);
+            if (e == hipSuccess && down) touch();
+        }
+        err[w] = e;
+    };
+    std::thread th[STAGE_WORKERS];
+    int started = 1;
+    try {
+        for (; started < workers; started++) th[started] = std::thread(work, started);
+    } catch (...) {
+        // no thread to be had: this one takes the shares that have none
+    }
+    work(0);
+    for (int w = started; w < workers; w++) work(w);
+    for (int w = 1; w < started; w++) th[w].join();
+    for (int w = 0; w < workers; w++)
+        if (err[w] != hipSuccess) return c->fail_hip(err[w], "copy of caller arrays");
+    return DEME_OK;
+}
+
 int readback_counters(deme_ctx* c) {
     DEME_HIP(c, hipMemcpyAsync(c->hctr, c->ctr.p, DEV_COUNTERS_HOST_BYTES, hipMemcpyDeviceToHost, c->stream));
     DEME_HIP(c, hipStreamSynchronize(c->stream));
@@ -556,6 +642,10 @@ int deme_ctx_destroy(deme_ctx* c) {
     c->pSph.release(); c->pPlane.release(); c->pPlaneOld.release(); c->candStartOld.release(); c->candBOld.release();
     c->pTerm.release(); c->nearBits.release(); c->pose0.release(); c->own0.release();
     c->skinStats.release();
+    c->pack.release();
+    if (c->stage) (void)hipHostFree(c->stage);
+    for (hipEvent_t e : c->stageEv)
+        if (e) (void)hipEventDestroy(e);
     if (c->hdstate) (void)hipHostFree(c->hdstate);
     if (c->hctr) (void)hipHostFree(c->hctr);
     if (c->evCounts) (void)hipEventDestroy(c->evCounts);
@@ -790,48 +880,63 @@ int deme_upload_families(deme_ctx* c, const uint8_t* mask, const deme_family_rul
     return DEME_OK;
 }
 
+}  // extern "C"
+
+namespace {
+
+// Byte offsets of a state's arrays in the packed buffer (Packing::NONE: array not given).
+struct StateOffsets {
+    size_t voxel, loc[3], f[10], acc[6], fam;
+};
+
+StateOffsets pack_state(Packing& k, const deme_owner_state* s, uint32_t n) {
+    StateOffsets o;
+    const uint16_t* loc[3] = {s->locX, s->locY, s->locZ};
+    const float* f[10] = {s->oriQw, s->oriQx, s->oriQy, s->oriQz, s->vX, s->vY, s->vZ, s->omgX, s->omgY, s->omgZ};
+    const float* acc[6] = {s->aX, s->aY, s->aZ, s->alphaX, s->alphaY, s->alphaZ};
+    o.voxel = k.add(s->voxelID, n * sizeof(uint64_t));
+    for (int q = 0; q < 3; q++) o.loc[q] = k.add(loc[q], n * sizeof(uint16_t));
+    for (int q = 0; q < 10; q++) o.f[q] = k.add(f[q], n * sizeof(float));
+    for (int q = 0; q < 6; q++) o.acc[q] = k.add(acc[q], n * sizeof(float));
+    o.fam = k.add(s->family, n);
+    return o;
+}
+
+StateArrays state_arrays(const deme_ctx* c, const StateOffsets& o) {
+    StateArrays a{};
+    auto at = [&](size_t off) { return off == Packing::NONE ? nullptr : c->pack.p + off; };
+    a.voxel = reinterpret_cast<uint64_t*>(at(o.voxel));
+    for (int q = 0; q < 3; q++) a.loc[q] = reinterpret_cast<uint16_t*>(at(o.loc[q]));
+    for (int q = 0; q < 10; q++) a.f[q] = reinterpret_cast<float*>(at(o.f[q]));
+    for (int q = 0; q < 6; q++) a.acc[q] = reinterpret_cast<float*>(at(o.acc[q]));
+    a.fam = at(o.fam);
+    return a;
+}
+
+}  // namespace
+
+extern "C" {
+
 int deme_upload_state(deme_ctx* c, const deme_owner_state* s) {
     c->posesValid = false;
     c->candValid = false;  // positions, radii or the margin changed: candidate lists are rebuilt
     c->adjReady = false;  // recorded adjoint checkpoints no longer describe the system
     if (!c->haveTemplates) return c->fail(DEME_ERR_NOT_READY, "upload templates before the owner state");
     const uint32_t n = c->nO;
-    std::vector<OwnerRec> h(n);
-    if (c->haveState && n) {
-        DEME_HIP(c, hipMemcpyAsync(h.data(), c->own.p, n * sizeof(OwnerRec), hipMemcpyDeviceToHost, c->stream));
-        DEME_HIP(c, hipStreamSynchronize(c->stream));
-    } else {
-        std::memset(h.data(), 0, n * sizeof(OwnerRec));
-        for (uint32_t o = 0; o < n; o++) h[o].qw = 1.f;
-    }
-    for (uint32_t o = 0; o < n; o++) {
-        OwnerRec& r = h[o];
-        if (s->voxelID) r.voxel = s->voxelID[o];
-        if (s->locX) r.lx = s->locX[o];
-        if (s->locY) r.ly = s->locY[o];
-        if (s->locZ) r.lz = s->locZ[o];
-        if (s->family) r.fam = s->family[o];
-        if (s->oriQw) r.qw = s->oriQw[o];
-        if (s->oriQx) r.qx = s->oriQx[o];
-        if (s->oriQy) r.qy = s->oriQy[o];
-        if (s->oriQz) r.qz = s->oriQz[o];
-        if (s->vX) r.vx = s->vX[o];
-        if (s->vY) r.vy = s->vY[o];
-        if (s->vZ) r.vz = s->vZ[o];
-        if (s->omgX) r.wx = s->omgX[o];
-        if (s->omgY) r.wy = s->omgY[o];
-        if (s->omgZ) r.wz = s->omgZ[o];
-        r.mass = c->hostMass[o];
-        r.pad0 = 0;
-        r.scene = c->hostScene[o];
-    }
-    if (n) DEME_HIP(c, hipMemcpyAsync(c->own.p, h.data(), n * sizeof(OwnerRec), hipMemcpyHostToDevice, c->stream));
-    // accelerations, when given
-    float* accs[6] = {s->aX, s->aY, s->aZ, s->alphaX, s->alphaY, s->alphaZ};
-    for (int k = 0; k < 6; k++)
-        if (accs[k] && n)
-            DEME_HIP(c, hipMemcpyAsync(c->acc.p + (size_t)k * n, accs[k], n * sizeof(float), hipMemcpyHostToDevice,
-                                       c->stream));
+    const bool fresh = !c->haveState;
+    Packing k;
+    const StateOffsets at = pack_state(k, s, n);
+    // (the first state of these templates brings the owners' masses and scenes along)
+    const size_t mass = fresh ? k.add(c->hostMass.data(), n * sizeof(float)) : Packing::NONE;
+    const size_t scene = fresh ? k.add(c->hostScene.data(), n * sizeof(uint32_t)) : Packing::NONE;
+    DEME_HIP(c, c->pack.ensure(k.total));
+    int r = move_packed(c, k, false);
+    if (r) return r;
+    DEME_LAUNCH(c, "state_put",
+                launch_state_put(c->own.p, c->acc.p, n, state_arrays(c, at),
+                                 fresh ? reinterpret_cast<const float*>(c->pack.p + mass) : nullptr,
+                                 fresh ? reinterpret_cast<const uint32_t*>(c->pack.p + scene) : nullptr, fresh,
+                                 c->stream));
     DEME_HIP(c, hipStreamSynchronize(c->stream));
     c->haveState = true;
     return DEME_OK;
@@ -851,36 +956,11 @@ int deme_clear_contacts(deme_ctx* c) {
 
 int deme_download_state(deme_ctx* c, deme_owner_state* s) {
     if (!c->haveState) return c->fail(DEME_ERR_NOT_READY, "no owner state");
-    const uint32_t n = c->nO;
-    std::vector<OwnerRec> h(n);
-    std::vector<float> a((size_t)6 * n);
-    if (n) {
-        DEME_HIP(c, hipMemcpyAsync(h.data(), c->own.p, n * sizeof(OwnerRec), hipMemcpyDeviceToHost, c->stream));
-        DEME_HIP(c, hipMemcpyAsync(a.data(), c->acc.p, (size_t)6 * n * sizeof(float), hipMemcpyDeviceToHost, c->stream));
-    }
-    DEME_HIP(c, hipStreamSynchronize(c->stream));
-    for (uint32_t o = 0; o < n; o++) {
-        const OwnerRec& r = h[o];
-        if (s->voxelID) s->voxelID[o] = r.voxel;
-        if (s->locX) s->locX[o] = r.lx;
-        if (s->locY) s->locY[o] = r.ly;
-        if (s->locZ) s->locZ[o] = r.lz;
-        if (s->family) s->family[o] = r.fam;
-        if (s->oriQw) s->oriQw[o] = r.qw;
-        if (s->oriQx) s->oriQx[o] = r.qx;
-        if (s->oriQy) s->oriQy[o] = r.qy;
-        if (s->oriQz) s->oriQz[o] = r.qz;
-        if (s->vX) s->vX[o] = r.vx;
-        if (s->vY) s->vY[o] = r.vy;
-        if (s->vZ) s->vZ[o] = r.vz;
-        if (s->omgX) s->omgX[o] = r.wx;
-        if (s->omgY) s->omgY[o] = r.wy;
-        if (s->omgZ) s->omgZ[o] = r.wz;
-    }
-    float* accs[6] = {s->aX, s->aY, s->aZ, s->alphaX, s->alphaY, s->alphaZ};
-    for (int k = 0; k < 6; k++)
-        if (accs[k]) std::memcpy(accs[k], a.data() + (size_t)k * n, n * sizeof(float));
-    return DEME_OK;
+    Packing k;
+    const StateOffsets at = pack_state(k, s, c->nO);
+    DEME_HIP(c, c->pack.ensure(k.total));
+    DEME_LAUNCH(c, "state_get", launch_state_get(c->own.p, c->acc.p, c->nO, state_arrays(c, at), c->stream));
+    return move_packed(c, k, true);
 }
 
 // ---------------------------------------------------------------------------------------------------------------
@@ -1573,12 +1653,18 @@ int deme_download_contacts(deme_ctx* c, uint32_t* idA, uint32_t* idB, uint8_t* t
     if (!c->contactsReady) return c->fail(DEME_ERR_NOT_READY, "no contact list");
     const size_t C = c->C;
     const int cu = c->cur;
-    if (C) {
-        if (idA) DEME_HIP(c, hipMemcpyAsync(idA, c->idA.p, C * 4, hipMemcpyDeviceToHost, c->stream));
-        if (idB) DEME_HIP(c, hipMemcpyAsync(idB, c->idB[cu].p, C * 4, hipMemcpyDeviceToHost, c->stream));
-        if (type) DEME_HIP(c, hipMemcpyAsync(type, c->ctype[cu].p, C, hipMemcpyDeviceToHost, c->stream));
-        if (map) DEME_HIP(c, hipMemcpyAsync(map, c->map.p, C * 4, hipMemcpyDeviceToHost, c->stream));
-    }
+    Packing k;
+    const void* dev[4] = {c->idA.p, c->idB[cu].p, c->ctype[cu].p, c->map.p};
+    void* host[4] = {idA, idB, type, map};
+    const size_t bytes[4] = {C * 4, C * 4, C, C * 4};
+    size_t off[4];
+    for (int q = 0; q < 4; q++) off[q] = k.add(host[q], bytes[q]);
+    DEME_HIP(c, c->pack.ensure(k.total));
+    for (int q = 0; q < 4; q++)
+        if (off[q] != Packing::NONE)
+            DEME_HIP(c, hipMemcpyAsync(c->pack.p + off[q], dev[q], bytes[q], hipMemcpyDeviceToDevice, c->stream));
+    int r = move_packed(c, k, true);
+    if (r) return r;
     DEME_HIP(c, hipStreamSynchronize(c->stream));
     return DEME_OK;
 }
@@ -2935,49 +3021,38 @@ int deme_download_forces(deme_ctx* c, float* F, float* T, float* cA, float* cB) 
     if (!c->contactsReady) return c->fail(DEME_ERR_NOT_READY, "no contact list");
     if (!c->forcesFull)
         return c->fail(DEME_ERR_NOT_READY, "contact records are kept by deme_force only (deme_step stores owner terms)");
-    std::vector<ForceRec> h(c->C);
-    if (c->C) DEME_HIP(c, hipMemcpyAsync(h.data(), c->frc.p, c->C * sizeof(ForceRec), hipMemcpyDeviceToHost, c->stream));
-    DEME_HIP(c, hipStreamSynchronize(c->stream));
-    for (size_t i = 0; i < c->C; i++) {
-        const ForceRec& f = h[i];
-        if (F) { F[3 * i] = f.fx; F[3 * i + 1] = f.fy; F[3 * i + 2] = f.fz; }
-        if (T) { T[3 * i] = f.tx; T[3 * i + 1] = f.ty; T[3 * i + 2] = f.tz; }
-        if (cA) { cA[3 * i] = f.ax; cA[3 * i + 1] = f.ay; cA[3 * i + 2] = f.az; }
-        if (cB) { cB[3 * i] = f.bx; cB[3 * i + 1] = f.by; cB[3 * i + 2] = f.bz; }
-    }
-    return DEME_OK;
+    Packing k;
+    float* host[4] = {F, T, cA, cB};
+    size_t off[4];
+    for (int q = 0; q < 4; q++) off[q] = k.add(host[q], c->C * 3 * sizeof(float));
+    DEME_HIP(c, c->pack.ensure(k.total));
+    for (int q = 0; q < 4; q++)
+        if (off[q] != Packing::NONE)
+            DEME_LAUNCH(c, "record_columns",
+                        launch_record_columns(c->frc.p, c->C, 3 * q, reinterpret_cast<float*>(c->pack.p + off[q]),
+                                              c->stream));
+    return move_packed(c, k, true);
 }
 
 int deme_download_wildcards(deme_ctx* c, float* w) {
     if (!c->contactsReady) return c->fail(DEME_ERR_NOT_READY, "no contact list");
     const size_t C = c->C;
-    std::vector<float4> h(C);
+    Packing k;
+    const size_t off = k.add(w, 4 * C * sizeof(float));
+    if (off == Packing::NONE) return DEME_OK;
+    DEME_HIP(c, c->pack.ensure(k.total));
+    float* out = reinterpret_cast<float*>(c->pack.p + off);
     if (c->fresh) {
         // Between a detection pass and the next force pass the history still lives in the previous order; the force
-        // kernel gathers it through the persistent-contact map. Apply the same gather here.
-        std::vector<uint32_t> m(C);
-        std::vector<float4> prev(c->havePrev ? c->Cprev : 0);
-        if (C) DEME_HIP(c, hipMemcpyAsync(m.data(), c->map.p, C * 4, hipMemcpyDeviceToHost, c->stream));
-        if (!prev.empty())
-            DEME_HIP(c, hipMemcpyAsync(prev.data(), c->hist[c->cur ^ 1].p, prev.size() * sizeof(float4),
-                                       hipMemcpyDeviceToHost, c->stream));
-        DEME_HIP(c, hipStreamSynchronize(c->stream));
-        for (size_t i = 0; i < C; i++)
-            h[i] = (m[i] == DEME_NULL_MAPPING_PARTNER || m[i] >= prev.size()) ? make_float4(0.f, 0.f, 0.f, 0.f)
-                                                                             : prev[m[i]];
+        // kernel gathers it through the persistent-contact map, and so does this.
+        const bool prev = c->havePrev;
+        DEME_LAUNCH(c, "history_columns",
+                    launch_history_columns(c->hist[c->cur ^ 1].p, c->map.p, prev ? c->Cprev : 0, C, out, c->stream));
     } else {
-        if (C)
-            DEME_HIP(c, hipMemcpyAsync(h.data(), c->hist[c->cur].p, C * sizeof(float4), hipMemcpyDeviceToHost,
-                                       c->stream));
-        DEME_HIP(c, hipStreamSynchronize(c->stream));
+        DEME_LAUNCH(c, "history_columns",
+                    launch_history_columns(c->hist[c->cur].p, nullptr, 0, C, out, c->stream));
     }
-    for (size_t i = 0; i < C; i++) {
-        w[i] = h[i].x;
-        w[C + i] = h[i].y;
-        w[2 * C + i] = h[i].z;
-        w[3 * C + i] = h[i].w;
-    }
-    return DEME_OK;
+    return move_packed(c, k, true);
 }
 
 int deme_upload_wildcards(deme_ctx* c, const float* w) {

@@ -292,6 +292,20 @@ hipError_t launch_direct_plane_bits(const KParams& P, const SphereRec* sph, cons
                                     uint32_t* clear, uint32_t nClear, hipStream_t st);
 hipError_t launch_direct_leave(const DirectList& D, const uint32_t* cidx, const uint32_t* rowStart, float4* listHist,
                                hipStream_t st, SpecGuard guard);
+// state.hip: device arrays of one value per owner (null: not asked for / not given)
+struct StateArrays {
+    uint64_t* voxel;
+    uint16_t* loc[3];
+    float* f[10];   // orientation w x y z, velocity x y z, angular velocity x y z
+    float* acc[6];  // linear x y z, angular x y z
+    uint8_t* fam;
+};
+hipError_t launch_state_get(const OwnerRec* own, const float* acc, uint32_t nO, const StateArrays& a, hipStream_t st);
+hipError_t launch_state_put(OwnerRec* own, float* acc, uint32_t nO, const StateArrays& a, const float* mass,
+                            const uint32_t* scene, bool fresh, hipStream_t st);
+hipError_t launch_record_columns(const ForceRec* rec, uint64_t n, int col, float* out, hipStream_t st);
+hipError_t launch_history_columns(const float4* hist, const uint32_t* map, uint64_t nPrev, uint64_t n, float* out,
+                                  hipStream_t st);
 // clock[0] = t (one lane; the time the owner update's motion rules read, written on the stream before the update)
 hipError_t launch_set_clock(double* clock, double t, hipStream_t st);
 // clock[0] += (double)h: the time step the host adds after each step, done on the device inside a captured step
