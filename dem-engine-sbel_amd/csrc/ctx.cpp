@@ -2075,10 +2075,11 @@ static DirectCheck direct_check(const deme_ctx* c) {
     k.unit = c->posUnit;
     k.limit = std::sqrt(stale_limit2(c));
     const double rmax = (double)c->maxRadius, bs = c->sp.binSize;
-    // an owner's spheres reach maxRel + r past it; a contact point strays from its spheres by under 1e-6 of the radii
-    // (the limits leave a hundred times that)
-    const double past = (double)c->maxRel * 1.00001 + rmax * 1.0001 + (double)c->sp.beta;
-    auto hi = [&](uint32_t nb) { return (double)nb * bs * (1.0 - 1e-12) - past; };
+    k.sph = c->sph.p;
+    k.ownerSphStart = c->ownerSphStart.p;
+    k.past = (double)c->maxRel * 1.00001 + rmax * 1.00001 + (double)c->sp.beta;
+    // a contact point strays from its spheres by under 1e-6 of the radii (the limits leave a hundred times that)
+    auto hi = [&](uint32_t nb) { return (double)nb * bs * (1.0 - 1e-12) - 1e-4 * rmax; };
     const double span = 2.0 * (rmax + (double)c->sp.beta) / bs + 2.0;
     const bool fits = span * span * span <= 65535.0;
     k.hiX = fits ? hi(c->sp.nbX) : -INFINITY;

@@ -566,18 +566,34 @@ struct __attribute__((aligned(16))) OwnerBuild {
 };
 static_assert(sizeof(OwnerBuild) == 32, "OwnerBuild must be 32 bytes");
 // What the owner update checks of the state it leaves: no sphere farther than limit from its position at the build
-// (bounded by its owner's motion since, own0, positions in units of unit), every owner clear of the bin grid's upper ends
-// (below hiX, hiY, hiZ: the bin ranges of its spheres, and the contact point of any pair, then lie inside the grid; the
-// host's limits are minus infinity where a sphere could touch too many bins), and no component moved by more than
-// planeLimit since the plane candidates were made (pose0; reach bounds a sphere's distance from the origin). A state
-// that fails is left to the contact-list path: its pass reports an error, or goes on.
+// (bounded by its owner's motion since, own0, positions in units of unit), every sphere clear of the bin grid's upper ends
+// (its upper corner below hiX, hiY, hiZ: its bin range, and the contact point of any pair, then lie inside the grid; the
+// host's limits are minus infinity where a sphere could touch too many bins; an owner more than past below them needs no
+// look at its spheres), and no component moved by more than planeLimit since the plane candidates were made (pose0; reach
+// bounds a sphere's distance from the origin). A state that fails is left to the contact-list path: its pass reports an
+// error, or goes on.
 struct DirectCheck {
     const OwnerBuild* own0;
+    const SphereRec* sph;
+    const uint32_t* ownerSphStart;
     double unit, limit;
-    double hiX, hiY, hiZ;
+    double hiX, hiY, hiZ, past;
     const PlanePose* pose0;
     double planeLimit, reach;
 };
+
+// The spheres of an owner near the grid's upper ends, one by one (in the general case an upper wall's layer: a clump's
+// bound past it would send a third of all worlds to the contact-list path).
+__device__ __forceinline__ uint32_t direct_edge(const KParams& P, const DirectCheck& C, const OwnerRec& r, uint32_t o) {
+    for (uint32_t s = C.ownerSphStart[o]; s < C.ownerSphStart[o + 1]; s++) {
+        const SphereRec sr = load_sphere(C.sph, s);
+        double X, Y, Z;
+        sphere_position(P, r, sr, X, Y, Z);
+        const double rCD = cd_radius(P, sr.r);
+        if (!(X + rCD < C.hiX && Y + rCD < C.hiY && Z + rCD < C.hiZ)) return ERRBIT_EDGE;
+    }
+    return 0;
+}
 
 // One owner's part of the check: ERRBIT_* bits, disp raised to the bound of its spheres' displacement. A sphere moves by
 // at most |dX| + |R(q) - R(q0)| relMax, and R is quadratic: R(q) - R(q0) = 2 M(q - q0, q + q0) with M symmetric and
@@ -595,7 +611,7 @@ __device__ __forceinline__ uint32_t direct_check_owner(const KParams& P, const D
     double X, Y, Z;
     owner_position(P, r.voxel, r.lx, r.ly, r.lz, X, Y, Z);
     uint32_t bad = 0;
-    if (!(X < C.hiX && Y < C.hiY && Z < C.hiZ)) bad = ERRBIT_EDGE;
+    if (!(X + C.past < C.hiX && Y + C.past < C.hiY && Z + C.past < C.hiZ)) bad = direct_edge(P, C, r, o);
     constexpr int32_t unfit = -2147483647 - 1;  // INT32_MIN (hipRTC has no limits)
     const double dx = X - (double)b.x * C.unit, dy = Y - (double)b.y * C.unit, dz = Z - (double)b.z * C.unit;
     double m = sqrt(dx * dx + dy * dy + dz * dz);
