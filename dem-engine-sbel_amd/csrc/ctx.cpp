@@ -139,6 +139,11 @@ struct deme_ctx {
     int skinDir = 0;
     uint32_t cellPassesLeft = 0, cellBackoff = 0;
     bool candValid = false, rebuildNext = true;
+    // The state was replaced since the last pass (uploaded, restored): if the lists are then found stale, that says
+    // nothing about their skin. An upload that made them stale has the next jumpSkip uploads drop the lists at once
+    // (one wasted pass less; doubling up to 15 while that repeats).
+    bool jumped = false;
+    uint32_t jumpSkip = 0, jumpBackoff = 0;
     uint64_t nCand = 0, candBuilds = 0, passesSinceBuild = 0;
     // passes the lists before the latest build lasted (~0 before the second build) and whether the pass in hand built
     uint64_t lastLifetime = ~0ull;
@@ -919,7 +924,12 @@ extern "C" {
 
 int deme_upload_state(deme_ctx* c, const deme_owner_state* s) {
     c->posesValid = false;
-    c->candValid = false;  // positions, radii or the margin changed: candidate lists are rebuilt
+    // candidate lists stay: the next pass measures every sphere against its position at the build, whatever moved it
+    if (c->jumpSkip > 0) {
+        c->jumpSkip--;
+        c->candValid = false;
+    }
+    c->jumped = true;
     c->adjReady = false;  // recorded adjoint checkpoints no longer describe the system
     if (!c->haveTemplates) return c->fail(DEME_ERR_NOT_READY, "upload templates before the owner state");
     const uint32_t n = c->nO;
@@ -936,7 +946,7 @@ int deme_upload_state(deme_ctx* c, const deme_owner_state* s) {
                 launch_state_put(c->own.p, c->acc.p, n, state_arrays(c, at),
                                  fresh ? reinterpret_cast<const float*>(c->pack.p + mass) : nullptr,
                                  fresh ? reinterpret_cast<const uint32_t*>(c->pack.p + scene) : nullptr, fresh,
-                                 c->stream));
+                                 c->candValid && c->nS > 0 ? c->pos0.p : nullptr, c->stream));
     DEME_HIP(c, hipStreamSynchronize(c->stream));
     c->haveState = true;
     return DEME_OK;
@@ -944,7 +954,7 @@ int deme_upload_state(deme_ctx* c, const deme_owner_state* s) {
 
 int deme_clear_contacts(deme_ctx* c) {
     c->graphGen++;
-    c->candValid = false;  // positions, radii or the margin changed: candidate lists are rebuilt
+    c->cidxGen[0] = c->cidxGen[1] = 0;
     c->adjReady = false;
     c->havePrev = c->contactsReady = c->fresh = false;
     c->termsReady = c->forcesFull = false;
@@ -1285,7 +1295,7 @@ static int build_candidates(deme_ctx* c) {
         c->skinAuto = c->skinNext;  // (chosen from the statistics of the lists being retired)
         c->skinCostPrev = -1.0;
         c->skinDir = 0;
-    } else if (c->skinSet < 0.0 && c->candBuilds > 0 && c->candValid) {
+    } else if (c->skinSet < 0.0 && c->candBuilds > 0 && c->candValid && !c->jumped) {
         // the retiring lists' lifetime and size judge their skin (lists dropped for other reasons -- a host change,
         // a return from the cell sweep -- do not)
         constexpr double BUILD_PASSES = 2.7;
@@ -1314,7 +1324,12 @@ static int build_candidates(deme_ctx* c) {
         c->skinAuto = std::min(std::max(next, 0.05 * m), 0.8 * m);
     }
     c->skinNext = 0.0;
-    c->lastLifetime = c->candBuilds > 0 ? c->passesSinceBuild : ~0ull;
+    c->lastLifetime = c->candBuilds > 0 && !c->jumped ? c->passesSinceBuild : ~0ull;
+    if (c->jumped && c->candValid) {
+        c->jumpBackoff = std::min<uint32_t>(2 * c->jumpBackoff + 1, 15);
+        c->jumpSkip = c->jumpBackoff;
+    }
+    c->jumped = false;
     c->builtThisPass = true;
     c->passesSinceBuild = 0;
     int mode = 0;
@@ -1455,6 +1470,8 @@ static void end_pass(deme_ctx* c, bool skinPass, double disp2) {
     const bool built = c->builtThisPass;
     c->builtThisPass = false;
     if (skinPass) {
+        if (c->jumped) c->jumpBackoff = 0;  // the lists outlived the new state
+        c->jumped = false;
         c->passesSinceBuild++;
         const double lim = 0.35 * c->skin();
         c->rebuildNext = disp2 > lim * lim;
@@ -1934,7 +1951,9 @@ static int enqueue_cycle(deme_ctx* c, int f, const SpecGuard& g, int mode) {
                                      s == 0 ? c->hist[q].p : c->hist[p].p, s == 0 ? c->map.p : nullptr, c->hist[p].p,
                                      nullptr, g));
         DEME_LAUNCH(c, "owner_update", launch_owner_ctx(c, 1, p, g));
-        DEME_LAUNCH(c, "advance_clock", launch_advance_clock(c->clock.p, c->sp.h, c->stream));
+        // (only motion rules read the clock; the launch costs 4 us a step)
+        if (c->ownerJitActive)
+            DEME_LAUNCH(c, "advance_clock", launch_advance_clock(c->clock.p, c->sp.h, c->stream));
     }
     return DEME_OK;
 }
@@ -2003,7 +2022,7 @@ static int run_cycle(deme_ctx* c, int f, bool* done) {
         int r = capture_cycle(c, p, f);
         if (r) return r;
     }
-    DEME_LAUNCH(c, "set_clock", launch_set_clock(c->clock.p, c->time, c->stream));
+    if (c->ownerJitActive) DEME_LAUNCH(c, "set_clock", launch_set_clock(c->clock.p, c->time, c->stream));
     DEME_HIP(c, hipGraphLaunch(cy.exec, c->stream));
     DEME_HIP(c, hipMemcpyAsync(c->hctr, c->ctr.p, DEV_COUNTERS_HOST_BYTES, hipMemcpyDeviceToHost, c->stream));
     DEME_HIP(c, hipStreamSynchronize(c->stream));
@@ -2368,7 +2387,7 @@ static int run_direct(deme_ctx* c, int n, int* done, bool* again) {
             std::memcpy(&v, &b, sizeof(v));
             dispMax = std::max(dispMax, v);
         }
-        if (c->passesSinceBuild >= 4)
+        if (c->passesSinceBuild >= 4 && !c->jumped)
             c->stepMove = std::max(dispMax, 0.125 * check.limit) / (double)c->passesSinceBuild;
         if (err & ERRBIT_STALE) c->rebuildNext = true;
         if (err & ~(uint32_t)ERRBIT_STALE) {
@@ -2378,6 +2397,8 @@ static int run_direct(deme_ctx* c, int n, int* done, bool* again) {
             break;
         }
         if (!err) {
+            if (c->jumped) c->jumpBackoff = 0;
+            c->jumped = false;
             c->directBackoff = 0;
             rebuilt = false;
             continue;
@@ -2723,7 +2744,9 @@ static int adj_save(deme_ctx* c, deme_ctx::AdjCk& k, bool full) {
 static int adj_restore(deme_ctx* c, const deme_ctx::AdjCk& k) {
     c->posesValid = false;
     c->graphGen++;
-    c->candValid = false;  // positions, radii or the margin changed: candidate lists are rebuilt
+    // (candidate lists stay, as when a state is uploaded; the restored list does not index them)
+    c->jumped = true;
+    c->cidxGen[0] = c->cidxGen[1] = 0;
     DEME_HIP(c, hipMemcpyAsync(c->own.p, k.own.p, c->nO * sizeof(OwnerRec), hipMemcpyDeviceToDevice, c->stream));
     const int cu = c->cur;
     if (k.haveList) {

@@ -302,7 +302,7 @@ struct StateArrays {
 };
 hipError_t launch_state_get(const OwnerRec* own, const float* acc, uint32_t nO, const StateArrays& a, hipStream_t st);
 hipError_t launch_state_put(OwnerRec* own, float* acc, uint32_t nO, const StateArrays& a, const float* mass,
-                            const uint32_t* scene, bool fresh, hipStream_t st);
+                            const uint32_t* scene, bool fresh, BuildPos* pos0, hipStream_t st);
 hipError_t launch_record_columns(const ForceRec* rec, uint64_t n, int col, float* out, hipStream_t st);
 hipError_t launch_history_columns(const float4* hist, const uint32_t* map, uint64_t nPrev, uint64_t n, float* out,
                                   hipStream_t st);

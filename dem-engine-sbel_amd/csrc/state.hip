@@ -29,10 +29,13 @@ __global__ __launch_bounds__(256) void k_state_get(const OwnerRec* __restrict__ 
 }
 
 // The given arrays into the owner records (fresh: no records yet, the others take their defaults and mass and scene
-// come along).
+// come along). pos0: the build positions of the candidate lists in force, or null. They tell every finite state whether
+// the lists still hold; an orientation that is not finite would pass unseen (no comparison holds for a NaN displacement),
+// so it marks the lists stale.
 __global__ __launch_bounds__(256) void k_state_put(OwnerRec* __restrict__ own, float* __restrict__ acc, uint32_t nO,
                                                    StateArrays a, const float* __restrict__ mass,
-                                                   const uint32_t* __restrict__ scene, bool fresh) {
+                                                   const uint32_t* __restrict__ scene, bool fresh,
+                                                   BuildPos* __restrict__ pos0) {
     const uint32_t o = blockIdx.x * blockDim.x + threadIdx.x;
     if (o >= nO) return;
     OwnerRec r{};
@@ -57,6 +60,7 @@ __global__ __launch_bounds__(256) void k_state_put(OwnerRec* __restrict__ own, f
     for (int k = 0; k < 6; k++)
         if (a.acc[k]) acc[(uint64_t)k * nO + o] = a.acc[k][o];
     if (a.fam) r.fam = a.fam[o];
+    if (pos0 && !(isfinite(r.qw) && isfinite(r.qx) && isfinite(r.qy) && isfinite(r.qz))) pos0[0].x = INT32_MIN;
     uint4* dst = reinterpret_cast<uint4*>(own + o);
     const uint4* src = reinterpret_cast<const uint4*>(&r);
     dst[0] = src[0];
@@ -104,9 +108,9 @@ hipError_t launch_state_get(const OwnerRec* own, const float* acc, uint32_t nO, 
 }
 
 hipError_t launch_state_put(OwnerRec* own, float* acc, uint32_t nO, const StateArrays& a, const float* mass,
-                            const uint32_t* scene, bool fresh, hipStream_t st) {
+                            const uint32_t* scene, bool fresh, BuildPos* pos0, hipStream_t st) {
     if (nO == 0) return hipSuccess;
-    k_state_put<<<blocks(nO), 256, 0, st>>>(own, acc, nO, a, mass, scene, fresh);
+    k_state_put<<<blocks(nO), 256, 0, st>>>(own, acc, nO, a, mass, scene, fresh, pos0);
     return hipGetLastError();
 }
 

@@ -167,3 +167,34 @@ def test_a_sphere_leaving_the_world_fails_at_the_same_step():
     sa, sb = a.get_state(), b.get_state()
     for k in sa:
         assert np.array_equal(sa[k], sb[k]), k
+
+
+@pytest.mark.parametrize("steps", [1, 9])
+def test_lists_kept_over_replaced_states(steps):
+    """States written between calls: moved a little (the lists hold), shuffled over the whole box (stale, again and again),
+    back to an earlier one; the contact-list path builds anew each pass."""
+    sc = scenes.sphere_settling(n=3001, spacing=1.98, velocity_sigma=0.3, seed=57)
+    a, b = _pair(sc)
+    rng = np.random.default_rng(4)
+    where = ("voxelID", "locX", "locY", "locZ")
+    first = None
+    for k, move in enumerate(["jitter", "jitter", "shuffle", "shuffle", "shuffle", "first", "jitter", "shuffle", "jitter"]):
+        for d in (a, b):
+            d.step(steps)
+        _same(a, b)
+        st = a.get_state()
+        first = first or {f: v.copy() for f, v in st.items()}
+        if move == "jitter":
+            st["locY"] ^= np.uint16(1 + k)
+        elif move == "shuffle":
+            p = np.arange(sc.n_owners)
+            rng.shuffle(p[:sc.n_clumps])
+            for f in where:
+                st[f] = st[f][p]
+        else:
+            st = first
+        for d in (a, b):
+            d.set_state(st)
+    for d in (a, b):
+        d.step(steps)
+    _same(a, b)
