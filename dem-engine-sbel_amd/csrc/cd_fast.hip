@@ -628,6 +628,14 @@ __global__ __launch_bounds__(256) void k_cand_flags(KParams P, uint32_t nK, cons
         (!mask || mask[mask_index(meta[ia].y, meta[ib].y)] == DEME_DONT_PREVENT_CONTACT))
         f = bin_rule_point(P, 1.0 / P.binSize, a, b) ? 1 : 0;  // a has the lower id
     acc[c] = f;
+    if (P.beta > 0.f && blockIdx.x % 64u == 0) {
+        const uint32_t listed = (uint32_t)__popcll(__ballot(f));
+        const uint32_t near = (uint32_t)__popcll(__ballot(f && expanded_overlap((double)a.r, a, (double)b.r, b)));
+        if ((threadIdx.x & 63u) == 0 && listed) {
+            atomicAdd(&ctr->sampled, listed);
+            atomicAdd(&ctr->touching, near);
+        }
+    }
 }
 
 // Per sphere: its row's touching candidates (aCnt) and those with it as partner (bCnt, its mirror row's length), with

@@ -143,6 +143,7 @@ struct deme_ctx {
     // nothing about their skin. An upload that made them stale has the next jumpSkip uploads drop the lists at once
     // (one wasted pass less; doubling up to 15 while that repeats).
     bool jumped = false;
+    bool fewTouch = false;  // few of the contacts listed with a drift margin touch (count_touching)
     uint32_t jumpSkip = 0, jumpBackoff = 0;
     uint64_t nCand = 0, candBuilds = 0, passesSinceBuild = 0;
     // passes the lists before the latest build lasted (~0 before the second build) and whether the pass in hand built
@@ -537,6 +538,11 @@ int move_packed(deme_ctx* c, const Packing& k, bool down) {
     for (int w = 0; w < workers; w++)
         if (err[w] != hipSuccess) return c->fail_hip(err[w], "copy of caller arrays");
     return DEME_OK;
+}
+
+// The sample of a candidate pass with a drift margin (0.4 with some slack: each change costs captured steps a capture).
+static void count_touching(deme_ctx* c, const DevCounters& h) {
+    if (h.sampled > 0) c->fewTouch = h.touching <= (c->fewTouch ? 0.45 : 0.35) * h.sampled;
 }
 
 int readback_counters(deme_ctx* c) {
@@ -1576,6 +1582,7 @@ int deme_cd_run(deme_ctx* c) {
         }
     }
     const double disp2 = max_disp2(*c->hctr);
+    count_touching(c, *c->hctr);
     const uint64_t C = c->hctr->total[1], nPairs = c->hctr->total[2];
     if (C > 0xFFFFFFFFull) return c->fail(DEME_ERR_CAPACITY, "contact count exceeds contactPairs_t (2^32 - 1)");
     if (nPairs > C) return c->fail(DEME_ERR_HIP, "inconsistent contact and mirror-row counts");
@@ -1707,7 +1714,7 @@ static int jit_rebuild(deme_ctx* c) {
 // Touch flags for the owner terms: used when lists are detected with a drift margin (most pairs of such a list may
 // not touch, and their zero terms are then neither written nor read); without a margin every pair touches at
 // detection and every term is written.
-static uint8_t* term_flags(deme_ctx* c, bool bSide) {
+static uint8_t* term_flags(const deme_ctx* c, bool bSide) {
     if (!(c->sp.beta > 0.f)) return nullptr;
     return bSide ? c->bOn.p : c->aOn.p;
 }
@@ -1734,18 +1741,28 @@ static hipError_t ensure_partials(deme_ctx* c, uint64_t nC, double grow = 1.25) 
     return c->analPartials.ensure(std::max<size_t>((size_t)anal_blocks(nC) * MAX_ANAL_OWNERS * 6, 1), grow);
 }
 
+// A list detected with a drift margin is tested first when it is long and few of its contacts touch. Testing costs a wave
+// a second round of gathers before the model (0.64M contacts of which a sixth touch: 29.8 us against 26.3, all through
+// the model); a long list is bound by the model's instructions (1.3M: 35.8 against 44.6 us; 4.9M: 125 against 181), and
+// each quarter of the contacts that touches adds a round of the model (all touching: 243 us, so 0.4 is about even).
+static ForceKind force_kind(const deme_ctx* c, uint64_t nC, bool settled) {
+    if (!term_flags(c, false) || nC < 1000000 || !c->fewTouch) return FORCE_KIND_ALL;
+    return settled ? FORCE_KIND_SETTLED : FORCE_KIND_MARGIN;
+}
+
 // The force kernel of the context: the specialised one when a model or placeholder values were given, else the
 // ahead-of-time kernel of the built-in model.
 static hipError_t launch_force_ctx(deme_ctx* c, bool full, uint32_t nC, const uint32_t* idB, const uint8_t* ctype,
                                    const OwnerRec* own, const float4* histIn, const uint32_t* map, float4* histOut,
-                                   ForceRec* out, SpecGuard guard = SpecGuard()) {
+                                   ForceRec* out, SpecGuard guard = SpecGuard(), bool settled = false) {
+    const ForceKind kind = force_kind(c, nC, settled);
     if (c->jitActive)
         return c->jit.launch(full, c->kp, nC, c->idA.p, idB, ctype, c->sph.p, own, c->moi.p, c->anal.p, c->pose.p,
                              c->mats.p, histIn, map, histOut, c->mirror.p, c->aTerm.p, c->bTerm.p, plane_sums(c),
-                             term_flags(c, false), term_flags(c, true), out, c->stream, guard);
+                             term_flags(c, false), term_flags(c, true), out, c->stream, guard, kind);
     return launch_force(c->kp, nC, c->idA.p, idB, ctype, c->sph.p, own, c->moi.p, c->anal.p, c->pose.p, c->mats.p,
                         histIn, map, histOut, c->mirror.p, c->aTerm.p, c->bTerm.p, plane_sums(c), term_flags(c, false),
-                        term_flags(c, true), out, c->stream, guard);
+                        term_flags(c, true), out, c->stream, guard, kind);
 }
 
 // The owner update of the context (the specialised kernel when motion strategies or rules were given): owner sums of
@@ -1763,7 +1780,8 @@ static hipError_t launch_owner_ctx(deme_ctx* c, int integrate, int cu, SpecGuard
                                c->rules.p, c->own.p, c->acc.p, integrate, c->clock.p, c->stream, nullptr, guard);
 }
 
-static int force_pass(deme_ctx* c, bool full) {
+// settled: the last force pass ran on this list, and nothing but the owner update since.
+static int force_pass(deme_ctx* c, bool full, bool settled = false) {
     int r = check_ready(c);
     if (r) return r;
     if (c->jitActive && c->jitStale && (r = jit_rebuild(c))) return r;
@@ -1777,7 +1795,8 @@ static int force_pass(deme_ctx* c, bool full) {
     DEME_LAUNCH(c, "force",
                 launch_force_ctx(c, full, (uint32_t)c->C, c->idB[cu].p, c->ctype[cu].p, c->own.p,
                                  remap ? (c->havePrev ? c->hist[pv].p : c->hist[cu].p) : c->hist[cu].p,
-                                 remap ? c->map.p : nullptr, c->hist[cu].p, full ? c->frc.p : nullptr));
+                                 remap ? c->map.p : nullptr, c->hist[cu].p, full ? c->frc.p : nullptr, SpecGuard(),
+                                 settled && !remap));
     c->fresh = false;
     c->forcesFull = full;
     c->termsReady = true;
@@ -1894,7 +1913,7 @@ static std::vector<const void*> cycle_fingerprint(deme_ctx* c, int p) {
             c->bTerm.p,      c->aOn.p,        c->bOn.p,         c->analPartials.p,
             c->acc.p,        c->clock.p,      c->ctr.p,         c->planeStart.p,
             reinterpret_cast<const void*>(c->jit.full), reinterpret_cast<const void*>(c->jit.terms),
-            reinterpret_cast<const void*>(c->jitOwner.fn),
+            reinterpret_cast<const void*>(c->jitOwner.fn), v(c->fewTouch),
             v(c->slabCap),   v(c->nCells),    v(c->nS),         v(c->nO),         v(c->grid.nx),   v(c->grid.ny),
             v(c->grid.nz),   v(invBits),      v(c->jitActive),  v(c->ownerJitActive), v(c->maskAny),
             c->pos.p,        c->pos0.p,       c->meta.p,        c->candStart.p,   c->candB.p,      v(skinBits),
@@ -1949,7 +1968,7 @@ static int enqueue_cycle(deme_ctx* c, int f, const SpecGuard& g, int mode) {
         DEME_LAUNCH(c, "force",
                     launch_force_ctx(c, false, capC, c->idB[p].p, c->ctype[p].p, c->own.p,
                                      s == 0 ? c->hist[q].p : c->hist[p].p, s == 0 ? c->map.p : nullptr, c->hist[p].p,
-                                     nullptr, g));
+                                     nullptr, g, s > 0));
         DEME_LAUNCH(c, "owner_update", launch_owner_ctx(c, 1, p, g));
         // (only motion rules read the clock; the launch costs 4 us a step)
         if (c->ownerJitActive)
@@ -2028,6 +2047,7 @@ static int run_cycle(deme_ctx* c, int f, bool* done) {
     DEME_HIP(c, hipStreamSynchronize(c->stream));
     const DevCounters& h = *c->hctr;
     const SpecGuard& g = cy.guard;
+    if (!h.err) count_touching(c, h);
     if (h.err || h.maxOcc > g.slabCap || h.total[1] > g.capC || h.total[2] > g.capP) {
         c->cycleFallbacks++;
         c->cycleBackoff = std::min<uint32_t>(std::max<uint32_t>(2 * c->cycleBackoff, 1), 64);
@@ -2485,7 +2505,7 @@ int deme_step(deme_ctx* c, int nSteps, int updateFreq) {
         if (!detect && !c->fresh && !records && c->useGraphs && !c->timing && !c->jitStale && c->stream) {
             if ((r = step_graph(c))) return r;
         } else {
-            r = force_pass(c, records);
+            r = force_pass(c, records, k > 0 && !detect);
             if (r) return r;
             r = collect_and_update(c, 1);
             if (r) return r;

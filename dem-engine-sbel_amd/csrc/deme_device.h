@@ -484,6 +484,8 @@ struct DevCounters {
     uint32_t pairCount;
     uint32_t err;
     uint32_t maxOcc;
+    // of the contacts listed with a drift margin, a sample (every 64th workgroup of candidates) and those that touch
+    uint32_t sampled, touching;
     uint32_t pad;
     unsigned long long nActive;
     unsigned long long total[4];

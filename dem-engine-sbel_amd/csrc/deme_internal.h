@@ -234,6 +234,11 @@ hipError_t launch_cand_tscatter(uint32_t nK, const uint32_t* candB, const uint32
                                 uint32_t* tC, hipStream_t st);
 hipError_t launch_cand_tsort(uint32_t nS, const uint32_t* tStart, uint32_t* tC, uint32_t* tPos, hipStream_t st);
 
+// Which kernel forms the terms of a list (the records of a list always come from the full one): every contact through
+// the model, or tested first and the contacts that touch packed (MARGIN; SETTLED: moreover the flags and histories are
+// those that the last launch on this list left).
+enum ForceKind { FORCE_KIND_ALL, FORCE_KIND_MARGIN, FORCE_KIND_SETTLED };
+
 // dyn.hip
 // aTerm: 6 floats per contact; bTerm: 6 floats per mirror entry; sums: the plane owners' partial sums, one set per
 // workgroup (anal_blocks(nC) of them); out (optional): full contact records
@@ -242,7 +247,7 @@ hipError_t launch_force(const KParams& P, uint32_t nC, const uint32_t* idA, cons
                         const PlanePose* pose, const deme_material* mats, const float4* histIn, const uint32_t* map,
                         float4* histOut, const uint32_t* mirror, float* aTerm, float* bTerm,
                         const PlaneSums& sums, uint8_t* aOn, uint8_t* bOn,
-                        ForceRec* out, hipStream_t st, SpecGuard guard = SpecGuard());
+                        ForceRec* out, hipStream_t st, SpecGuard guard = SpecGuard(), ForceKind kind = FORCE_KIND_ALL);
 // The owner update: nClumps clump owners and sums.nOwners analytical owners (numbered from sums.first). The first
 // workgroup folds the force kernel's partial sums, moves the analytical owners and refreshes the plane poses.
 hipError_t launch_owner_update(const KParams& P, uint32_t nO, uint32_t nClumps, const uint32_t* ownerSphStart,
@@ -322,7 +327,7 @@ inline uint32_t owner_blocks(uint32_t nClumps, uint32_t nAnalOwners) {
 }
 struct JitForce {
     hipModule_t mod = nullptr;
-    hipFunction_t full = nullptr, terms = nullptr, direct = nullptr;
+    hipFunction_t full = nullptr, terms = nullptr, margin = nullptr, direct = nullptr;
     void release();
     hipError_t load(const std::vector<char>& code);
     hipError_t launch(bool wantFull, const KParams& P, uint32_t nC, const uint32_t* idA, const uint32_t* idB,
@@ -330,7 +335,7 @@ struct JitForce {
                       const deme_anal_obj* anal, const PlanePose* pose, const deme_material* mats,
                       const float4* histIn, const uint32_t* map, float4* histOut, const uint32_t* mirror,
                       float* aTerm, float* bTerm, const PlaneSums& sums, uint8_t* aOn, uint8_t* bOn, ForceRec* out,
-                      hipStream_t st, SpecGuard guard = SpecGuard()) const;
+                      hipStream_t st, SpecGuard guard = SpecGuard(), ForceKind kind = FORCE_KIND_ALL) const;
     hipError_t launch_direct(const KParams& P, const DirectList& D, const SphereRec* sph, const OwnerRec* own,
                              const float4* moi, const deme_anal_obj* anal, const PlanePose* pose,
                              const deme_material* mats, float* aTerm, float* bTerm, const PlaneSums& sums,

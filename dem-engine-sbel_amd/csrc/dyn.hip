@@ -43,16 +43,20 @@ hipError_t launch_force(const KParams& P, uint32_t nC, const uint32_t* idA, cons
                         const SphereRec* sph, const OwnerRec* own, const float4* moi, const deme_anal_obj* anal,
                         const PlanePose* pose, const deme_material* mats, const float4* histIn, const uint32_t* map,
                         float4* histOut, const uint32_t* mirror, float* aTerm, float* bTerm,
-                        const PlaneSums& sums, uint8_t* aOn, uint8_t* bOn, ForceRec* out, hipStream_t st, SpecGuard guard) {
+                        const PlaneSums& sums, uint8_t* aOn, uint8_t* bOn, ForceRec* out, hipStream_t st, SpecGuard guard, ForceKind kind) {
     if (nC == 0) return hipSuccess;
     if (out)
         deme_force_full<<<blocks(nC, 256), 256, 0, st>>>(P, nC, idA, idB, ctype, sph, own, moi, anal, pose, mats, histIn,
                                                        map, histOut, mirror, aTerm, bTerm, sums, aOn, bOn, out,
-                                                       guard);
+                                                       guard, kind == FORCE_KIND_SETTLED);
+    else if (kind != FORCE_KIND_ALL)
+        deme_force_margin<<<blocks(nC, 1024), 256, 0, st>>>(P, nC, idA, idB, ctype, sph, own, moi, anal, pose, mats,
+                                                            histIn, map, histOut, mirror, aTerm, bTerm, sums, aOn,
+                                                            bOn, nullptr, guard, kind == FORCE_KIND_SETTLED);
     else
         deme_force_terms<<<blocks(nC, 256), 256, 0, st>>>(P, nC, idA, idB, ctype, sph, own, moi, anal, pose, mats,
                                                         histIn, map, histOut, mirror, aTerm, bTerm, sums, aOn, bOn,
-                                                        nullptr, guard);
+                                                        nullptr, guard, kind == FORCE_KIND_SETTLED);
     return hipGetLastError();
 }
 

@@ -123,7 +123,7 @@ int jit_compile(const std::string& src, const std::string& arch, std::vector<cha
 void JitForce::release() {
     if (mod) (void)hipModuleUnload(mod);
     mod = nullptr;
-    full = terms = direct = nullptr;
+    full = terms = margin = direct = nullptr;
 }
 
 hipError_t JitForce::load(const std::vector<char>& code) {
@@ -135,6 +135,7 @@ hipError_t JitForce::load(const std::vector<char>& code) {
     }
     if ((e = hipModuleGetFunction(&full, mod, "deme_force_full")) != hipSuccess) return e;
     if ((e = hipModuleGetFunction(&terms, mod, "deme_force_terms")) != hipSuccess) return e;
+    if ((e = hipModuleGetFunction(&margin, mod, "deme_force_margin")) != hipSuccess) return e;
     return hipModuleGetFunction(&direct, mod, "deme_force_direct");
 }
 
@@ -155,14 +156,16 @@ hipError_t JitForce::launch(bool wantFull, const KParams& P, uint32_t nC, const 
                             const float4* histIn, const uint32_t* map, float4* histOut, const uint32_t* mirror,
                             float* aTerm, float* bTerm, const PlaneSums& sums, uint8_t* aOn, uint8_t* bOn,
                             ForceRec* out,
-                            hipStream_t st, SpecGuard guard) const {
+                            hipStream_t st, SpecGuard guard, ForceKind kind) const {
     if (nC == 0) return hipSuccess;
     KParams p = P;
     PlaneSums ps = sums;
+    const bool tiles = !wantFull && kind != FORCE_KIND_ALL;
+    bool settled = kind == FORCE_KIND_SETTLED;
     void* args[] = {&p,    &nC,     &idA, &idB,     &ctype,  &sph,   &own,   &moi, &anal, &pose, &mats,
-                    &histIn, &map, &histOut, &mirror, &aTerm, &bTerm, &ps, &aOn, &bOn, &out, &guard};
-    const uint32_t grid = (nC + 255) / 256;
-    return hipModuleLaunchKernel(wantFull ? full : terms, grid, 1, 1, 256, 1, 1, 0, st, args, nullptr);
+                    &histIn, &map, &histOut, &mirror, &aTerm, &bTerm, &ps, &aOn, &bOn, &out, &guard, &settled};
+    const uint32_t grid = tiles ? (uint32_t)(((uint64_t)nC + 1023) / 1024) : (uint32_t)(((uint64_t)nC + 255) / 256);
+    return hipModuleLaunchKernel(wantFull ? full : tiles ? margin : terms, grid, 1, 1, 256, 1, 1, 0, st, args, nullptr);
 }
 
 void JitOwner::release() {

@@ -198,3 +198,20 @@ def test_lists_kept_over_replaced_states(steps):
     for d in (a, b):
         d.step(steps)
     _same(a, b)
+
+
+@pytest.mark.parametrize("how", ["ahead of time", "user model", "captured"])
+def test_margin_lists_tested_first_equal_all_through_the_model(how):
+    """A list of over 1M contacts with a drift margin, a sixth of them touching: tested in groups of 256 and packed,
+    against every contact through the model (the cell sweep knows no share that touches). Calls end within and between
+    detection passes; plane contacts' sums are folded from their places."""
+    sc = scenes.clump_settling(n_clumps=100_003, update_freq=5, beta_frac=0.2, velocity_sigma=0.3, omega_sigma=5.0,
+                               seed=58)
+    a, b = _pair(sc, (lambda d: d.set_force_model(LINEAR, ["contact_age"])) if how == "user model" else None)
+    if how == "captured":
+        a.set_step_graphs(True)
+    for chunk in (7, 3, 1, 14):
+        a.step(chunk, 5)
+        b.step(chunk, 5)
+        _same(a, b)
+    assert a.counts().nContacts > 1_000_000 and a.counts().nContacts % 256
