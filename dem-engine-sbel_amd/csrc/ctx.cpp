@@ -244,6 +244,7 @@ struct deme_ctx {
     DBuf<deme_anal_obj> anal;
     DBuf<PlanePose> pose;
     DBuf<deme_material> mats;
+    DBuf<MatPair> matPairs;
     DBuf<deme_family_rule> rules;
     DBuf<uint8_t> mask;
     DBuf<float> acc;  // 6 x nO
@@ -612,7 +613,7 @@ int deme_ctx_destroy(deme_ctx* c) {
     }
     for (auto e : c->evPool) (void)hipEventDestroy(e);
     c->sph.release(); c->own.release(); c->moi.release(); c->ownerSphStart.release(); c->anal.release();
-    c->pose.release(); c->mats.release(); c->rules.release(); c->mask.release(); c->acc.release();
+    c->pose.release(); c->mats.release(); c->matPairs.release(); c->rules.release(); c->mask.release(); c->acc.release();
     c->binCount.release(); c->binStart.release(); c->numBins.release(); c->numAnal.release(); c->rec.release();
     c->binEnt.release(); c->pairs.release(); c->rowCount.release(); c->bCnt.release(); c->bRowStart.release();
     c->bPart.release(); c->mirror.release(); c->scanScratch.release(); c->ctr.release();
@@ -811,7 +812,11 @@ int deme_upload_materials(deme_ctx* c, uint32_t n, const deme_material* m) {
     c->adjReady = false;  // recorded adjoint checkpoints no longer describe the system
     if (n == 0 || n > 256) return c->fail(DEME_ERR_INVALID_ARGUMENT, "1..256 materials required");
     DEME_HIP(c, c->mats.ensure(n, 1.0));
+    DEME_HIP(c, c->matPairs.ensure((size_t)n * n, 1.0));
     DEME_HIP(c, hipMemcpyAsync(c->mats.p, m, n * sizeof(deme_material), hipMemcpyHostToDevice, c->stream));
+    DEME_LAUNCH(c, "material_pairs", launch_material_pairs(c->mats.p, n, c->matPairs.p, c->stream));
+    c->kp.nM = n;
+    c->kp.pairs = c->matPairs.p;
     DEME_HIP(c, hipStreamSynchronize(c->stream));
     c->nM = n;
     c->hostMats.assign(m, m + n);

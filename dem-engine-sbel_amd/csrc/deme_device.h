@@ -96,7 +96,26 @@ struct KParams {
     // (at most 64). A single scene has planeStart = {0, nA}.
     const uint32_t* planeStart;
     uint32_t nScenes;
+    // what the frictional model makes of each pair of materials (a, b), at pairs[a * nM + b]
+    uint32_t nM;
+    const struct MatPair* pairs;
 };
+
+// Effective parameters of a pair of materials and the damping ratio of its restitution (0 to 1, negative).
+struct alignas(16) MatPair {
+    float E, G, mu, Crr, beta, pad[3];
+};
+__device__ __forceinline__ MatPair load_pair(const KParams& P, uint32_t a, uint32_t b) {
+    const float4* q = reinterpret_cast<const float4*>(P.pairs + a * P.nM + b);
+    const float4 v = q[0];
+    MatPair m;
+    m.E = v.x;
+    m.G = v.y;
+    m.mu = v.z;
+    m.Crr = v.w;
+    m.beta = reinterpret_cast<const float*>(q)[4];
+    return m;
+}
 
 // Range of analytical components a body of the given scene can touch.
 __device__ __forceinline__ void scene_planes(const KParams& P, uint32_t scene, uint32_t& a0, uint32_t& a1) {

@@ -76,6 +76,7 @@ using deme_dev::OwnerBuild;
 using deme_dev::PART_FROM_COUNTERS;
 using deme_dev::PlaneRefresh;
 using deme_dev::PlaneSums;
+using deme_dev::MatPair;
 // Plane-owner sums: each workgroup of the force kernel folds its ANAL_TILE contacts (256 lanes x ANAL_ITEMS) into
 // nAnalOwners x 6 partials, so the partials buffer holds anal_blocks(nC) x nAnalOwners x 6 floats.
 constexpr uint32_t ANAL_ITEMS = 1;
@@ -238,6 +239,9 @@ hipError_t launch_cand_tsort(uint32_t nS, const uint32_t* tStart, uint32_t* tC, 
 // the model, or tested first and the contacts that touch packed (MARGIN; SETTLED: moreover the flags and histories are
 // those that the last launch on this list left).
 enum ForceKind { FORCE_KIND_ALL, FORCE_KIND_MARGIN, FORCE_KIND_SETTLED };
+
+// The table of material pairs (nM x nM) that the frictional model reads.
+hipError_t launch_material_pairs(const deme_material* mats, uint32_t nM, MatPair* pairs, hipStream_t st);
 
 // dyn.hip
 // aTerm: 6 floats per contact; bTerm: 6 floats per mirror entry; sums: the plane owners' partial sums, one set per

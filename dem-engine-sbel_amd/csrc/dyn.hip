@@ -35,9 +35,21 @@ __global__ __launch_bounds__(256) void k_change_family(OwnerRec* own, uint32_t n
     if (o < nO && own[o].fam == from) own[o].fam = to;
 }
 
+__global__ __launch_bounds__(256) void k_material_pairs(const deme_material* __restrict__ mats, uint32_t nM,
+                                                        MatPair* __restrict__ pairs) {
+    const uint32_t k = blockIdx.x * blockDim.x + threadIdx.x;
+    if (k < nM * nM) pairs[k] = materialPair(mats[k / nM], mats[k % nM]);
+}
+
 inline uint32_t blocks(uint64_t n, uint32_t b) { return (uint32_t)((n + b - 1) / b); }
 
 }  // namespace
+
+hipError_t launch_material_pairs(const deme_material* mats, uint32_t nM, MatPair* pairs, hipStream_t st) {
+    if (nM == 0) return hipSuccess;
+    k_material_pairs<<<blocks((uint64_t)nM * nM, 256), 256, 0, st>>>(mats, nM, pairs);
+    return hipGetLastError();
+}
 
 hipError_t launch_force(const KParams& P, uint32_t nC, const uint32_t* idA, const uint32_t* idB, const uint8_t* ctype,
                         const SphereRec* sph, const OwnerRec* own, const float4* moi, const deme_anal_obj* anal,

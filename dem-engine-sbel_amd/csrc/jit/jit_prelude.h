@@ -58,6 +58,17 @@ __device__ __forceinline__ void matProxy2ContactParam(T& E_eff, T& G_eff, T& CoR
     Crr_eff = fmaxf(Crr_A, Crr_B);
 }
 
+// What the frictional model makes of a pair of materials: the effective parameters and the damping ratio of CoR.
+__device__ __forceinline__ deme_dev::MatPair materialPair(const deme_material& a, const deme_material& b) {
+    deme_dev::MatPair p{};
+    float CoR_cnt;
+    matProxy2ContactParam<float>(p.E, p.G, CoR_cnt, p.mu, p.Crr, a.E, a.nu, a.CoR, a.mu, a.Crr, b.E, b.nu, b.CoR, b.mu,
+                                 b.Crr);
+    const float loge = (CoR_cnt < DEME_TINY_FLOAT) ? log(DEME_TINY_FLOAT) : log(CoR_cnt);
+    p.beta = loge / sqrt(loge * loge + deme::PI_SQUARED);
+    return p;
+}
+
 // The two-output form (frictionless models): E* and CoR only. Model strings also call it mat2ProxyContactParam.
 template <typename T>
 __device__ __forceinline__ void matProxy2ContactParam(T& E_eff, T& CoR_eff, T E_A, T nu_A, T CoR_A, T E_B, T nu_B,
