@@ -786,6 +786,7 @@ int deme_upload_templates(deme_ctx* c, uint32_t nS, const uint32_t* sphOwner, co
     DEME_HIP(c, hipStreamSynchronize(c->stream));
     c->nS = nS;
     c->kp.nS = nS;
+    c->kp.oneSphere = c->singleSpheres ? 1 : 0;
     c->haveVolumes = false;  // per clump: re-uploaded with the templates
     c->nO = nO;
     c->nClumps = nClumps;
@@ -3273,6 +3274,7 @@ int deme_append_clumps(deme_ctx* c, uint32_t nNewSph, const uint32_t* sphOwner, 
     c->singleSpheres = single;
     c->nS = nS;
     c->kp.nS = nS;
+    c->kp.oneSphere = c->singleSpheres ? 1 : 0;
     c->nO = nO;
     c->nClumps = nC;
     c->maxMatSph = maxMat;

@@ -99,6 +99,7 @@ struct KParams {
     // what the frictional model makes of each pair of materials (a, b), at pairs[a * nM + b]
     uint32_t nM;
     const struct MatPair* pairs;
+    uint32_t oneSphere;  // 1: clump o is sphere o alone (its row bounds need no look-up of its spheres)
 };
 
 // Effective parameters of a pair of materials and the damping ratio of its restitution (0 to 1, negative).
@@ -563,7 +564,8 @@ __device__ __forceinline__ bool spec_skip(const SpecGuard& g) {
 // the same step obeys (that kernel itself checks the state it leaves, so it cannot read err); steps: owner updates
 // done; disp: the largest displacements since the build (bits of doubles, spread over DISP_SLOTS words).
 struct DirectState {
-    uint32_t err, skip, steps, pad;
+    // lines of their own: a word read by every wave beside one that atomics change misses the caches
+    uint32_t err, pad0[31], skip, pad1[31], steps, pad2[31];
     unsigned long long disp[64];
 };
 // The candidates: pairs c < nPair (candA < candB, tPos: slot of c in the transposed rows) and planes q < nPlane (sphere
