@@ -77,7 +77,8 @@ int deme_upload_families(deme_ctx* ctx, const uint8_t* mask, const deme_family_r
  * owner's scene. Spheres only meet analytical components of their owner's scene; components must come grouped by
  * scene, at most 64 per scene. Without this call everything is scene 0. Call after deme_upload_analytical. */
 int deme_upload_scenes(deme_ctx* ctx, uint32_t nScenes, const uint32_t* ownerScene, const uint32_t* analScene);
-/* State I/O (dT getters/setters, src/DEM/dT.cpp:1722-1806; initial encoding dT.cpp:572-575). */
+/* State I/O (dT getters/setters, src/DEM/dT.cpp:1722-1806; initial encoding dT.cpp:572-575). Candidate lists are kept:
+ * the next pass measures every sphere against them. */
 int deme_upload_state(deme_ctx* ctx, const deme_owner_state* s);
 int deme_download_state(deme_ctx* ctx, deme_owner_state* s);
 /* Drops the contact list with its tangential histories and restarts the step count and time at zero, so the next step
@@ -133,7 +134,9 @@ int deme_integrate(deme_ctx* ctx);
  * contact forces; needs no contact list. */
 int deme_integrate_owners(deme_ctx* ctx);
 /* The step loop (DEMDynamicThread::workerThread, dT.cpp:1527-1585) with a deterministic contact-update schedule:
- * detection on the state at steps k*f (f = max(update_freq, 1)), force -> collect -> integrate each step. */
+ * detection on the state at steps k*f (f = max(update_freq, 1)), force -> collect -> integrate each step. Detecting
+ * every step without a drift margin, all steps of a call but the last run on the candidate lists (deme_set_skin)
+ * without forming a contact list; the last runs its own pass, so list, map and records are those of every step. */
 int deme_step(deme_ctx* ctx, int n_steps, int update_freq);
 /* HIP-graph replay in deme_step (no counterpart in the reference, which launches every kernel and waits on the host
  * for each detection pass's counts). When on, each whole detection interval -- the detection pass and the update_freq
@@ -156,7 +159,8 @@ int deme_set_graph_headroom(deme_ctx* ctx, double factor, uint64_t slack);
  * automatic, starting at 0.2 x the mean sphere radius and adapted at each build, within 0.05-0.8 x, to the lists it
  * retires (widened 1.5x when they died within a pass, narrowed 0.75x when they outlasted 400 passes, left alone from
  * 30 passes on; lists shorter-lived than that steer it 1.25x at a time by their candidates x (1 + 2.7 / passes
- * lasted)); when lists die within 4 passes even at the widest skin, the cell sweep runs every pass for 64 passes
+ * lasted)), and where steps run on the candidates also chosen from the gaps between them and the largest speed; when
+ * lists die within 4 passes even at the widest skin, the cell sweep runs every pass for 64 passes
  * (doubling while that repeats, up to 4096) before lists are tried again. 0: off (the cell sweep every pass). The
  * build positions are kept in fixed point (a power-of-two unit u, about 2^-31 of twice the bin grid's largest
  * extent); a skin with skin / 2 <= 1 nm + 4u also runs the cell sweep (deme_candidate_stats then reports 0). */
