@@ -1344,6 +1344,9 @@ static int build_candidates(deme_ctx* c) {
     c->jumped = false;
     c->builtThisPass = true;
     c->passesSinceBuild = 0;
+    // from here on the lists in force are overwritten array by array (and their skin is no longer theirs): a build that
+    // fails part-way leaves none
+    c->candValid = false;
     int mode = 0;
     int r = cd_buffers(c, &mode);
     if (r) return r;

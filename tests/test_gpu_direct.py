@@ -215,3 +215,42 @@ def test_margin_lists_tested_first_equal_all_through_the_model(how):
         b.step(chunk, 5)
         _same(a, b)
     assert a.counts().nContacts > 1_000_000 and a.counts().nContacts % 256
+
+
+def test_a_failed_list_build_leaves_no_lists():
+    """A build that fails part-way (lists due for renewal, a sphere outside the world), then the state that the old lists
+    were built from: the next call builds anew instead of stepping on lists that are half the old build's. The other
+    system has its lists dropped by hand after the error."""
+    r, skin, v, h = 0.005, 1e-3, 2.0, 1e-5
+    g = np.stack(np.meshgrid(*[np.arange(6)] * 3, indexing="ij"), -1).reshape(-1, 3) * (2 * r * 0.9999)
+    xyz = np.concatenate([g - g.mean(0), [[0.055, 0.055, -0.055]]])
+    vel = np.random.default_rng(5).normal(0, 0.01, xyz.shape)
+    vel[-1] = (0.0, 0.0, v)
+    sc = scenes.spheres_scene(xyz, r, (0.1295, 0.1295, 0.1295), vel=vel, g=(0.0, 0.0, 0.0), planes=False, h=h)
+    # single steps until a pass renews the lists ahead of time (before they are stale, at one skin of the lone sphere's
+    # path: passes subtract the midpoint of the displacements): one step fewer leaves them due
+    probe = DeviceSystem(sc)
+    probe.set_skin(skin)
+    n = 0
+    while probe.candidate_stats()[2] < 2:
+        probe.step(1)
+        n += 1
+    assert 4 < n and n * v * h < 0.95 * skin
+    a, b = DeviceSystem(sc), DeviceSystem(sc)
+    for d in (a, b):
+        d.set_skin(skin)
+        for _ in range(n - 1):
+            d.step(1)
+        assert d.candidate_stats()[2] == 1
+        bad = d.get_state()
+        z = np.uint64(sc.params.nvXp2 + sc.params.nvYp2)
+        bad["voxelID"][-1] |= (~np.uint64(0) >> z) << z  # the last voxel in z: past the grid by its radius
+        d.set_state(bad)
+        with pytest.raises(DemeError):
+            d.step(20)
+        assert d.counts().nContacts > 200
+        if d is b:
+            d.set_skin(skin)
+        d.set_state(sc.state)
+        d.step(20)
+    _same(a, b)
