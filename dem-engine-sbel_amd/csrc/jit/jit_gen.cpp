@@ -73,6 +73,7 @@ bool model_substitutions(const std::string& model, std::vector<std::string> wild
     }
     out.push_back({"_materialDefs_", "const deme_jit::MatProp E{mats, 0}, nu{mats, 1}, CoR{mats, 2}, mu{mats, 3}, "
                                      "Crr{mats, 4}"});
+    out.push_back({"_materialPair_", "load_pair(P, pairMatA, pairMatB)"});
     out.push_back({"_forceModelIngredientDefinition_", def});
     out.push_back({"_forceModelIngredientAcqForA_", acqA});
     out.push_back({"_forceModelIngredientAcqForB_", acqB});
@@ -81,6 +82,28 @@ bool model_substitutions(const std::string& model, std::vector<std::string> wild
     out.push_back({"_forceModelContactWildcardDestroy_", wDestroy});
     out.push_back({"_DEMForceModel_", model});
     return true;
+}
+
+void apply_overrides(const Subst& overrides, Subst& out) {
+    bool arrays = false, pair = false;
+    for (const auto& kv : overrides) {
+        arrays |= kv.first == "_materialDefs_";
+        out.push_back(kv);
+    }
+    // (only for a model that reads the pair: replaced arrays need not hold all five properties)
+    for (const auto& kv : out)
+        pair |= kv.first != "_materialPair_" && whole_word(kv.second, "pairAB");
+    if (!arrays || !pair) return;
+    std::string v = "materialPair(";
+    for (const char* m : {"pairMatA", "pairMatB"}) {
+        v += "deme_material{";
+        for (const char* a : {"E", "nu", "CoR", "mu", "Crr"}) {
+            v += std::string("(float)") + a + "[" + m + "]";
+            v += std::string(a) == "Crr" ? "}" : ", ";
+        }
+        v += std::string(m) == "pairMatA" ? ", " : ")";
+    }
+    out.push_back({"_materialPair_", v});
 }
 
 void owner_substitutions(const std::string& velStrategy, const std::string& posStrategy,

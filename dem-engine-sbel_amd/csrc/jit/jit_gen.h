@@ -22,6 +22,10 @@ constexpr size_t MAX_CONTACT_WILDCARDS = 4;
 // reason) for more than MAX_CONTACT_WILDCARDS wildcards or a name that is not an identifier.
 bool model_substitutions(const std::string& model, std::vector<std::string> wildcards, Subst& out, std::string& err);
 
+// Explicit placeholder values in place of the generated ones. Where they replace the material arrays and the model reads
+// the record of its pair of materials, that record is formed from the arrays, since the uploaded table is not theirs.
+void apply_overrides(const Subst& overrides, Subst& out);
+
 // Simulation constants: read from the kernel parameters (p == nullptr) or written into the source as literals that
 // parse back to the exact values.
 void param_substitutions(const deme_sim_params* p, Subst& out);

@@ -49,7 +49,7 @@ bool jit_force_source(const std::string& model, const std::vector<std::string>& 
     deme_jitgen::Subst s;
     deme_jitgen::param_substitutions(p, s);
     if (!deme_jitgen::model_substitutions(model, wildcards, s, err)) return false;
-    for (const auto& kv : overrides) s.push_back(kv);
+    deme_jitgen::apply_overrides(overrides, s);
     src = deme_jitgen::render(deme_jit_text::force_kernel_tpl, s);
     return true;
 }

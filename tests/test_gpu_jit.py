@@ -110,3 +110,56 @@ def test_compile_errors_surface_and_the_adjoint_refuses_custom_models():
         dev.adjoint_forward(5, 5)
     dev.set_force_model(None)
     dev.adjoint_forward(5, 5)  # the built-in model differentiates again
+
+
+@pytest.mark.parametrize("skin", [None, 0.0])
+def test_baked_material_arrays_are_the_ones_the_builtin_model_uses(skin):
+    """The material arrays replaced by literals: states, records and histories are bit for bit those of the same values
+    uploaded, whatever the uploaded table holds, for steps on the candidates and on the contact list."""
+    sc = _scene()
+    sc.materials = np.repeat(sc.materials, 2)
+    sc.sph_mat = (np.arange(sc.n_spheres) % 2).astype(np.uint8)
+    sc.anal["material"] = 1
+    want = {"E": (2e6, 7e6), "nu": (0.25, 0.35), "CoR": (0.0, 0.7), "mu": (0.2, 0.6), "Crr": (0.02, 0.0)}
+    defs = "const float " + ", ".join(f"{k}[2] = {{{float(a)!r}f, {float(b)!r}f}}" for k, (a, b) in want.items())
+
+    def run(mats, arrays):
+        sc.materials = mats
+
+        def setup(d):
+            if skin is not None:
+                d.set_skin(skin)
+            if arrays:
+                d.jit_build({"_materialDefs_": arrays})
+
+        return _run(sc, setup)
+
+    other, mats = sc.materials.copy(), sc.materials.copy()
+    for k, v in want.items():
+        mats[k] = v
+    _, sa, fa, wa = run(mats, None)
+    _, sb, fb, wb = run(other, defs)
+    _, so, _, _ = run(other, None)
+    for k in STATE_KEYS:
+        assert np.array_equal(sa[k], sb[k]), k
+    for x, y in zip(fa, fb):
+        assert np.array_equal(x, y)
+    assert np.array_equal(wa, wb)
+    assert not np.array_equal(sa["vZ"], so["vZ"])
+
+
+def test_baked_arrays_of_a_user_model_hold_what_it_names():
+    """A user model that names one property compiles with that array alone."""
+    sc = _scene()
+    model = "force = (float)(E[bodyAMatType] * overlapDepth) * B2A;"
+    devs = []
+    for arrays in (None, "const double E[1] = {3.0e4}"):
+        sc.materials["E"] = 3.0e4 if arrays is None else 1.0
+        d = DeviceSystem(sc)
+        d.set_force_model(model)
+        if arrays:
+            d.jit_build({"_materialDefs_": arrays})
+        d.step(20)
+        devs.append(d.get_state())
+    for k in STATE_KEYS:
+        assert np.array_equal(devs[0][k], devs[1][k]), k
