@@ -206,7 +206,8 @@ struct deme_ctx {
     uint64_t cycleSlack = 1024;
     // force kernel specialised at run time (hipRTC); inactive: the ahead-of-time kernel of the built-in model
     JitForce jit;
-    bool jitActive = false, jitStale = false, jitCustom = false;
+    // jitHistory: the caller replaced how histories are read, written or destroyed
+    bool jitActive = false, jitStale = false, jitCustom = false, jitHistory = false;
     // owner update specialised with motion strategies / family change rules (inactive: the ahead-of-time kernel)
     JitOwner jitOwner;
     bool ownerJitActive = false;
@@ -1754,8 +1755,10 @@ static hipError_t ensure_partials(deme_ctx* c, uint64_t nC, double grow = 1.25) 
 // a second round of gathers before the model (0.64M contacts of which a sixth touch: 29.8 us against 26.3, all through
 // the model); a long list is bound by the model's instructions (1.3M: 35.8 against 44.6 us; 4.9M: 125 against 181), and
 // each quarter of the contacts that touches adds a round of the model (all touching: 243 us, so 0.4 is about even).
+// Testing first clears the history of a contact that does not touch; a caller's own way of destroying it runs in the
+// kernel that takes every contact.
 static ForceKind force_kind(const deme_ctx* c, uint64_t nC, bool settled) {
-    if (!term_flags(c, false) || nC < 1000000 || !c->fewTouch) return FORCE_KIND_ALL;
+    if (!term_flags(c, false) || nC < 1000000 || !c->fewTouch || (c->jitActive && c->jitHistory)) return FORCE_KIND_ALL;
     return settled ? FORCE_KIND_SETTLED : FORCE_KIND_MARGIN;
 }
 
@@ -2996,7 +2999,7 @@ int deme_set_force_model(deme_ctx* c, const char* model, const char* const* wild
     c->adjReady = false;
     if (!model) {
         c->jit.release();
-        c->jitActive = c->jitStale = c->jitCustom = false;
+        c->jitActive = c->jitStale = c->jitCustom = c->jitHistory = false;
         c->jitOverrides.clear();
         return DEME_OK;
     }
@@ -3013,6 +3016,7 @@ int deme_set_force_model(deme_ctx* c, const char* model, const char* const* wild
     c->jitActive = true;
     c->jitStale = true;
     c->jitCustom = true;
+    c->jitHistory = false;
     return jit_rebuild(c);
 }
 
@@ -3043,8 +3047,11 @@ int deme_jit_build(deme_ctx* c, const char* const* keys, const char* const* valu
         c->jitWildcards = {"delta_tan_x", "delta_tan_y", "delta_tan_z", "delta_time"};
         c->jitCustom = false;
     }
-    for (const auto& kv : ov)
+    c->jitHistory = false;
+    for (const auto& kv : ov) {
         if (kv.first == "_DEMForceModel_" || kv.first.rfind("_forceModel", 0) == 0) c->jitCustom = true;
+        if (kv.first.rfind("_forceModelContactWildcard", 0) == 0) c->jitHistory = true;
+    }
     c->jitOverrides = ov;
     c->jitActive = true;
     c->jitStale = true;

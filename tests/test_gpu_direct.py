@@ -254,3 +254,17 @@ def test_a_failed_list_build_leaves_no_lists():
         d.set_state(sc.state)
         d.step(20)
     _same(a, b)
+
+
+def test_margin_lists_destroy_histories_as_the_caller_says():
+    """A long margin list whose non-touching contacts get a caller's history instead of zeros."""
+    sc = scenes.clump_settling(n_clumps=100_003, update_freq=5, beta_frac=0.2, velocity_sigma=0.3, omega_sigma=5.0,
+                               seed=58)
+    away = "delta_tan_x = 0.f; delta_tan_y = 0.f; delta_tan_z = 0.f; delta_time -= 1.f;"
+    a, b = _pair(sc, lambda d: d.jit_build({"_forceModelContactWildcardDestroy_": away}))
+    for chunk in (7, 3, 6):
+        a.step(chunk, 5)
+        b.step(chunk, 5)
+        _same(a, b)
+    assert a.counts().nContacts > 1_000_000
+    assert (a.wildcards()[3] <= -1.0).mean() > 0.5
