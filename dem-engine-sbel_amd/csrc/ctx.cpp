@@ -2246,20 +2246,28 @@ static int direct_planes(deme_ctx* c) {
     return DEME_OK;
 }
 
-// The contact list's histories to the candidates, and the check of the current state.
-static int direct_enter(deme_ctx* c) {
-    int r = direct_planes(c);
+// The status cleared, then the check of the current state into it: a status is never cleared without the check of the
+// state that the next step starts from.
+static int direct_begin(deme_ctx* c) {
+    int r = direct_clear_state(c);
     if (r) return r;
-    if ((r = direct_clear_state(c))) return r;
-    const int cu = c->cur;
-    DEME_LAUNCH(c, "direct_enter", launch_direct_enter(direct_list(c), c->cidx[cu].p, c->rowStart[cu].p, c->idB[cu].p,
-                                                       c->ctype[cu].p, c->hist[cu].p, c->stream));
     DEME_LAUNCH(c, "direct_check", launch_direct_check(c->kp, direct_check(c), c->own.p, c->nClumps, c->pose.p, c->nA,
                                                        c->dstate.p, c->stream));
     return DEME_OK;
 }
 
-// New candidates from the current state, with the flags and histories of the old ones carried over.
+// The contact list's histories to the candidates, and the check of the current state.
+static int direct_enter(deme_ctx* c) {
+    int r = direct_planes(c);
+    if (r) return r;
+    const int cu = c->cur;
+    DEME_LAUNCH(c, "direct_enter", launch_direct_enter(direct_list(c), c->cidx[cu].p, c->rowStart[cu].p, c->idB[cu].p,
+                                                       c->ctype[cu].p, c->hist[cu].p, c->stream));
+    return direct_begin(c);
+}
+
+// New candidates from the current state, with the flags and histories of the old ones carried over, and the check of that
+// state (the status of the check before may not have been read yet).
 static int direct_rebuild(deme_ctx* c) {
     const DirectList old = direct_list(c);
     const int cu = c->cur;
@@ -2278,7 +2286,7 @@ static int direct_rebuild(deme_ctx* c) {
     DEME_LAUNCH(c, "direct_join",
                 launch_direct_join(c->nS, c->candStartOld.p, c->candBOld.p, c->candStart.p, c->candB.p, c->pStartOld.p,
                                    c->pPlaneOld.p, old, direct_list(c), c->stream));
-    return direct_clear_state(c);
+    return direct_begin(c);
 }
 
 // The contact list of the last step taken on the candidates, in place of the list it was entered with: the rows of the

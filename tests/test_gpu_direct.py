@@ -268,3 +268,62 @@ def test_margin_lists_destroy_histories_as_the_caller_says():
         _same(a, b)
     assert a.counts().nContacts > 1_000_000
     assert (a.wildcards()[3] <= -1.0).mean() > 0.5
+
+
+def _grazing_past_the_grid(m=17):
+    """A bin grid one bin wide in x. A pair at its upper end in x grazes along y: the contact point, moved past the lower
+    sphere's top by the rounding of the direction, falls into the next bin in y, which the sphere's linear bin ids hold
+    only because its range in x passes the grid's end (bin (1, j) is bin (0, j + 1)). A cloud with many near neighbours
+    makes a thinner skin pay at once."""
+    f32 = np.float32
+    r, rb, face = 0.005, 0.05, 0.5
+    ra64, rb64 = np.float64(f32(r)), np.float64(f32(rb))
+    g = np.stack(np.meshgrid(*[np.arange(m)] * 3, indexing="ij"), -1).reshape(-1, 3) * (2.1 * r)
+    xyz = np.concatenate([[[0.498, 0.49, 0.3], [0.498, 0.56, 0.3]], g + np.array([0.1, 0.6, 0.1])])
+    rad = np.full(len(xyz), r)
+    rad[1] = rb
+    sc = scenes.spheres_scene(xyz - 0.5, rad, (1.0, 1.0, 1.0), lbf=(-0.5, -0.5, -0.5), planes=False, g=(0, 0, 0))
+    p = sc.params
+    p.binSize, p.nbX, p.nbY, p.nbZ = face, 1, 4, 4
+
+    def enc(v):
+        k = int(v // p.voxelSize)
+        return k, int(round((v - k * p.voxelSize) / p.l))
+
+    def dec(q):
+        return np.float64(q[0]) * p.voxelSize + np.float64(q[1]) * p.l
+
+    rng = np.random.default_rng(0)
+    for _ in range(20000):
+        t = rng.uniform(1e-4, 6e-4)
+        qa = [enc(v) for v in (0.498, face - r - 8e-10, 0.3)]
+        a = np.array([dec(q) for q in qa])
+        d = ra64 + rb64 - 2e-10
+        qb = [enc(v) for v in (a[0] + d * np.sin(t), a[1] + d * np.cos(t), a[2])]
+        b = np.array([dec(q) for q in qb])
+        if max(q[1] for q in qa + qb) > 65535 or ((a - b) ** 2).sum() > (ra64 + rb64) ** 2:
+            continue
+        n = (a - b).astype(f32)
+        n /= np.sqrt(n[0] * n[0] + n[1] * n[1] + n[2] * n[2])
+        half = (ra64 + rb64 - np.sqrt(((a - b) ** 2).sum())) / 2
+        c = b + (rb64 - half) * n.astype(np.float64)
+        if a[1] / face + ra64 / face < 1.0 <= c[1] / face:
+            break
+    else:
+        raise AssertionError("no such pair")
+    for k, q in enumerate((qa, qb)):
+        sc.state["voxelID"][k] = q[0][0] | q[1][0] << p.nvXp2 | q[2][0] << (p.nvXp2 + p.nvYp2)
+        for f, v in zip(("locX", "locY", "locZ"), q):
+            sc.state[f][k] = v[1]
+    return sc
+
+
+def test_a_skin_narrowed_on_entry_keeps_the_check_of_the_state():
+    """The state is checked against the grid's end although the call's first act is to rebuild its lists."""
+    a, b = _pair(_grazing_past_the_grid())
+    for chunk in (1, 1, 2000):
+        for d in (a, b):
+            d.step(chunk)
+        assert chunk > 1 or b.counts().nContacts == 1
+        _same(a, b)
+    assert a.candidate_stats()[0] < 0.5 * b.scene.sph_radius.mean() * 0.2 and a.candidate_stats()[2] == 2
