@@ -194,9 +194,10 @@ struct deme_ctx {
     DBuf<PlanePose> pose0;
     DBuf<OwnerBuild> own0;  // the owners' poses at the build
     DBuf<SkinStats> skinStats;
-    // the automatic skin chosen from a build's statistics for the next build (0: none chosen), and the largest
-    // displacement per step seen lately (0: unknown)
-    double skinNext = 0.0, skinNextRatio = 1.0, stepMove = 0.0;  // (its candidates over the current lists')
+    // the automatic skin chosen from a build's statistics for the next build (skin 0: none chosen, the lists' lifetimes
+    // steer it), and the largest displacement per step seen lately (0: unknown)
+    SkinChoice skinNext{0.0, 1.0, 0.0};
+    double stepMove = 0.0;
     uint32_t nPlane = 0;
     uint64_t planesGen = 0;
     uint32_t directSkip = 0, directBackoff = 0;
@@ -1304,8 +1305,8 @@ static double stale_limit2(const deme_ctx* c) {
 // Candidate lists from the current state: the cell sweep in its build mode (pairs of different owners within the
 // skin of touching), rows of higher-id partners in id order (candStart / candB) and the build positions (pos0).
 static int build_candidates(deme_ctx* c) {
-    if (c->skinSet < 0.0 && c->skinNext > 0.0) {
-        c->skinAuto = c->skinNext;  // (chosen from the statistics of the lists being retired)
+    if (c->skinSet < 0.0 && c->skinNext.skin > 0.0) {
+        c->skinAuto = c->skinNext.skin;  // (chosen from the statistics of the lists being retired)
         c->skinCostPrev = -1.0;
         c->skinDir = 0;
     } else if (c->skinSet < 0.0 && c->candBuilds > 0 && c->candValid && !c->jumped) {
@@ -1334,9 +1335,9 @@ static int build_candidates(deme_ctx* c) {
             else if (c->skinDir < 0) next = cur * 0.8;
         }
         c->skinCostPrev = cost;
-        c->skinAuto = std::min(std::max(next, 0.05 * m), 0.8 * m);
+        c->skinAuto = std::min(std::max(next, 0.05 * m), SKIN_WIDEST * m);
     }
-    c->skinNext = 0.0;
+    c->skinNext.skin = 0.0;
     c->lastLifetime = c->candBuilds > 0 && !c->jumped ? c->passesSinceBuild : ~0ull;
     if (c->jumped && c->candValid) {
         c->jumpBackoff = std::min<uint32_t>(2 * c->jumpBackoff + 1, 15);
@@ -1493,7 +1494,7 @@ static void end_pass(deme_ctx* c, bool skinPass, double disp2) {
         c->rebuildNext = disp2 > lim * lim;
         // lists about to be rebuilt after fewer than 4 passes, or just rebuilt (found stale) after fewer than 4
         const bool dying = (c->rebuildNext && c->passesSinceBuild < 4) || (built && c->lastLifetime < 4);
-        if (dying && c->skinSet < 0.0 && c->skinAuto >= 0.8 * (double)c->meanRadius * (1.0 - 1e-9)) {
+        if (dying && c->skinSet < 0.0 && c->skinAuto >= SKIN_WIDEST * (double)c->meanRadius * (1.0 - 1e-9)) {
             c->cellBackoff = std::min<uint32_t>(c->cellBackoff ? 2 * c->cellBackoff : 64, 4096);
             c->cellPassesLeft = c->cellBackoff;
             c->candValid = false;
@@ -2149,51 +2150,17 @@ static int direct_clear_state(deme_ctx* c) {
     return DEME_OK;
 }
 
-// Seconds of a step on k candidates and of a build, fitted to 600 spheres to 1M clumps: the launches, then 70 ps a
-// candidate; a build some 25 launches and three waits, then about three steps over its candidates.
-static double direct_step_s(double k) { return 14e-6 + 70e-12 * k; }
-static double direct_build_s(double k) { return 300e-6 + 3.0 * 70e-12 * k; }
-
-// The automatic skin the statistics of the lists in force ask for: the smallest time per step, builds included, among
-// sixteenths of their skin and 1.25 and 1.5 times it, a build coming every time the fastest sphere moves half the skin.
-// *candRatio: its candidates over the current lists'. (1M clumps moving at 0.02 m/s: 0.2 r lists 4.98M candidates, 352 us
-// a step; the skin chosen 4.40M, 269 us.)
-static double choose_skin(const deme_ctx* c, const SkinStats& st, double* candRatio) {
-    const double s = c->skin(), m = (double)c->meanRadius;
+// The automatic skin that the statistics of the lists in force ask for (skin_choice.h).
+static SkinChoice chosen_skin(const deme_ctx* c, const SkinStats& st) {
     float speed;
     std::memcpy(&speed, &st.speedBits, sizeof(speed));
-    const double move = std::max({(double)speed * (double)c->sp.h, c->stepMove, 1e-30});
-    double total = 0.0;
-    for (uint32_t g : st.gaps) total += g;
-    *candRatio = 1.0;
-    if (!(total > 0.0) || !std::isfinite(move)) return s;
-    const double nK = (double)c->nCand;
-    auto cost = [&](double k, double skin) {
-        return direct_step_s(k * nK) + direct_build_s(k * nK) / std::max(0.5 * skin / move, 1.0);
-    };
-    double best = cost(1.0, s), bestSkin = s, below = 0.0;
-    for (uint32_t j = 1; j < SKIN_BUCKETS; j++) {
-        below += st.gaps[j - 1] / total;
-        const double skin = s * j / SKIN_BUCKETS;
-        if (skin < 0.01 * m) continue;
-        if (cost(below, skin) < best) {
-            best = cost(below, skin);
-            bestSkin = skin;
-            *candRatio = below;
-        }
-    }
-    // beyond the skin the lists say nothing: the count grows on as over their last quarter, somewhat faster
-    double last = 0.0;
-    for (uint32_t j = SKIN_BUCKETS - SKIN_BUCKETS / 4; j < SKIN_BUCKETS; j++) last += st.gaps[j] / total;
-    for (int q = 1; q <= 2; q++) {
-        const double skin = s * (1.0 + 0.25 * q), k = 1.0 + 1.2 * last * q;
-        if (skin <= 0.8 * m && cost(k, skin) < best) {
-            best = cost(k, skin);
-            bestSkin = skin;
-            *candRatio = k;
-        }
-    }
-    return bestSkin;
+    SkinView v;
+    v.skin = c->skin();
+    v.meanRadius = (double)c->meanRadius;
+    v.nCand = (double)c->nCand;
+    v.gaps = st.gaps;
+    v.move = std::max({(double)speed * (double)c->sp.h, c->stepMove, 1e-30});
+    return choose_skin(v);
 }
 
 // The plane candidates of the current state and the buffers of both kinds of candidates; with a new build also the skin
@@ -2219,10 +2186,7 @@ static int direct_planes(deme_ctx* c) {
                                        c->stream));
         }
         if ((r = readback_counters(c))) return r;
-        if (choose) {
-            const double s = choose_skin(c, c->hdstate->stats, &c->skinNextRatio);
-            c->skinNext = s != c->skin() ? s : 0.0;
-        }
+        if (choose) c->skinNext = chosen_skin(c, c->hdstate->stats);
         const uint64_t n = c->hctr->total[2];
         if (n > 0xFFFFFFFFull) return c->fail(DEME_ERR_CAPACITY, "plane candidate count exceeds 2^32 - 1");
         c->nPlane = (uint32_t)n;
@@ -2367,10 +2331,10 @@ static int run_direct(deme_ctx* c, int n, int* done, bool* again) {
     while (*done < n) {
         // a skin with clearly fewer candidates is taken at once when it pays for the build within its lifetime or the
         // rest of the call
-        if (c->skinNext > 0.0 && c->skinNext < c->skin() && !rebuilt) {
-            const double life = 0.5 * c->skinNext / std::max(c->stepMove, 1e-30), nK = (double)c->nCand;
-            const double gain = direct_step_s(nK) - direct_step_s(nK * c->skinNextRatio);
-            if (gain * std::min((double)(n - *done), life) > 1.5 * direct_build_s(nK * c->skinNextRatio)) {
+        const SkinChoice next = c->skinNext;
+        if (next.skin > 0.0 && next.skin < c->skin() && !rebuilt) {
+            const double nK = (double)c->nCand, gain = direct_step_s(nK) - direct_step_s(nK * next.ratio);
+            if (gain * std::min((double)(n - *done), next.life) > 1.5 * direct_build_s(nK * next.ratio)) {
                 if ((r = direct_rebuild(c))) {
                     c->contactsReady = c->havePrev = c->candValid = false;
                     return r;
@@ -2427,7 +2391,8 @@ static int run_direct(deme_ctx* c, int n, int* done, bool* again) {
             std::memcpy(&v, &b, sizeof(v));
             dispMax = std::max(dispMax, v);
         }
-        if (c->passesSinceBuild >= 4 && !c->jumped)
+        // (displacements under an eighth of the limit are not reported; lists found stale after a step or two tell exactly)
+        if (c->passesSinceBuild > 0 && (c->passesSinceBuild >= 4 || (err & ERRBIT_STALE)) && !c->jumped)
             c->stepMove = std::max(dispMax, 0.125 * check.limit) / (double)c->passesSinceBuild;
         if (err & ERRBIT_STALE) c->rebuildNext = true;
         if (err & ~(uint32_t)ERRBIT_STALE) {
@@ -2447,7 +2412,7 @@ static int run_direct(deme_ctx* c, int n, int* done, bool* again) {
         // lists that die within 4 steps at the widest automatic skin give way to the cell sweep for a while, lists stale
         // right after a build to the pass (which reports why)
         giveUp = c->skinSet < 0.0 && c->passesSinceBuild < 4 &&
-                 c->skinAuto >= 0.8 * (double)c->meanRadius * (1.0 - 1e-9);
+                 c->skinAuto >= SKIN_WIDEST * (double)c->meanRadius * (1.0 - 1e-9);
         if (giveUp || (rebuilt && steps == 0)) {
             *again = false;
             break;
@@ -2562,7 +2527,7 @@ int deme_set_skin(deme_ctx* c, double skin) {
     c->skinSet = skin < 0.0 ? -1.0 : skin;
     c->skinAuto = 0.0;
     c->skinCostPrev = -1.0;
-    c->skinNext = c->stepMove = 0.0;
+    c->skinNext.skin = c->stepMove = 0.0;
     c->skinDir = 0;
     c->cellPassesLeft = 0;
     c->cellBackoff = 0;

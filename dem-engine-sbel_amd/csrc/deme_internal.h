@@ -8,6 +8,7 @@
 #include <vector>
 
 #include "deme_device.h"
+#include "skin_choice.h"
 
 namespace deme_int {
 
@@ -42,7 +43,7 @@ __device__ __forceinline__ int32_t build_fix(double x, double scale) {
     return (v > -2147483648.0 && v < 2147483648.0) ? (int32_t)v : INT32_MIN;
 }
 
-constexpr uint32_t SKIN_BUCKETS = 16, SKIN_SAMPLES = 65536;
+constexpr uint32_t SKIN_SAMPLES = 65536;
 struct SkinStats {
     uint32_t gaps[SKIN_BUCKETS];
     uint32_t speedBits;

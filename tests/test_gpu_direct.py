@@ -327,3 +327,39 @@ def test_a_skin_narrowed_on_entry_keeps_the_check_of_the_state():
         assert chunk > 1 or b.counts().nContacts == 1
         _same(a, b)
     assert a.candidate_stats()[0] < 0.5 * b.scene.sph_radius.mean() * 0.2 and a.candidate_stats()[2] == 2
+
+
+def test_a_calm_system_made_fast_gets_wider_lists():
+    """Thin lists of a system at rest, then all spheres at 0.04 radii a step: the lists must come to last some steps."""
+    r = 0.005
+    g = np.stack(np.meshgrid(*[np.arange(17)] * 3, indexing="ij"), -1).reshape(-1, 3) * (2.1 * r)
+    sc = scenes.spheres_scene(g - g.mean(0), r, (0.3, 0.3, 0.3), g=(0.0, 0.0, 0.0))
+    a, b = _pair(sc)
+    for d in (a, b):
+        d.step(1)
+        d.step(2000)
+    assert a.candidate_stats()[0] < 0.05 * r
+    v = np.random.default_rng(6).normal(size=(sc.n_clumps, 3))
+    v *= 0.04 * r / sc.params.h / np.linalg.norm(v, axis=1, keepdims=True)
+    st = a.get_state()
+    for k, f in enumerate(("vX", "vY", "vZ")):
+        st[f][:sc.n_clumps] = v[:, k]
+    before = a.candidate_stats()[2]
+    for d in (a, b):
+        d.set_state(st)
+        d.step(300)
+    _same(a, b)
+    assert a.candidate_stats()[0] > 0.25 * r
+    assert a.candidate_stats()[2] - before < 300 / 4
+
+
+def test_lists_that_never_last_give_way_to_the_cell_sweep():
+    sc, _ = _fast_gas()
+    a = DeviceSystem(sc)
+    a.step(1)
+    a.step(40)
+    assert a.candidate_stats()[0] == 0.0
+    builds = a.candidate_stats()[2]
+    assert builds < 20
+    a.step(200)
+    assert a.candidate_stats()[2] < builds + 20
