@@ -179,7 +179,7 @@ struct deme_ctx {
     // Stepping on the candidates (direct.hip): the status, the candidates' histories and the plane candidates with their
     // rows, flags, histories and terms; the old build's during a rebuild. The pairs' flags are candAcc[cur].
     // planesGen: the build (candBuilds) the plane candidates go with. directSkip: calls of deme_step that do not try
-    // (after a state near the grid's end, doubling up to 64 while that repeats).
+    // (after a state near the grid's end or with a plane owner that forces move, doubling up to 64 while that repeats).
     DBuf<DirectState> dstate;
     struct HostStatus {
         DirectState d;
@@ -189,7 +189,7 @@ struct deme_ctx {
     DBuf<float4> dHist, dHistOld, dPHist, dPHistOld;
     DBuf<uint8_t> dPOn, dPOnOld, dOnOld;
     DBuf<uint32_t> pStart, pStartOld, pSph, pPlane, pPlaneOld, candStartOld, candBOld;
-    DBuf<float> pTerm;
+    DBuf<float> pTerm, pForce;
     DBuf<unsigned long long> nearBits;
     DBuf<PlanePose> pose0;
     DBuf<OwnerBuild> own0;  // the owners' poses at the build
@@ -211,7 +211,7 @@ struct deme_ctx {
     bool jitActive = false, jitStale = false, jitCustom = false, jitHistory = false;
     // owner update specialised with motion strategies / family change rules (inactive: the ahead-of-time kernel)
     JitOwner jitOwner;
-    bool ownerJitActive = false;
+    bool ownerJitActive = false, rulesReadAcc = false;  // (family change rules that read the accelerations)
     std::vector<std::pair<std::string, std::string>> ownerValues;
     std::string jitModel;
     std::vector<std::string> jitWildcards;
@@ -654,7 +654,7 @@ int deme_ctx_destroy(deme_ctx* c) {
     c->dstate.release(); c->dHist.release(); c->dHistOld.release(); c->dPHist.release(); c->dPHistOld.release();
     c->dPOn.release(); c->dPOnOld.release(); c->dOnOld.release(); c->pStart.release(); c->pStartOld.release();
     c->pSph.release(); c->pPlane.release(); c->pPlaneOld.release(); c->candStartOld.release(); c->candBOld.release();
-    c->pTerm.release(); c->nearBits.release(); c->pose0.release(); c->own0.release();
+    c->pTerm.release(); c->pForce.release(); c->nearBits.release(); c->pose0.release(); c->own0.release();
     c->skinStats.release();
     c->pack.release();
     if (c->stage) (void)hipHostFree(c->stage);
@@ -884,6 +884,7 @@ int deme_upload_scenes(deme_ctx* c, uint32_t nScenes, const uint32_t* ownerScene
 
 int deme_upload_families(deme_ctx* c, const uint8_t* mask, const deme_family_rule* rules) {
     c->graphGen++;
+    c->directSkip = c->directBackoff = 0;  // (forces may no longer move a plane owner)
     c->adjReady = false;  // recorded adjoint checkpoints no longer describe the system
     DEME_HIP(c, c->mask.ensure(DEME_NUM_MASK_ENTRIES, 1.0));
     DEME_HIP(c, c->rules.ensure(DEME_NUM_FAMILIES, 1.0));
@@ -2111,7 +2112,9 @@ static DirectList direct_list(const deme_ctx* c) {
     d.hist = c->dHist.p;
     d.pHist = c->dPHist.p;
     d.pTerm = c->pTerm.p;
+    d.pForce = c->pForce.p;
     d.mask = c->maskAny ? c->mask.p : nullptr;
+    d.planesByList = c->rulesReadAcc ? 1 : 0;
     d.st = c->dstate.p;
     return d;
 }
@@ -2202,6 +2205,7 @@ static int direct_planes(deme_ctx* c) {
     DEME_HIP(c, c->dPOn.ensure(nP));
     DEME_HIP(c, c->dPHist.ensure(nP));
     DEME_HIP(c, c->pTerm.ensure(6 * nP));
+    DEME_HIP(c, c->pForce.ensure(6 * nP));
     DEME_HIP(c, c->dHist.ensure(nK));
     DEME_HIP(c, c->aTerm.ensure(6 * nK));
     DEME_HIP(c, c->bTerm.ensure(6 * nK));
@@ -2309,6 +2313,29 @@ static int direct_leave(deme_ctx* c) {
     return DEME_OK;
 }
 
+// The update of the plane owners that the last step on the candidates (at time t) held back: their sums by the places of
+// that step's contact list.
+static int direct_move_planes(deme_ctx* c, uint32_t held, double t) {
+    c->posesValid = false;
+    DEME_HIP(c, ensure_partials(c, c->C));
+    PlaneSums sums = plane_sums(c);
+    sums.nPart = anal_blocks(c->C);
+    sums.skip = ~held;
+    const PlaneRefresh planes = plane_refresh(c);
+    const int cu = c->cur;
+    DEME_LAUNCH(c, "direct_plane_sums", launch_direct_plane_sums(direct_list(c), (uint32_t)c->C, c->idA.p, c->idB[cu].p,
+                                                                 c->ctype[cu].p, c->anal.p, sums, c->stream));
+    if (c->ownerJitActive) DEME_LAUNCH(c, "set_clock", launch_set_clock(c->clock.p, t, c->stream));
+    DEME_LAUNCH(c, "owner_update",
+                c->ownerJitActive
+                    ? c->jitOwner.launch(c->kp, c->nO, 0, nullptr, nullptr, nullptr, nullptr, nullptr, nullptr, nullptr,
+                                         sums, planes, c->rules.p, c->own.p, c->own.p, c->acc.p, 1, c->clock.p, c->stream)
+                    : launch_owner_update(c->kp, c->nO, 0, nullptr, nullptr, nullptr, nullptr, nullptr, nullptr, nullptr,
+                                          sums, planes, c->rules.p, c->own.p, c->acc.p, 1, c->clock.p, c->stream));
+    c->posesValid = true;
+    return DEME_OK;
+}
+
 // Whether the next steps may run on the candidates: detection every step, no drift margin (a list with a margin holds
 // pairs that do not touch, which only a pass lists), and the current list and its histories index the lists in force.
 static bool direct_ready(const deme_ctx* c) {
@@ -2326,7 +2353,8 @@ static int run_direct(deme_ctx* c, int n, int* done, bool* again) {
     if (c->jitActive && c->jitStale && (r = jit_rebuild(c))) return r;
     if ((r = direct_enter(c))) return r;
     bool rebuilt = false, giveUp = false;
-    double dispMax = 0.0;
+    uint32_t held = 0;
+    double dispMax = 0.0, tLast = 0.0;  // (tLast: the time of the last step)
     uint32_t counted = 0;
     while (*done < n) {
         // a skin with clearly fewer candidates is taken at once when it pays for the build within its lifetime or the
@@ -2379,9 +2407,11 @@ static int run_direct(deme_ctx* c, int n, int* done, bool* again) {
         const uint32_t steps = c->hdstate->d.steps - counted, err = c->hdstate->d.err;
         counted = c->hdstate->d.steps;
         for (uint32_t k = 0; k < steps; k++) {
+            tLast = c->time;
             c->time += (double)c->sp.h;
             c->nSteps++;
         }
+        held = err & ERRBIT_DRIVEN ? c->hdstate->d.held : 0;
         *done += (int)steps;
         c->passesSinceBuild += steps;
         if (c->passesSinceBuild >= 4) c->cellBackoff = 0;
@@ -2428,6 +2458,7 @@ static int run_direct(deme_ctx* c, int n, int* done, bool* again) {
     }
     if (*done > 0 || rebuilt) {
         if ((r = direct_leave(c))) return r;
+        if (held && (r = direct_move_planes(c, held, tLast))) return r;
     }
     if (giveUp) {
         c->cellBackoff = std::min<uint32_t>(c->cellBackoff ? 2 * c->cellBackoff : 64, 4096);
@@ -3012,6 +3043,9 @@ int deme_jit_build(deme_ctx* c, const char* const* keys, const char* const* valu
             return c->fail(DEME_ERR_JIT, "hipRTC compilation of the motion rules failed:\n" + log);
         DEME_HIP(c, c->jitOwner.load(code));
         c->ownerValues = own;
+        c->rulesReadAcc = false;
+        for (const auto& kv : own)
+            c->rulesReadAcc |= kv.first == "_familyChangeRules_" && deme_jitgen::whole_word(kv.second, "acc");
         c->ownerJitActive = true;
         if (ov.empty()) return DEME_OK;
     }
@@ -3035,7 +3069,7 @@ int deme_clear_motion_rules(deme_ctx* c) {
     c->graphGen++;
     c->adjReady = false;
     c->jitOwner.release();
-    c->ownerJitActive = false;
+    c->ownerJitActive = c->rulesReadAcc = false;
     c->ownerValues.clear();
     return DEME_OK;
 }
@@ -3046,6 +3080,7 @@ int deme_change_family(deme_ctx* c, int from, int to) {
     if (!c->haveState) return c->fail(DEME_ERR_NOT_READY, "no owner state");
     c->adjReady = false;
     c->posesValid = false;  // (a component's family is part of its pose record)
+    c->directSkip = c->directBackoff = 0;  // (forces may no longer move a plane owner)
     DEME_LAUNCH(c, "change_family", launch_change_family(c->own.p, c->nO, (uint8_t)from, (uint8_t)to, c->stream));
     return DEME_OK;
 }

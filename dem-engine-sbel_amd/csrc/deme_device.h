@@ -238,12 +238,14 @@ __device__ __forceinline__ CdRec load_cd(const CdRec* __restrict__ p, uint32_t i
 
 // ERRBIT_STALE: a sphere moved too far since the candidate lists were built; they must be rebuilt and the pass redone
 // ERRBIT_EDGE: a sphere too near the bin grid's upper ends for stepping on the candidates
+// ERRBIT_DRIVEN: a plane owner that its contacts' forces move (see DirectList), whose update was left out
 enum : uint32_t {
     ERRBIT_CAPACITY = 1u,
     ERRBIT_PAIR_OVERFLOW = 2u,
     ERRBIT_OUTSIDE = 4u,
     ERRBIT_STALE = 8u,
-    ERRBIT_EDGE = 16u
+    ERRBIT_EDGE = 16u,
+    ERRBIT_DRIVEN = 32u
 };
 
 // --------------------------------------------------------------------------------------------------------------
@@ -491,7 +493,40 @@ struct PlaneSums {
     float* part = nullptr;
     uint32_t first = 0, nOwners = 0;  // owner numbers first .. first + nOwners - 1
     uint32_t nPart = 0;
+    uint32_t skip = 0;  // owners that the update leaves as they are (a bit each)
 };
+// The workgroup's partial sums of the plane owners' terms (gOwner < 0: the lane has none): per owner, wave butterflies
+// and the four waves in order, a fixed tree. Every lane of the workgroup calls this. Folding here instead of storing a
+// term per contact and launching two more kernels over the list saves those launches (6-9 us each at any size).
+__device__ __forceinline__ void fold_plane_terms(const PlaneSums& sums, int gOwner, const float (&g)[6]) {
+    if (sums.nOwners == 0) return;
+    __shared__ float waveSum[4][6];
+    float* dst = sums.part + (uint64_t)blockIdx.x * sums.nOwners * 6;
+    if (!__syncthreads_or(gOwner >= 0)) {
+        if (threadIdx.x < sums.nOwners * 6) dst[threadIdx.x] = 0.f;
+        return;
+    }
+    for (uint32_t k = 0; k < sums.nOwners; k++) {
+        const bool mine = gOwner == (int)k;
+        if (__any(mine)) {
+#pragma unroll
+            for (int c = 0; c < 6; c++) {
+                float v = mine ? g[c] : 0.f;
+#pragma unroll
+                for (int off = 32; off > 0; off >>= 1) v += __shfl_xor(v, off, 64);
+                if ((threadIdx.x & 63u) == 0) waveSum[threadIdx.x >> 6][c] = v;
+            }
+        } else if ((threadIdx.x & 63u) < 6) {
+            waveSum[threadIdx.x >> 6][threadIdx.x & 63u] = 0.f;
+        }
+        __syncthreads();
+        if (threadIdx.x < 6) {
+            const uint32_t c = threadIdx.x;
+            dst[k * 6 + c] = ((waveSum[0][c] + waveSum[1][c]) + waveSum[2][c]) + waveSum[3][c];
+        }
+        __syncthreads();
+    }
+}
 // What the owner update refreshes after moving the analytical owners: the poses of all nA components (pose null: none).
 struct PlaneRefresh {
     const deme_anal_obj* anal = nullptr;
@@ -562,22 +597,28 @@ __device__ __forceinline__ bool spec_skip(const SpecGuard& g) {
 // --------------------------------------------------------------------------------------------------------------
 // err: set by the checks of a state (ERRBIT_*), sticky; the force kernel copies it to skip, which the owner update of
 // the same step obeys (that kernel itself checks the state it leaves, so it cannot read err); steps: owner updates
-// done; disp: the largest displacements since the build (bits of doubles, spread over DISP_SLOTS words).
+// done; held: the plane owners left where they are (a bit each); disp: the largest displacements since the build (bits of doubles, spread over DISP_SLOTS words).
 struct DirectState {
     // lines of their own: a word read by every wave beside one that atomics change misses the caches
-    uint32_t err, pad0[31], skip, pad1[31], steps, pad2[31];
+    uint32_t err, pad0[31], skip, pad1[31], steps, held, pad2[30];
     unsigned long long disp[64];
 };
 // The candidates: pairs c < nPair (candA < candB, tPos: slot of c in the transposed rows) and planes q < nPlane (sphere
 // pSph, component pPlane; rows pStart by sphere). on / pOn: touched in the last step, whose history then stands in hist /
-// pHist; bOn: on by transposed slot. aTerm, pTerm: A's owner terms; bTerm: B's, by transposed slot.
+// pHist; bOn: on by transposed slot. aTerm, pTerm: A's owner terms; bTerm: B's, by transposed slot; pForce: the plane
+// owner's. A clump's terms are summed in the list's order. The plane owners' sums are folded by the places of the plane
+// candidates, which depend on the lists: their last bits may reach an owner's accelerations (which the last step of a
+// call, a pass's, writes anew) but not its motion. Where the forces would move one (its velocities not prescribed) the
+// owner update leaves it where it is and reports ERRBIT_DRIVEN; the host then sums that step's pForce by the contact list's
+// places and moves it. planesByList: treat any plane owner so (family change rules that read the accelerations).
 struct DirectList {
     uint32_t nPair, nPlane;
     const uint32_t *candA, *candB, *tPos, *pSph, *pPlane, *pStart;
     uint8_t *on, *pOn, *bOn;
     float4 *hist, *pHist;
-    float* pTerm;
+    float *pTerm, *pForce;
     const uint8_t* mask;  // family mask, null when every pair is allowed
+    uint32_t planesByList;
     DirectState* st;      // null: not stepping on candidates
 };
 // An owner's pose at a candidate build: its position in fixed point (as BuildPos), its orientation, and the largest

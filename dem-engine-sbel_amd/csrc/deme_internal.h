@@ -22,6 +22,7 @@ using deme_dev::ERRBIT_CAPACITY;
 using deme_dev::ERRBIT_PAIR_OVERFLOW;
 using deme_dev::ERRBIT_OUTSIDE;
 using deme_dev::ERRBIT_STALE;
+using deme_dev::ERRBIT_DRIVEN;
 using deme_dev::ForceRec;
 using deme_dev::KParams;
 using deme_dev::OwnerRec;
@@ -302,6 +303,9 @@ hipError_t launch_direct_plane_bits(const KParams& P, const SphereRec* sph, cons
                                     uint32_t* clear, uint32_t nClear, hipStream_t st);
 hipError_t launch_direct_leave(const DirectList& D, const uint32_t* cidx, const uint32_t* rowStart, float4* listHist,
                                hipStream_t st, SpecGuard guard);
+hipError_t launch_direct_plane_sums(const DirectList& D, uint32_t nC, const uint32_t* idA, const uint32_t* idB,
+                                    const uint8_t* ctype, const deme_anal_obj* anal, const PlaneSums& sums,
+                                    hipStream_t st);
 // state.hip: device arrays of one value per owner (null: not asked for / not given)
 struct StateArrays {
     uint64_t* voxel;

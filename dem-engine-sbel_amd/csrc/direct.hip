@@ -5,8 +5,9 @@
 // the history map (220 of 400 us a step), and small systems pay the launches. Between builds the candidates' own order
 // already is the canonical order, so the force kernel can take them directly: history and owner terms live in the
 // candidate's slots, a flag says whether it touched, and the owner update sums the flagged terms of the candidate rows
-// -- the same terms in the same order, bit for bit. A step is then two kernels (force, owner update), and the host reads
-// one status per batch of steps.
+// -- the same terms in the same order, bit for bit. Only the plane owners' sums are folded in another order; an owner that
+// they would move is left to the host, which folds that step's terms in the list's order (k_direct_plane_sums) and goes on
+// with passes. A step is then two kernels (force, owner update), and the host reads one status per batch of steps.
 //
 // This file holds what connects the two forms: the plane candidates (spheres near a plane, which the pair lists do not
 // hold), histories carried from the contact list to the candidates and back, and from one build's candidates to the
@@ -271,6 +272,27 @@ __global__ __launch_bounds__(256) void k_direct_leave(DirectList D, uint32_t pai
     listHist[rowStart[s] + k] = D.pHist[q];
 }
 
+// The plane owners' partial sums of the last step on the candidates by the places of the contact list (idA, idB, ctype; as
+// the force kernel over the list folds them), from the terms that the step left per plane candidate.
+__global__ __launch_bounds__(256) void k_direct_plane_sums(DirectList D, uint32_t nC, const uint32_t* __restrict__ idA,
+                                                           const uint32_t* __restrict__ idB,
+                                                           const uint8_t* __restrict__ ctype,
+                                                           const deme_anal_obj* __restrict__ anal, PlaneSums sums) {
+    const uint32_t i = blockIdx.x * 256u + threadIdx.x;
+    int gOwner = -1;
+    float g[6] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+    if (i < nC && ctype[i] == DEME_SPHERE_PLANE_CONTACT) {
+        const uint32_t s = idA[i], p = idB[i];
+        for (uint32_t q = D.pStart[s]; q < D.pStart[s + 1]; q++)
+            if (D.pPlane[q] == p) {
+                gOwner = (int)(anal[p].owner - sums.first);
+#pragma unroll
+                for (int k = 0; k < 6; k++) g[k] = D.pForce[(uint64_t)q * 6 + k];
+            }
+    }
+    fold_plane_terms(sums, gOwner, g);
+}
+
 inline uint32_t blocks(uint64_t n) { return (uint32_t)((n + 255) / 256); }
 
 }  // namespace
@@ -336,6 +358,14 @@ hipError_t launch_direct_plane_bits(const KParams& P, const SphereRec* sph, cons
                                     uint32_t* clear, uint32_t nClear, hipStream_t st) {
     if (nS == 0) return hipSuccess;
     k_direct_plane_bits<<<blocks(nS), 256, 0, st>>>(P, sph, own, nS, D, numAnal, planeBits, clear, nClear);
+    return hipGetLastError();
+}
+
+hipError_t launch_direct_plane_sums(const DirectList& D, uint32_t nC, const uint32_t* idA, const uint32_t* idB,
+                                    const uint8_t* ctype, const deme_anal_obj* anal, const PlaneSums& sums,
+                                    hipStream_t st) {
+    if (nC == 0) return hipSuccess;
+    k_direct_plane_sums<<<blocks(nC), 256, 0, st>>>(D, nC, idA, idB, ctype, anal, sums);
     return hipGetLastError();
 }
 

@@ -363,3 +363,49 @@ def test_lists_that_never_last_give_way_to_the_cell_sweep():
     assert builds < 20
     a.step(200)
     assert a.candidate_stats()[2] < builds + 20
+
+
+@pytest.mark.parametrize("how", ["free", "freed by a rule", "rule on its force"])
+def test_a_plate_that_its_contacts_move_does_not_depend_on_the_lists(how):
+    """A light plate thrown onto a bed: its accelerations move it, so their last bits must be those of the contact list
+    whatever the lists and however the steps are split into calls. It is free from the start, or let go by a family
+    change rule within a call, or held by a rule that reads its acceleration."""
+    n = 1500
+    sc = scenes.sphere_settling(n=n, spacing=1.98, jitter=0.0, velocity_sigma=0.2, omega_sigma=5.0, seed=61)
+    top = float(scenes.decode_positions(sc.params, *(sc.state[k] for k in ("voxelID", "locX", "locY", "locZ")))[:n, 2].max())
+    nc = sc.n_clumps
+    extra = np.zeros(1, ANAL_DTYPE)
+    extra[0]["owner"] = nc + 1
+    extra[0]["relPos"] = (0.0, 0.0, top + 0.97 * 0.005)
+    extra[0]["rot"] = (0.0, 0.0, -1.0)
+    extra[0]["mass"] = 0.3
+    sc.anal = np.concatenate([sc.anal, extra])
+    sc.state = {q: np.concatenate([v, v[nc:nc + 1]]) for q, v in sc.state.items()}
+    sc.state["family"][nc + 1] = 0 if how == "free" else 9
+    sc.state["vZ"][nc + 1] = -0.2
+    rule = np.zeros(1, RULE_DTYPE)[0]
+    rule["used"] = rule["linVelPrescribed"] = rule["rotVelPrescribed"] = 1
+    sc.rules[9] = rule
+    sc.n_owners = nc + 2
+    sc.owner_mass = np.append(sc.owner_mass, np.float32(0.3))
+    sc.owner_moi = np.ascontiguousarray(np.append(sc.owner_moi, np.full((1, 3), 0.003, np.float32), 0))
+    rules = {"free": None, "freed by a rule": "if (family_code == 9 && t > 2.35e-4f) newFamily = 0;",
+             "rule on its force": "if (family_code == 9 && acc.z > 2.0f) newFamily = 0;"}[how]
+    setup = (lambda d: d.set_motion_rules(family_change_rules=rules)) if rules else None
+    a, b = _pair(sc, setup)
+    c = DeviceSystem(sc)  # the automatic skin again, other calls
+    if setup:
+        setup(c)
+    total = 0
+    for chunk in (1, 40, 7, 60, 1, 90):
+        for d in (a, b):
+            d.step(chunk)
+        total += chunk
+        _same(a, b)
+    for _ in range(total // 9):
+        c.step(9)
+    c.step(total % 9)
+    sa, sb = a.get_state(), c.get_state()
+    for k in sa:
+        assert np.array_equal(sa[k], sb[k]), k
+    assert sa["vZ"][nc + 1] != sc.state["vZ"][nc + 1] and sa["omgX"][nc + 1] != 0.0
