@@ -2295,10 +2295,12 @@ static int direct_leave(deme_ctx* c) {
         const uint64_t C = c->hctr->total[1], nPairs = c->hctr->total[2];
         if (C > 0xFFFFFFFFull) return c->fail(DEME_ERR_CAPACITY, "contact count exceeds contactPairs_t (2^32 - 1)");
         if (nPairs > C) return c->fail(DEME_ERR_HIP, "inconsistent contact and mirror-row counts");
-        c->C = C;
-        c->nPairs = nPairs;
-        c->nGeo = C - nPairs;
-        if (C <= g.capC) break;
+        if (C <= g.capC) {
+            c->C = C;
+            c->nPairs = nPairs;
+            c->nGeo = C - nPairs;
+            break;
+        }
         if (attempt) return c->fail(DEME_ERR_CAPACITY, "contact list could not be sized");
         DEME_HIP(c, c->idB[cu].ensure(C));
         DEME_HIP(c, c->ctype[cu].ensure(C));
@@ -2343,15 +2345,9 @@ static bool direct_ready(const deme_ctx* c) {
            c->candValid && c->cidxGen[c->cur] == c->candBuilds;
 }
 
-// Up to n steps on the candidates, in batches the host enqueues without waiting: a batch whose state fails the check
-// part-way leaves the rest of its kernels skipped, and the count of steps done comes back with its status. *done: steps
-// taken; *again: the lists were kept or rebuilt to the end (else the caller goes on with passes).
-static int run_direct(deme_ctx* c, int n, int* done, bool* again) {
-    *done = 0;
-    *again = true;
+// Steps on the candidates once their histories are in place, and back to the contact list (run_direct).
+static int direct_steps(deme_ctx* c, int n, int* done, bool* again) {
     int r = 0;
-    if (c->jitActive && c->jitStale && (r = jit_rebuild(c))) return r;
-    if ((r = direct_enter(c))) return r;
     bool rebuilt = false, giveUp = false;
     uint32_t held = 0;
     double dispMax = 0.0, tLast = 0.0;  // (tLast: the time of the last step)
@@ -2363,10 +2359,7 @@ static int run_direct(deme_ctx* c, int n, int* done, bool* again) {
         if (next.skin > 0.0 && next.skin < c->skin() && !rebuilt) {
             const double nK = (double)c->nCand, gain = direct_step_s(nK) - direct_step_s(nK * next.ratio);
             if (gain * std::min((double)(n - *done), next.life) > 1.5 * direct_build_s(nK * next.ratio)) {
-                if ((r = direct_rebuild(c))) {
-                    c->contactsReady = c->havePrev = c->candValid = false;
-                    return r;
-                }
+                if ((r = direct_rebuild(c))) return r;
                 rebuilt = true;
                 dispMax = 0.0;
                 counted = 0;
@@ -2447,11 +2440,7 @@ static int run_direct(deme_ctx* c, int n, int* done, bool* again) {
             *again = false;
             break;
         }
-        if ((r = direct_rebuild(c))) {
-            // (out of memory in the build) the candidates and their histories are gone
-            c->contactsReady = c->havePrev = c->candValid = false;
-            return r;
-        }
+        if ((r = direct_rebuild(c))) return r;
         rebuilt = true;
         dispMax = 0.0;
         counted = 0;
@@ -2467,6 +2456,25 @@ static int run_direct(deme_ctx* c, int n, int* done, bool* again) {
         c->graphGen++;
     }
     return DEME_OK;
+}
+
+// Up to n steps on the candidates, in batches the host enqueues without waiting: a batch whose state fails the check
+// part-way leaves the rest of its kernels skipped, and the count of steps done comes back with its status. *done: steps
+// taken; *again: the lists were kept or rebuilt to the end (else the caller goes on with passes).
+static int run_direct(deme_ctx* c, int n, int* done, bool* again) {
+    *done = 0;
+    *again = true;
+    int r = 0;
+    if (c->jitActive && c->jitStale && (r = jit_rebuild(c))) return r;
+    c->termsReady = false;  // (the terms' buffers hold the candidates' from here on)
+    if ((r = direct_enter(c))) return r;
+    if ((r = direct_steps(c, n, done, again))) {
+        // (out of memory) neither the lists nor the contact list can be relied on: the candidates' histories and flags
+        // moved on, the list's buffers may be short of its count
+        c->contactsReady = c->havePrev = c->candValid = c->forcesFull = false;
+        c->C = c->nPairs = c->nGeo = 0;
+    }
+    return r;
 }
 
 // Steps on the candidates pay once a call holds this many: entering and leaving cost about two passes.
