@@ -464,6 +464,21 @@ int ensure_poses(deme_ctx* c) {
 }
 
 // ---- caller arrays: packed on the device, moved through pinned slots ----
+// The context's device as the calling thread's current one, and the caller's again at the end: these calls allocate and
+// launch, whatever device the thread is on (plain copies on the context's stream would not care).
+struct DeviceScope {
+    int prev = -1;
+    explicit DeviceScope(int device) {
+        int d = device;
+        if (hipGetDevice(&d) == hipSuccess && d != device && hipSetDevice(device) == hipSuccess) prev = d;
+    }
+    ~DeviceScope() {
+        if (prev >= 0) (void)hipSetDevice(prev);
+    }
+    DeviceScope(const DeviceScope&) = delete;
+    DeviceScope& operator=(const DeviceScope&) = delete;
+};
+
 // One array of the caller at byte `off` of the packed buffer.
 struct PackedArray {
     size_t off, bytes;
@@ -938,6 +953,7 @@ StateArrays state_arrays(const deme_ctx* c, const StateOffsets& o) {
 extern "C" {
 
 int deme_upload_state(deme_ctx* c, const deme_owner_state* s) {
+    const DeviceScope onDevice(c->device);
     c->posesValid = false;
     // candidate lists stay: the next pass measures every sphere against its position at the build, whatever moved it
     if (c->jumpSkip > 0) {
@@ -980,6 +996,7 @@ int deme_clear_contacts(deme_ctx* c) {
 }
 
 int deme_download_state(deme_ctx* c, deme_owner_state* s) {
+    const DeviceScope onDevice(c->device);
     if (!c->haveState) return c->fail(DEME_ERR_NOT_READY, "no owner state");
     Packing k;
     const StateOffsets at = pack_state(k, s, c->nO);
@@ -1686,6 +1703,7 @@ int deme_download_bins(deme_ctx* c, uint32_t* binStart, uint32_t* binSphere) {
 }
 
 int deme_download_contacts(deme_ctx* c, uint32_t* idA, uint32_t* idB, uint8_t* type, uint32_t* map) {
+    const DeviceScope onDevice(c->device);
     if (!c->contactsReady) return c->fail(DEME_ERR_NOT_READY, "no contact list");
     const size_t C = c->C;
     const int cu = c->cur;
@@ -3094,6 +3112,7 @@ int deme_change_family(deme_ctx* c, int from, int to) {
 }
 
 int deme_download_forces(deme_ctx* c, float* F, float* T, float* cA, float* cB) {
+    const DeviceScope onDevice(c->device);
     if (!c->contactsReady) return c->fail(DEME_ERR_NOT_READY, "no contact list");
     if (!c->forcesFull)
         return c->fail(DEME_ERR_NOT_READY, "contact records are kept by deme_force only (deme_step stores owner terms)");
@@ -3111,6 +3130,7 @@ int deme_download_forces(deme_ctx* c, float* F, float* T, float* cA, float* cB) 
 }
 
 int deme_download_wildcards(deme_ctx* c, float* w) {
+    const DeviceScope onDevice(c->device);
     if (!c->contactsReady) return c->fail(DEME_ERR_NOT_READY, "no contact list");
     const size_t C = c->C;
     Packing k;
