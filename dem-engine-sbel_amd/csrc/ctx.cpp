@@ -174,8 +174,9 @@ struct deme_ctx {
         else s = skinAuto > 0.0 ? skinAuto : 0.2 * (double)meanRadius;
         // a skin too thin for the build positions' fixed-point unit (a world very large for its spheres) would find
         // every pass stale: the cell sweep runs instead
-        return 0.5 * s > SKIN_SLACK + 4.0 * posUnit ? s : 0.0;
+        return s > least_skin() ? s : 0.0;
     }
+    double least_skin() const { return 2.0 * (SKIN_SLACK + 4.0 * posUnit); }
     // Stepping on the candidates (direct.hip): the status, the candidates' histories and the plane candidates with their
     // rows, flags, histories and terms; the old build's during a rebuild. The pairs' flags are candAcc[cur].
     // planesGen: the build (candBuilds) the plane candidates go with. directSkip: calls of deme_step that do not try
@@ -2181,6 +2182,7 @@ static SkinChoice chosen_skin(const deme_ctx* c, const SkinStats& st) {
     v.nCand = (double)c->nCand;
     v.gaps = st.gaps;
     v.move = std::max({(double)speed * (double)c->sp.h, c->stepMove, 1e-30});
+    v.least = 1.001 * c->least_skin();
     return choose_skin(v);
 }
 

@@ -24,6 +24,7 @@ struct SkinView {
     double nCand;          // candidates of the lists in force
     const uint32_t* gaps;  // a sample of their gaps, in sixteenths of the skin
     double move;           // the largest displacement of a step
+    double least;          // thinner skins are not kept (the build positions' unit)
 };
 struct SkinChoice {
     double skin;
@@ -59,7 +60,7 @@ inline SkinChoice choose_skin(const SkinView& v) {
     for (uint32_t j = 1; j < SKIN_BUCKETS; j++) {
         below += v.gaps[j - 1] / total;
         const double skin = s * j / SKIN_BUCKETS;
-        if (skin >= 0.01 * m) look(skin, below);
+        if (skin >= std::max(0.01 * m, v.least)) look(skin, below);
     }
     // beyond the skin the lists say nothing: the count grows on as over their last quarter, somewhat faster, and with the
     // area of the shell

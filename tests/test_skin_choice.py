@@ -12,8 +12,9 @@ ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
 BUCKETS = 16
 SRC = """
 #include "skin_choice.h"
-extern "C" void choose(double skin, double radius, double nCand, const uint32_t* gaps, double move, double* out) {
-    const deme_int::SkinChoice c = deme_int::choose_skin({skin, radius, nCand, gaps, move});
+extern "C" void choose(double skin, double radius, double nCand, const uint32_t* gaps, double move, double least,
+                       double* out) {
+    const deme_int::SkinChoice c = deme_int::choose_skin({skin, radius, nCand, gaps, move, least});
     out[0] = c.skin;
     out[1] = c.ratio;
     out[2] = c.life;
@@ -29,11 +30,11 @@ def choose(tmp_path_factory):
     subprocess.run(["g++", "-std=c++17", "-O1", "-shared", "-fPIC", "-Wall", "-Werror", "-I", inc, str(d / "s.cpp"), "-o",
                     str(d / "s.so")], check=True)
     lib = C.CDLL(str(d / "s.so"))
-    lib.choose.argtypes = [C.c_double, C.c_double, C.c_double, C.c_void_p, C.c_double, C.c_void_p]
+    lib.choose.argtypes = [C.c_double, C.c_double, C.c_double, C.c_void_p, C.c_double, C.c_double, C.c_void_p]
 
-    def call(skin, radius, n_cand, gaps, move):
+    def call(skin, radius, n_cand, gaps, move, least=0.0):
         out = np.zeros(3)
-        lib.choose(skin, radius, n_cand, gaps.ctypes.data, move, out.ctypes.data)
+        lib.choose(skin, radius, n_cand, gaps.ctypes.data, move, least, out.ctypes.data)
         return out
 
     return call
@@ -81,3 +82,15 @@ def test_a_skin_is_kept_when_nothing_is_known(choose):
     assert choose(0.2, 1.0, 1e5, none, 0.01)[0] == 0.2
     for move in (np.nan, np.inf):
         assert choose(0.2, 1.0, 1e5, some, move)[0] == 0.2
+
+
+def test_no_skin_thinner_than_is_kept_is_chosen(choose):
+    """A world so large for its spheres that the build positions' unit rules out skins that gaps and speed ask for."""
+    skin, least = 0.2, 0.03
+    for _ in range(20):
+        edges = _partners(np.arange(BUCKETS + 1) * skin / BUCKETS, 1e6, 0.6, 3.0)
+        edges[0] = 0.0
+        gaps = np.round(np.diff(edges) / edges[-1] * 65536).astype(np.uint32)
+        skin = choose(skin, 1.0, edges[-1], gaps, 1e-9, least)[0]
+        assert skin >= least
+    assert skin < 0.06
