@@ -539,11 +539,13 @@ struct DevCounters {
     uint32_t pairCount;
     uint32_t err;
     uint32_t maxOcc;
-    // of the contacts listed with a drift margin, a sample (every 64th workgroup of candidates) and those that touch
-    uint32_t sampled, touching;
     uint32_t pad;
     unsigned long long nActive;
     unsigned long long total[4];
+    uint32_t pad1[18];
+    // of the contacts listed with a drift margin, a sample (every 64th workgroup of candidates) and those that touch; on a
+    // line of their own, since every wave that counts them reads err first
+    uint32_t sampled, touching, pad2[30];
     // largest squared displacement (bits of a non-negative double) of a sphere since the candidate lists were built,
     // spread over DISP_SLOTS words (workgroup b folds into word b % DISP_SLOTS: one address per workgroup would
     // serialize the atomics); the largest word is the maximum
@@ -552,6 +554,8 @@ struct DevCounters {
     // images of the doubles, the minima complemented, so every word folds with atomicMax from a cleared zero)
     unsigned long long dispLo[3][64], dispHi[3][64];
 };
+static_assert(__builtin_offsetof(DevCounters, sampled) == 128 && __builtin_offsetof(DevCounters, disp2) == 256,
+              "the sample's counters have a cache line of their own");
 constexpr uint32_t DISP_SLOTS = 64;
 // The host reads the counters up to the displacement extremes (the device alone uses those).
 constexpr size_t DEV_COUNTERS_HOST_BYTES = __builtin_offsetof(DevCounters, dispLo);
