@@ -190,7 +190,7 @@ struct deme_ctx {
     DBuf<float4> dHist, dHistOld, dPHist, dPHistOld;
     DBuf<uint8_t> dPOn, dPOnOld, dOnOld;
     DBuf<uint32_t> pStart, pStartOld, pSph, pPlane, pPlaneOld, candStartOld, candBOld;
-    DBuf<float> pTerm, pForce;
+    DBuf<float> pTerm;
     DBuf<unsigned long long> nearBits;
     DBuf<PlanePose> pose0;
     DBuf<OwnerBuild> own0;  // the owners' poses at the build
@@ -670,7 +670,7 @@ int deme_ctx_destroy(deme_ctx* c) {
     c->dstate.release(); c->dHist.release(); c->dHistOld.release(); c->dPHist.release(); c->dPHistOld.release();
     c->dPOn.release(); c->dPOnOld.release(); c->dOnOld.release(); c->pStart.release(); c->pStartOld.release();
     c->pSph.release(); c->pPlane.release(); c->pPlaneOld.release(); c->candStartOld.release(); c->candBOld.release();
-    c->pTerm.release(); c->pForce.release(); c->nearBits.release(); c->pose0.release(); c->own0.release();
+    c->pTerm.release(); c->nearBits.release(); c->pose0.release(); c->own0.release();
     c->skinStats.release();
     c->pack.release();
     if (c->stage) (void)hipHostFree(c->stage);
@@ -2131,9 +2131,7 @@ static DirectList direct_list(const deme_ctx* c) {
     d.hist = c->dHist.p;
     d.pHist = c->dPHist.p;
     d.pTerm = c->pTerm.p;
-    d.pForce = c->pForce.p;
     d.mask = c->maskAny ? c->mask.p : nullptr;
-    d.planesByList = c->rulesReadAcc ? 1 : 0;
     d.st = c->dstate.p;
     return d;
 }
@@ -2224,8 +2222,7 @@ static int direct_planes(deme_ctx* c) {
     const size_t nK = std::max<size_t>(c->nCand, 1), nP = std::max<size_t>(c->nPlane, 1);
     DEME_HIP(c, c->dPOn.ensure(nP));
     DEME_HIP(c, c->dPHist.ensure(nP));
-    DEME_HIP(c, c->pTerm.ensure(6 * nP));
-    DEME_HIP(c, c->pForce.ensure(6 * nP));
+    DEME_HIP(c, c->pTerm.ensure(12 * nP));
     DEME_HIP(c, c->dHist.ensure(nK));
     DEME_HIP(c, c->aTerm.ensure(6 * nK));
     DEME_HIP(c, c->bTerm.ensure(6 * nK));
@@ -2342,7 +2339,7 @@ static int direct_move_planes(deme_ctx* c, uint32_t held, double t) {
     DEME_HIP(c, ensure_partials(c, c->C));
     PlaneSums sums = plane_sums(c);
     sums.nPart = anal_blocks(c->C);
-    sums.skip = ~held;
+    sums.flags = ~held & 0xFFu;
     const PlaneRefresh planes = plane_refresh(c);
     const int cu = c->cur;
     DEME_LAUNCH(c, "direct_plane_sums", launch_direct_plane_sums(direct_list(c), (uint32_t)c->C, c->idA.p, c->idB[cu].p,
@@ -2393,6 +2390,7 @@ static int direct_steps(deme_ctx* c, int n, int* done, bool* again) {
         const DirectList d = direct_list(c);
         PlaneSums sums = plane_sums(c);
         sums.nPart = (c->nPlane + 255) / 256;
+        sums.flags = c->rulesReadAcc ? PLANES_BY_LIST : 0u;
         const PlaneRefresh planes = plane_refresh(c);
         double t = c->time;
         for (int k = 0; k < batch; k++) {

@@ -488,12 +488,13 @@ __device__ __forceinline__ PlanePose plane_pose_of(const KParams& P, const deme_
 // force workgroup (ANAL_TILE contacts) writes nOwners x 6 partial sums at part[block * nOwners * 6]; the owner update
 // folds nPart of them (PART_FROM_COUNTERS: the number of blocks of the guard's contact count).
 constexpr uint32_t PART_FROM_COUNTERS = 0xFFFFFFFFu;
+constexpr uint32_t PLANES_BY_LIST = 0x100u;  // (see DirectList)
 constexpr uint32_t MAX_ANAL_OWNERS = 8;
 struct PlaneSums {
     float* part = nullptr;
     uint32_t first = 0, nOwners = 0;  // owner numbers first .. first + nOwners - 1
     uint32_t nPart = 0;
-    uint32_t skip = 0;  // owners that the update leaves as they are (a bit each)
+    uint32_t flags = 0;  // a bit for each owner that the update leaves as it is, and PLANES_BY_LIST
 };
 // The workgroup's partial sums of the plane owners' terms (gOwner < 0: the lane has none): per owner, wave butterflies
 // and the four waves in order, a fixed tree. Every lane of the workgroup calls this. Folding here instead of storing a
@@ -609,20 +610,21 @@ struct DirectState {
 };
 // The candidates: pairs c < nPair (candA < candB, tPos: slot of c in the transposed rows) and planes q < nPlane (sphere
 // pSph, component pPlane; rows pStart by sphere). on / pOn: touched in the last step, whose history then stands in hist /
-// pHist; bOn: on by transposed slot. aTerm, pTerm: A's owner terms; bTerm: B's, by transposed slot; pForce: the plane
-// owner's. A clump's terms are summed in the list's order. The plane owners' sums are folded by the places of the plane
-// candidates, which depend on the lists: their last bits may reach an owner's accelerations (which the last step of a
-// call, a pass's, writes anew) but not its motion. Where the forces would move one (its velocities not prescribed) the
-// owner update leaves it where it is and reports ERRBIT_DRIVEN; the host then sums that step's pForce by the contact list's
-// places and moves it. planesByList: treat any plane owner so (family change rules that read the accelerations).
+// pHist; bOn: on by transposed slot. aTerm: A's owner terms; bTerm: B's, by transposed slot; pTerm: A's of the planes, and
+// behind them, from 6 nPlane on, the plane owners'. A clump's terms are summed in the list's order. The plane owners' sums
+// are folded by the places of the plane candidates, which depend on the lists: their last bits may reach an owner's
+// accelerations (which the last step of a call, a pass's, writes anew) but not its motion. Where the forces would move one
+// (its velocities not prescribed) the owner update leaves it where it is and reports ERRBIT_DRIVEN; the host then sums that
+// step's terms by the contact list's places and moves it. PLANES_BY_LIST: so with any plane owner (family change rules that
+// read the accelerations).
+// (No more fields than these: three more words of kernel arguments cost 600 spheres 0.35 us a step.)
 struct DirectList {
     uint32_t nPair, nPlane;
     const uint32_t *candA, *candB, *tPos, *pSph, *pPlane, *pStart;
     uint8_t *on, *pOn, *bOn;
     float4 *hist, *pHist;
-    float *pTerm, *pForce;
+    float* pTerm;
     const uint8_t* mask;  // family mask, null when every pair is allowed
-    uint32_t planesByList;
     DirectState* st;      // null: not stepping on candidates
 };
 // An owner's pose at a candidate build: its position in fixed point (as BuildPos), its orientation, and the largest

@@ -76,6 +76,7 @@ using deme_dev::DirectList;
 using deme_dev::DirectState;
 using deme_dev::OwnerBuild;
 using deme_dev::PART_FROM_COUNTERS;
+using deme_dev::PLANES_BY_LIST;
 using deme_dev::PlaneRefresh;
 using deme_dev::PlaneSums;
 using deme_dev::MatPair;

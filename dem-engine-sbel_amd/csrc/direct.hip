@@ -287,7 +287,7 @@ __global__ __launch_bounds__(256) void k_direct_plane_sums(DirectList D, uint32_
             if (D.pPlane[q] == p) {
                 gOwner = (int)(anal[p].owner - sums.first);
 #pragma unroll
-                for (int k = 0; k < 6; k++) g[k] = D.pForce[(uint64_t)q * 6 + k];
+                for (int k = 0; k < 6; k++) g[k] = D.pTerm[((uint64_t)D.nPlane + q) * 6 + k];
             }
     }
     fold_plane_terms(sums, gOwner, g);
