@@ -303,7 +303,8 @@ struct deme_ctx {
     DBuf<float> lam, lAcc, adjA, adjB, matPart, matGrad;
     DBuf<float4> lDt[2], lDtPrev;
     bool termsReady = false;  // owner terms belong to the current contact list
-    DBuf<float> analPartials;  // plane owners' partial sums, one set per force workgroup
+    DBuf<float> analPartials;  // plane owners' partial sums, one set per force workgroup, and the owners that have them
+    DBuf<uint8_t> analMark;
     bool posesValid = false;   // pose[] belongs to the owners' current state (the owner update refreshes it)
     DBuf<double> clock;  // simulation time read by the owner update's motion rules (written before each such update)
     // cell-list detection
@@ -639,7 +640,7 @@ int deme_ctx_destroy(deme_ctx* c) {
     for (int k = 0; k < 2; k++) {
         c->rowStart[k].release(); c->idB[k].release(); c->ctype[k].release(); c->hist[k].release();
     }
-    c->idA.release(); c->map.release(); c->frc.release(); c->analPartials.release();
+    c->idA.release(); c->map.release(); c->frc.release(); c->analPartials.release(); c->analMark.release();
     c->clock.release();
     c->cellCount.release(); c->cellStart.release(); c->cellOf.release(); c->slotOf.release(); c->posOf.release();
     c->survSlab.release(); c->rowSlab.release(); c->mirSlab.release(); c->sorted.release(); c->planeBits.release();
@@ -1754,6 +1755,7 @@ static uint8_t* term_flags(const deme_ctx* c, bool bSide) {
 static PlaneSums plane_sums(const deme_ctx* c) {
     PlaneSums s;
     s.part = c->analPartials.p;
+    s.mark = c->analMark.p;
     s.first = c->nClumps;
     s.nOwners = c->nAnalOwners;
     return s;
@@ -1769,7 +1771,9 @@ static PlaneRefresh plane_refresh(const deme_ctx* c) {
 
 // Room for the partial sums of a force launch over nC contacts.
 static hipError_t ensure_partials(deme_ctx* c, uint64_t nC, double grow = 1.25) {
-    return c->analPartials.ensure(std::max<size_t>((size_t)anal_blocks(nC) * MAX_ANAL_OWNERS * 6, 1), grow);
+    const size_t n = std::max<size_t>(anal_blocks(nC), 1);
+    const hipError_t e = c->analMark.ensure(n, grow);
+    return e != hipSuccess ? e : c->analPartials.ensure(n * MAX_ANAL_OWNERS * 6, grow);
 }
 
 // A list detected with a drift margin is tested first when it is long and few of its contacts touch. Testing costs a wave
@@ -1943,7 +1947,7 @@ static std::vector<const void*> cycle_fingerprint(deme_ctx* c, int p) {
             c->scanScratch.p, c->survSlab.p,  c->rowSlab.p,     c->mirSlab.p,     c->rowStart[p].p, c->rowStart[q].p,
             c->bRowStart.p,  c->idA.p,        c->idB[p].p,      c->idB[q].p,      c->ctype[p].p,   c->ctype[q].p,
             c->hist[p].p,    c->hist[q].p,    c->map.p,         c->mirror.p,      c->bPart.p,      c->aTerm.p,
-            c->bTerm.p,      c->aOn.p,        c->bOn.p,         c->analPartials.p,
+            c->bTerm.p,      c->aOn.p,        c->bOn.p,         c->analPartials.p, c->analMark.p,
             c->acc.p,        c->clock.p,      c->ctr.p,         c->planeStart.p,
             reinterpret_cast<const void*>(c->jit.full), reinterpret_cast<const void*>(c->jit.terms),
             reinterpret_cast<const void*>(c->jitOwner.fn), v(c->fewTouch),
@@ -1975,7 +1979,8 @@ static int cycle_capacity(deme_ctx* c, int p, SpecGuard& g) {
     g = SpecGuard();
     g.ctr = c->ctr.p;
     g.slabCap = c->slabCap;
-    const uint64_t analCap = (uint64_t)(c->analPartials.cap / (MAX_ANAL_OWNERS * 6)) * ANAL_TILE;
+    const uint64_t analCap =
+        std::min<uint64_t>(c->analPartials.cap / (MAX_ANAL_OWNERS * 6), c->analMark.cap) * ANAL_TILE;
     g.capC = std::min<uint64_t>({c->idB[p].cap, c->ctype[p].cap, c->hist[p].cap, c->idA.cap, c->map.cap,
                                  c->mirror.cap, c->aTerm.cap / 6, c->aOn.cap, analCap,
                                  0xFFFFFFFFull});

@@ -485,13 +485,15 @@ __device__ __forceinline__ PlanePose plane_pose_of(const KParams& P, const deme_
 }
 
 // Sums over the sphere-plane contacts per analytical owner, passed from the force kernel to the owner update. Each
-// force workgroup (ANAL_TILE contacts) writes nOwners x 6 partial sums at part[block * nOwners * 6]; the owner update
-// folds nPart of them (PART_FROM_COUNTERS: the number of blocks of the guard's contact count).
+// force workgroup (ANAL_TILE contacts) marks the owners that it has terms for (a bit each, mark[block]) and writes their 6
+// partial sums at part[(block * nOwners + owner) * 6]; the owner update folds those of nPart blocks (PART_FROM_COUNTERS:
+// the number of blocks of the guard's contact count).
 constexpr uint32_t PART_FROM_COUNTERS = 0xFFFFFFFFu;
 constexpr uint32_t PLANES_BY_LIST = 0x100u;  // (see DirectList)
 constexpr uint32_t MAX_ANAL_OWNERS = 8;
 struct PlaneSums {
     float* part = nullptr;
+    uint8_t* mark = nullptr;
     uint32_t first = 0, nOwners = 0;  // owner numbers first .. first + nOwners - 1
     uint32_t nPart = 0;
     uint32_t flags = 0;  // a bit for each owner that the update leaves as it is, and PLANES_BY_LIST
@@ -502,17 +504,21 @@ struct PlaneSums {
 __device__ __forceinline__ void fold_plane_terms(const PlaneSums& sums, int gOwner, const float (&g)[6]) {
     if (sums.nOwners == 0) return;
     __shared__ float waveSum[4][6];
+    __shared__ uint32_t waveMark[4];
+    static_assert(MAX_ANAL_OWNERS <= 8, "a bit of mark[] per owner");
+    uint32_t mine = 0;
+    for (uint32_t k = 0; k < sums.nOwners; k++) mine |= __any(gOwner == (int)k) ? 1u << k : 0u;
+    if ((threadIdx.x & 63u) == 0) waveMark[threadIdx.x >> 6] = mine;
+    __syncthreads();
+    const uint32_t mark = waveMark[0] | waveMark[1] | waveMark[2] | waveMark[3];
+    if (threadIdx.x == 0) sums.mark[blockIdx.x] = (uint8_t)mark;
     float* dst = sums.part + (uint64_t)blockIdx.x * sums.nOwners * 6;
-    if (!__syncthreads_or(gOwner >= 0)) {
-        if (threadIdx.x < sums.nOwners * 6) dst[threadIdx.x] = 0.f;
-        return;
-    }
     for (uint32_t k = 0; k < sums.nOwners; k++) {
-        const bool mine = gOwner == (int)k;
-        if (__any(mine)) {
+        if (!(mark >> k & 1u)) continue;
+        if (mine >> k & 1u) {
 #pragma unroll
             for (int c = 0; c < 6; c++) {
-                float v = mine ? g[c] : 0.f;
+                float v = gOwner == (int)k ? g[c] : 0.f;
 #pragma unroll
                 for (int off = 32; off > 0; off >>= 1) v += __shfl_xor(v, off, 64);
                 if ((threadIdx.x & 63u) == 0) waveSum[threadIdx.x >> 6][c] = v;

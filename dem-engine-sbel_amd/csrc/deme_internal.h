@@ -255,8 +255,8 @@ hipError_t launch_force(const KParams& P, uint32_t nC, const uint32_t* idA, cons
                         float4* histOut, const uint32_t* mirror, float* aTerm, float* bTerm,
                         const PlaneSums& sums, uint8_t* aOn, uint8_t* bOn,
                         ForceRec* out, hipStream_t st, SpecGuard guard = SpecGuard(), ForceKind kind = FORCE_KIND_ALL);
-// The owner update: nClumps clump owners and sums.nOwners analytical owners (numbered from sums.first). The first
-// workgroup folds the force kernel's partial sums, moves the analytical owners and refreshes the plane poses.
+// The owner update: nClumps clump owners and sums.nOwners analytical owners (numbered from sums.first). A
+// workgroup each folds the force kernel's partial sums of an analytical owner, moves it and refreshes its planes' poses.
 hipError_t launch_owner_update(const KParams& P, uint32_t nO, uint32_t nClumps, const uint32_t* ownerSphStart,
                                const uint32_t* rowStart, const uint32_t* bRowStart, const float* aTerm,
                                const float* bTerm, const uint8_t* aOn, const uint8_t* bOn, const PlaneSums& sums,
@@ -331,10 +331,8 @@ hipError_t launch_fill_u32(uint32_t* p, uint64_t n, uint32_t v, hipStream_t st, 
 hipError_t launch_change_family(OwnerRec* own, uint32_t nO, uint8_t from, uint8_t to, hipStream_t st);
 
 // jit_rt.cpp: the force kernel specialised at run time by hipRTC
-// workgroups of the owner update: one for the analytical owners (when there are any), then 256 clumps each
-inline uint32_t owner_blocks(uint32_t nClumps, uint32_t nAnalOwners) {
-    return (nAnalOwners ? 1u : 0u) + (nClumps + 255) / 256;
-}
+// workgroups of the owner update: one for each analytical owner, then 256 clumps each
+inline uint32_t owner_blocks(uint32_t nClumps, uint32_t nAnalOwners) { return nAnalOwners + (nClumps + 255) / 256; }
 struct JitForce {
     hipModule_t mod = nullptr;
     hipFunction_t full = nullptr, terms = nullptr, margin = nullptr, direct = nullptr;

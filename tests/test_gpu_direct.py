@@ -409,3 +409,26 @@ def test_a_plate_that_its_contacts_move_does_not_depend_on_the_lists(how):
     for k in sa:
         assert np.array_equal(sa[k], sb[k]), k
     assert sa["vZ"][nc + 1] != sc.state["vZ"][nc + 1] and sa["omgX"][nc + 1] != 0.0
+
+
+def test_margin_lists_over_six_plane_owners():
+    """Six floors of as many owners: the kernel that tests a long margin list first marks and folds each as the other kernel
+    does."""
+    sc = scenes.clump_settling(n_clumps=100_003, update_freq=5, beta_frac=0.2, velocity_sigma=0.3, omega_sigma=5.0,
+                               seed=58)
+    nc = sc.n_clumps
+    sc.anal[:] = sc.anal[0]
+    sc.anal["owner"] = nc + np.arange(len(sc.anal))
+    sc.anal["relPos"][:, 2] += 1e-6 * np.arange(len(sc.anal), dtype=np.float32)
+    more = len(sc.anal) - 1
+    sc.state = {q: np.concatenate([v] + [v[nc:nc + 1]] * more) for q, v in sc.state.items()}
+    sc.n_owners = nc + 1 + more
+    sc.owner_mass = np.append(sc.owner_mass, np.full(more, 1e15, np.float32)).astype(np.float32)
+    sc.owner_moi = np.ascontiguousarray(np.append(sc.owner_moi, np.full((more, 3), 1e15, np.float32), 0))
+    a, b = _pair(sc)
+    for chunk in (7, 3, 11):
+        a.step(chunk, 5)
+        b.step(chunk, 5)
+        _same(a, b)
+    assert a.counts().nContacts > 1_000_000
+    assert np.all(a.get_state()["aZ"][nc:] != 0.0)

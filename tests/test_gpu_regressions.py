@@ -191,3 +191,45 @@ def test_plane_owner_sums_at_workgroup_edges(n):
     assert len(a[0]) >= 2 * n
     for x, y in zip(a[:3], b[:3]):
         assert np.array_equal(x, y)
+
+
+@pytest.mark.parametrize("n", [1, 32, 33, 9001])
+def test_sums_of_eight_plane_owners(n):
+    """Every sphere on eight planes of as many owners (every other one free): each owner's partial sums are marked, folded
+    by a workgroup of its own and moved, at 8 n contacts around the edges of a workgroup, against the oracle."""
+    import pyoracle
+
+    side = int(np.ceil(np.sqrt(n)))
+    r = 0.002
+    k = np.arange(n)
+    xyz = np.stack([(k % side) * 2.2 * r, (k // side) * 2.2 * r, np.zeros(n)], 1)
+    L = max(side * 2.2 * r + 8 * r, 0.05)
+    xyz += np.array([-L / 2 + 4 * r, -L / 2 + 4 * r, -L / 2 + 0.9 * r])
+    sc = scenes.spheres_scene(xyz, r, (L, L, L))
+    sc.anal = np.zeros(8, ANAL_DTYPE)
+    for j in range(8):
+        sc.anal[j]["owner"] = n + j
+        sc.anal[j]["relPos"] = (0.0, 0.0, -L / 2 + 0.01 * r * j)
+        sc.anal[j]["rot"] = (0.0, 0.0, 1.0)
+        sc.anal[j]["mass"] = 1e15
+    sc.state = {q: np.concatenate([v] + [v[n:n + 1]] * 7) for q, v in sc.state.items()}
+    sc.state["family"][n + 1::2] = 0
+    sc.n_owners = n + 8
+    sc.owner_mass = np.append(sc.owner_mass, np.full(7, 1e15, np.float32)).astype(np.float32)
+    sc.owner_moi = np.ascontiguousarray(np.append(sc.owner_moi, np.full((7, 3), 1e15, np.float32), 0))
+    dev, ora = DeviceSystem(sc), pyoracle.OracleSystem(sc)
+    for _ in range(3):
+        dev.step(1, 1)
+        ora.step(1, 1)
+        sd, so = dev.get_state(), ora.get_state()
+        for q in ("aX", "aY", "aZ", "alphaX", "alphaY"):
+            d, o = sd[q][n:].astype(np.float64), so[q][n:].astype(np.float64)
+            # sums of n float terms in another order: n ulps of the largest partial sum
+            bound = 1e-5 * np.abs(so["aZ"][n:]) * (L if q.startswith("alpha") else 1.0) + 1e-30
+            assert np.all(np.abs(d - o) <= bound), (q, d, o)
+        for q in ("voxelID", "locX", "locY", "locZ"):
+            assert np.array_equal(sd[q][n:], so[q][n:]), q
+    a, b = dev.contacts(), ora.contacts()
+    assert len(a[0]) >= 8 * n
+    for x, y in zip(a[:3], b[:3]):
+        assert np.array_equal(x, y)
