@@ -560,9 +560,10 @@ int move_packed(deme_ctx* c, const Packing& k, bool down) {
     return DEME_OK;
 }
 
-// The sample of a candidate pass with a drift margin (0.4 with some slack: each change costs captured steps a capture).
+// The sample of a candidate pass with a drift margin: few touch when a wave's 256 contacts mostly leave one round of 64 for
+// the model (force_kind; with some slack, since each change costs captured steps a capture).
 static void count_touching(deme_ctx* c, const DevCounters& h) {
-    if (h.sampled > 0) c->fewTouch = h.touching <= (c->fewTouch ? 0.45 : 0.35) * h.sampled;
+    if (h.sampled > 0) c->fewTouch = h.touching <= (c->fewTouch ? 0.24 : 0.22) * h.sampled;
 }
 
 int readback_counters(deme_ctx* c) {
@@ -1777,9 +1778,13 @@ static hipError_t ensure_partials(deme_ctx* c, uint64_t nC, double grow = 1.25) 
 }
 
 // A list detected with a drift margin is tested first when it is long and few of its contacts touch. Testing costs a wave
-// a second round of gathers before the model (0.64M contacts of which a sixth touch: 29.8 us against 26.3, all through
-// the model); a long list is bound by the model's instructions (1.3M: 35.8 against 44.6 us; 4.9M: 125 against 181), and
-// each quarter of the contacts that touches adds a round of the model (all touching: 243 us, so 0.4 is about even).
+// a second round of gathers before the model, which a short list waits for, while a long one is bound by the model's
+// instructions; and a wave that finds more than 64 of its 256 contacts touching runs the model a second time for the rest.
+// Tested first against all through the model, us, with the share that touches:
+//   0.16: 1.1M contacts 35.6 / 36.7, 1.8M 46.5 / 54.8, 5.6M 138 / 186, 18.9M 462 / 608
+//   0.20: 1.3M 40.5 / 41.6, 4.4M 123 / 152, 14.9M 399 / 490
+//   0.26: 1.1M 47.1 / 38.4, 3.3M 123 / 124, 11.2M 383 / 393
+//   0.42: 7.0M 296 / 275;  0.24: 0.65M 34.1 / 27.5
 // Testing first clears the history of a contact that does not touch; a caller's own way of destroying it runs in the
 // kernel that takes every contact.
 static ForceKind force_kind(const deme_ctx* c, uint64_t nC, bool settled) {
