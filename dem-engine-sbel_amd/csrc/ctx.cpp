@@ -202,6 +202,7 @@ struct deme_ctx {
     uint32_t nPlane = 0;
     uint64_t planesGen = 0;
     uint32_t directSkip = 0, directBackoff = 0;
+    uint64_t directSteps = 0, directBuilds = 0, marginLaunches = 0;  // (deme_path_stats)
     int pairMode = -1;  // pair sweep mode (launch_cell_pairs); -1: chosen from the radius spread
     uint32_t pairBlock = 256;  // pair sweep workgroup size
     double cycleHeadroom = 1.25;  // capacity of a captured interval: headroom x the current counts + slack
@@ -1802,6 +1803,7 @@ static hipError_t launch_force_ctx(deme_ctx* c, bool full, uint32_t nC, const ui
                                    const OwnerRec* own, const float4* histIn, const uint32_t* map, float4* histOut,
                                    ForceRec* out, SpecGuard guard = SpecGuard(), bool settled = false) {
     const ForceKind kind = force_kind(c, nC, settled);
+    if (!full && kind != FORCE_KIND_ALL) c->marginLaunches++;
     if (c->jitActive)
         return c->jit.launch(full, c->kp, nC, c->idA.p, idB, ctype, c->sph.p, own, c->moi.p, c->anal.p, c->pose.p,
                              c->mats.p, histIn, map, histOut, c->mirror.p, c->aTerm.p, c->bTerm.p, plane_sums(c),
@@ -2285,6 +2287,7 @@ static int direct_rebuild(deme_ctx* c) {
     DEME_LAUNCH(c, "direct_join",
                 launch_direct_join(c->nS, c->candStartOld.p, c->candBOld.p, c->candStart.p, c->candB.p, c->pStartOld.p,
                                    c->pPlaneOld.p, old, direct_list(c), c->stream));
+    c->directBuilds++;
     return direct_begin(c);
 }
 
@@ -2437,6 +2440,7 @@ static int direct_steps(deme_ctx* c, int n, int* done, bool* again) {
             c->nSteps++;
         }
         held = err & ERRBIT_DRIVEN ? c->hdstate->d.held : 0;
+        c->directSteps += steps;
         *done += (int)steps;
         c->passesSinceBuild += steps;
         if (c->passesSinceBuild >= 4) c->cellBackoff = 0;
@@ -2628,6 +2632,13 @@ int deme_graph_stats(deme_ctx* c, uint64_t out[3]) {
     out[0] = c->cycleCaptures;
     out[1] = c->cycleReplays;
     out[2] = c->cycleFallbacks;
+    return DEME_OK;
+}
+
+int deme_path_stats(deme_ctx* c, uint64_t out[3]) {
+    out[0] = c->directSteps;
+    out[1] = c->directBuilds;
+    out[2] = c->marginLaunches;
     return DEME_OK;
 }
 

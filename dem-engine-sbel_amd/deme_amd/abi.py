@@ -90,7 +90,7 @@ EXPORTED = [
     "deme_change_clump_sizes",
     "deme_clear_motion_rules", "deme_change_family", "deme_jit_render_owner", "deme_jit_render_inspect",
     "deme_prefix_scan_u32", "deme_integrate_owners", "deme_prefix_scan_u32_noalloc", "deme_set_graph_headroom",
-    "deme_graph_stats", "deme_set_pair_sweep", "deme_autotune_sweep", "deme_set_skin", "deme_candidate_stats",
+    "deme_graph_stats", "deme_path_stats", "deme_set_pair_sweep", "deme_autotune_sweep", "deme_set_skin", "deme_candidate_stats",
 ]
 
 _lib = None
@@ -138,7 +138,7 @@ def load(path: str = LIB_PATH):
         "deme_prefix_scan_u32": ([vp, vp, vp, u64, C.POINTER(u64)], i32),
         "deme_prefix_scan_u32_noalloc": ([vp, vp, vp, u64, vp], i32),
         "deme_set_graph_headroom": ([vp, C.c_double, u64], i32),
-        "deme_graph_stats": ([vp, vp], i32),
+        "deme_graph_stats": ([vp, vp], i32), "deme_path_stats": ([vp, vp], i32),
         "deme_set_pair_sweep": ([vp, i32, i32], i32),
         "deme_set_skin": ([vp, C.c_double], i32),
         "deme_candidate_stats": ([vp, vp, vp, vp], i32),
@@ -422,6 +422,13 @@ class DeviceSystem:
         """(captures, replays that advanced the system, replays that fell back to direct launches)"""
         out = np.zeros(3, np.uint64)
         self._chk(self.lib.deme_graph_stats(self.ctx, C.c_void_p(out.ctypes.data)))
+        return tuple(int(x) for x in out)
+
+    def path_stats(self):
+        """(steps taken on the candidates, list builds between them, launches of the force kernel that tests a long
+        margin list first)"""
+        out = np.zeros(3, np.uint64)
+        self._chk(self.lib.deme_path_stats(self.ctx, C.c_void_p(out.ctypes.data)))
         return tuple(int(x) for x in out)
 
     def set_owner_volumes(self, volume):

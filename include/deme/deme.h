@@ -138,6 +138,9 @@ int deme_integrate_owners(deme_ctx* ctx);
  * every step without a drift margin, all steps of a call but the last run on the candidate lists (deme_set_skin)
  * without forming a contact list; the last runs its own pass, so list, map and records are those of every step. */
 int deme_step(deme_ctx* ctx, int n_steps, int update_freq);
+/* Which ways steps went so far: out[0] steps taken on the candidates, out[1] list builds between them, out[2] launches
+ * (captured ones counted once) of the force kernel that tests a long margin list first. */
+int deme_path_stats(deme_ctx* ctx, uint64_t out[3]);
 /* HIP-graph replay in deme_step (no counterpart in the reference, which launches every kernel and waits on the host
  * for each detection pass's counts). When on, each whole detection interval -- the detection pass and the update_freq
  * steps up to the next one -- is one graph launch, captured once per list parity and replayed while the buffers it

@@ -105,6 +105,7 @@ def test_steps_on_the_candidates_equal_the_contact_list_path(name, skin):
     a, b = _pair(sc, setup)
     if skin is not None:
         a.set_skin(skin)
+    done = 0
     for chunk in (1, 5, 6, 7, 40, 1, 70):
         a.step(chunk, 1)
         b.step(chunk, 1)
@@ -112,6 +113,12 @@ def test_steps_on_the_candidates_equal_the_contact_list_path(name, skin):
         if name == "model":
             for x, y in zip(a.forces(), b.forces()):
                 assert np.array_equal(x, y)
+        # all but the last step of a call of six or more; the gas's lists die at once, so that the automatic skin gives way
+        # to the cell sweep before a call is long enough
+        now = a.path_stats()[0] - done
+        assert now == 0 if chunk < 6 or (name, skin) == ("fast_gas", None) else chunk - 2 <= now <= chunk - 1
+        done += now
+    assert b.path_stats()[:2] == (0, 0)
     if name not in ("apart",):
         assert a.counts().nContacts > 20
 
@@ -215,6 +222,7 @@ def test_margin_lists_tested_first_equal_all_through_the_model(how):
         b.step(chunk, 5)
         _same(a, b)
     assert a.counts().nContacts > 1_000_000 and a.counts().nContacts % 256
+    assert a.path_stats()[2] > 0 and b.path_stats()[2] == 0
 
 
 def test_a_failed_list_build_leaves_no_lists():
@@ -268,6 +276,7 @@ def test_margin_lists_destroy_histories_as_the_caller_says():
         _same(a, b)
     assert a.counts().nContacts > 1_000_000
     assert (a.wildcards()[3] <= -1.0).mean() > 0.5
+    assert a.path_stats()[2] == 0
 
 
 def _grazing_past_the_grid(m=17):
@@ -327,6 +336,7 @@ def test_a_skin_narrowed_on_entry_keeps_the_check_of_the_state():
         assert chunk > 1 or b.counts().nContacts == 1
         _same(a, b)
     assert a.candidate_stats()[0] < 0.5 * b.scene.sph_radius.mean() * 0.2 and a.candidate_stats()[2] == 2
+    assert a.path_stats()[:2] == (0, 1)  # narrowed on entry, and no step taken from that state
 
 
 def test_a_calm_system_made_fast_gets_wider_lists():
@@ -409,6 +419,8 @@ def test_a_plate_that_its_contacts_move_does_not_depend_on_the_lists(how):
     for k in sa:
         assert np.array_equal(sa[k], sb[k]), k
     assert sa["vZ"][nc + 1] != sc.state["vZ"][nc + 1] and sa["omgX"][nc + 1] != 0.0
+    # the step that held the plate back, and those before it was let go
+    assert a.path_stats()[0] >= (20 if how == "freed by a rule" else 1) and c.path_stats()[0] >= 1
 
 
 def test_margin_lists_over_six_plane_owners():
@@ -432,3 +444,4 @@ def test_margin_lists_over_six_plane_owners():
         _same(a, b)
     assert a.counts().nContacts > 1_000_000
     assert np.all(a.get_state()["aZ"][nc:] != 0.0)
+    assert a.path_stats()[2] > 0 and b.path_stats()[2] == 0
