@@ -503,7 +503,7 @@ struct Packing {
     }
 };
 
-// The packed buffer c->pack to the caller's arrays (down) or the other way, in chunks of one pinned slot per worker:
+// The packed buffer c->pack to the caller's arrays (down) or the other way, in chunks of a pinned slot:
 // while one chunk is on the link, the workers copy others to or from the caller's pageable memory, whose first touch
 // (page by page) costs more than the transfer itself and spreads over the workers. Measured for 1M owners (85 MB, fresh
 // arrays): 23 ms by the runtime's own pageable copies and one host loop over the records.
@@ -511,43 +511,63 @@ constexpr size_t STAGE_SLOT = 2u << 20;
 constexpr int STAGE_WORKERS = 8;
 int move_packed(deme_ctx* c, const Packing& k, bool down) {
     if (!k.total) return DEME_OK;
-    const size_t slot = std::min(STAGE_SLOT, (k.total + 65535) & ~(size_t)65535);
+    // Up to four slots' worth is the calling thread's alone, in halves of a slot: one is on the link while it copies another.
+    // Threads save nothing there, and beside a program's spinning OpenMP threads they may not start for 3 to 4 ms. Down / up,
+    // ms, one thread against one per slot:
+    //   100k owners (8 MB): 0.40 / 0.32 against 0.45 / 0.32; between torch reductions, mean of 25, 0.40 / 0.36 against
+    //   1.33 / 0.84
+    //   50k owners (4 MB): 0.24 / 0.19 against 0.28 / 0.22; 0.24 / 0.21 against 0.50 / 0.72
+    // 200k owners (16 MB): 1.0 / 0.7 alone, 0.83 / 0.61 with eight threads (3.8 / 3.9 between reductions).
+    const bool alone = k.total <= 4 * STAGE_SLOT;
+    const size_t part = alone ? std::min(k.total, STAGE_SLOT / 2) : STAGE_SLOT;
+    const size_t slot = (part + 65535) & ~(size_t)65535;
     const size_t chunks = (k.total + slot - 1) / slot;
-    // One or two slots' worth is the calling thread's alone. A second thread saves nothing there (50k owners, 4 MB: 0.26 and
-    // 0.20 ms with one, 0.25 and 0.22 with two, down and up), and beside a program's spinning OpenMP threads it may not
-    // start for 3 to 4 ms (of 25 calls between torch reductions the mean is 0.27 and 0.23 ms with one, 0.50 and 0.72 with
-    // two).
-    const int workers = chunks <= 2 ? 1 : (int)std::min<size_t>(chunks, STAGE_WORKERS);
-    if (c->stageBytes < slot * workers) {
+    const int workers = alone ? 1 : (int)std::min<size_t>(chunks, STAGE_WORKERS);
+    const int depth = alone ? 2 : 1;  // slots of a worker
+    if (c->stageBytes < slot * workers * depth) {
         if (c->stage) DEME_HIP(c, hipHostFree(c->stage));
         c->stage = nullptr;
         c->stageBytes = 0;
-        DEME_HIP(c, hipHostMalloc((void**)&c->stage, slot * workers, hipHostMallocDefault));
-        c->stageBytes = slot * workers;
+        DEME_HIP(c, hipHostMalloc((void**)&c->stage, slot * workers * depth, hipHostMallocDefault));
+        c->stageBytes = slot * workers * depth;
     }
-    for (int w = 0; w < workers; w++)
+    for (int w = 0; w < workers * depth; w++)
         if (!c->stageEv[w]) DEME_HIP(c, hipEventCreateWithFlags(&c->stageEv[w], hipEventDisableTiming));
     hipError_t err[STAGE_WORKERS] = {};
     auto work = [&](int w) {
-        uint8_t* s = c->stage + slot * w;
         hipError_t e = hipSetDevice(c->device);
-        for (size_t j = w; j < chunks && e == hipSuccess; j += workers) {
-            const size_t lo = j * slot, hi = std::min(lo + slot, k.total);
-            auto touch = [&] {  // the chunk's part of every array that overlaps it
-                for (const PackedArray& a : k.arrays) {
-                    const size_t b = std::max(lo, a.off), f = std::min(hi, a.off + a.bytes);
-                    if (b >= f) continue;
-                    if (down) std::memcpy(a.host + (b - a.off), s + (b - lo), f - b);
-                    else std::memcpy(s + (b - lo), a.host + (b - a.off), f - b);
-                }
-            };
-            if (!down) touch();
-            e = down ? hipMemcpyAsync(s, c->pack.p + lo, hi - lo, hipMemcpyDeviceToHost, c->stream)
-                     : hipMemcpyAsync(c->pack.p + lo, s, hi - lo, hipMemcpyHostToDevice, c->stream);
-            if (e == hipSuccess) e = hipEventRecord(c->stageEv[w], c->stream);
-            if (e == hipSuccess) e = hipEventSynchronize(c->stageEv[w]);
-            if (e == hipSuccess && down) touch();
+        const size_t mine = chunks > (size_t)w ? (chunks - w + workers - 1) / workers : 0;  // chunks w, w + workers, ...
+        auto at = [&](size_t i) { return w * depth + (int)(i % depth); };
+        auto touch = [&](size_t i) {  // the i-th chunk's part of every array that overlaps it
+            uint8_t* s = c->stage + slot * at(i);
+            const size_t lo = (w + i * workers) * slot, hi = std::min(lo + slot, k.total);
+            for (const PackedArray& a : k.arrays) {
+                const size_t b = std::max(lo, a.off), f = std::min(hi, a.off + a.bytes);
+                if (b >= f) continue;
+                if (down) std::memcpy(a.host + (b - a.off), s + (b - lo), f - b);
+                else std::memcpy(s + (b - lo), a.host + (b - a.off), f - b);
+            }
+        };
+        auto send = [&](size_t i) {
+            uint8_t* s = c->stage + slot * at(i);
+            const size_t lo = (w + i * workers) * slot, n = std::min(slot, k.total - lo);
+            e = down ? hipMemcpyAsync(s, c->pack.p + lo, n, hipMemcpyDeviceToHost, c->stream)
+                     : hipMemcpyAsync(c->pack.p + lo, s, n, hipMemcpyHostToDevice, c->stream);
+            if (e == hipSuccess) e = hipEventRecord(c->stageEv[at(i)], c->stream);
+        };
+        if (down)
+            for (size_t i = 0; i < mine && i < (size_t)depth && e == hipSuccess; i++) send(i);
+        for (size_t i = 0; i < mine && e == hipSuccess; i++) {
+            // (down: the chunk has arrived; up: the chunk before it in this slot has left)
+            if (down || i >= (size_t)depth) e = hipEventSynchronize(c->stageEv[at(i)]);
+            if (e != hipSuccess) break;
+            touch(i);
+            if (!down) send(i);
+            else if (i + depth < mine) send(i + depth);
         }
+        if (!down)
+            for (size_t i = mine > (size_t)depth ? mine - depth : 0; i < mine && e == hipSuccess; i++)
+                e = hipEventSynchronize(c->stageEv[at(i)]);
         err[w] = e;
     };
     std::thread th[STAGE_WORKERS];

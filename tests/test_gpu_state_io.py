@@ -20,8 +20,9 @@ def _random_state(n, rng):
     return st
 
 
-# 79 bytes an owner: 2 MiB slots end near 26,546 owners; 400,001 take more chunks than there are slots
-@pytest.mark.parametrize("n", [1, 2, 63, 26_545, 26_547, 400_001])
+# 79 bytes an owner: the calling thread alone takes halves of a slot (1 MiB, near 13,273 owners) up to 8 MiB (near 106,184);
+# beyond, 2 MiB slots end near multiples of 26,546 owners, and 400,001 take more chunks than there are slots
+@pytest.mark.parametrize("n", [1, 2, 63, 13_272, 13_274, 26_545, 26_547, 106_180, 106_190, 400_001])
 def test_states_come_back_as_they_went(n):
     rng = np.random.default_rng(n)
     g = np.arange(n)
