@@ -124,8 +124,9 @@ struct deme_ctx {
     // Candidate-list detection: pairs within `skin` of touching, kept from a build until some sphere has moved half
     // the skin; each pass then tests only them. skinSet < 0: automatic (0.2 x the mean radius); 0: off (the cell
     // sweep every pass).
-    // The automatic skin (any skin gives the same contacts) adapts at each build, within 0.05 to 0.8 x the mean
-    // radius, to the lists just retired. Lists that die within a pass widen it 1.5x; lists that outlast 400 passes
+    // The automatic skin (any skin gives the same contacts): where steps run on the candidates, chosen from a build's
+    // statistics (skinNext, skin_choice.h). Else it adapts at each build, within 0.05 to 0.8 x the mean radius, to the
+    // lists just retired. Lists that die within a pass widen it 1.5x; lists that outlast 400 passes
     // narrow it 0.75x. Lists that last 30 passes or more leave it alone (their builds cost little). Shorter-lived
     // lists steer it by their cost per pass -- candidates times (1 + BUILD_PASSES / the passes they lasted), a build
     // costing about as much as BUILD_PASSES passes over its candidates: it moves 1.25x (widening first when lists

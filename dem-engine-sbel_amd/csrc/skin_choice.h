@@ -37,7 +37,7 @@ struct SkinChoice {
 // it. Where none of them lasts -- a calm system made fast, its lists thin -- the wider ones up to SKIN_WIDEST are looked
 // at too, and the widest is taken where none lasts at all: a list that lives a step costs a build at any skin, so the
 // thinnest would look cheapest, and neither a wider skin nor the cell sweep would ever be tried.
-// (1M clumps moving at 0.02 m/s: 0.2 r lists 4.98M candidates, 352 us a step; the skin chosen 2.97M, 269 us.)
+// (1M clumps moving at 0.02 m/s: 0.2 r lists 4.95M candidates, 343 us a step; the skin chosen 2.98M, 247 to 288 us.)
 inline SkinChoice choose_skin(const SkinView& v) {
     const double s = v.skin, m = v.meanRadius, widest = SKIN_WIDEST * m;
     auto life = [&](double skin) { return 0.5 * skin / v.move; };

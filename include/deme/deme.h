@@ -135,8 +135,10 @@ int deme_integrate(deme_ctx* ctx);
 int deme_integrate_owners(deme_ctx* ctx);
 /* The step loop (DEMDynamicThread::workerThread, dT.cpp:1527-1585) with a deterministic contact-update schedule:
  * detection on the state at steps k*f (f = max(update_freq, 1)), force -> collect -> integrate each step. Detecting
- * every step without a drift margin, all steps of a call but the last run on the candidate lists (deme_set_skin)
- * without forming a contact list; the last runs its own pass, so list, map and records are those of every step. */
+ * every step without a drift margin, all steps of a call of six or more but the last run on the candidate lists
+ * (deme_set_skin) without forming a contact list; the last runs its own pass, so list, map and records are those of
+ * every step. Results do not depend on it. Not with deme_set_step_graphs, and only up to the first step for an
+ * external object that contact forces move. */
 int deme_step(deme_ctx* ctx, int n_steps, int update_freq);
 /* Which ways steps went so far: out[0] steps taken on the candidates, out[1] list builds between them, out[2] launches
  * (captured ones counted once) of the force kernel that tests a long margin list first. */
@@ -148,7 +150,8 @@ int deme_path_stats(deme_ctx* ctx, uint64_t out[3]);
  * the pass failed or its lists outgrew the captured capacity, in which case the replay changes nothing and the
  * interval runs directly (regrowing the buffers) before the next capture. Steps outside whole intervals replay a
  * per-step graph. Off by default (direct launches). Results are identical either way. Kernel timing
- * (deme_enable_kernel_timing) runs directly. */
+ * (deme_enable_kernel_timing) runs directly. With detection every step and no drift margin direct launches are the
+ * faster choice: steps then run on the candidate lists (deme_step), which graphs exclude. */
 int deme_set_step_graphs(deme_ctx* ctx, int on);
 /* Capacity a captured interval gets over the current list: factor x the contact (and mirror-row) count + slack
  * (defaults 1.25 and 1024). */
@@ -162,8 +165,9 @@ int deme_set_graph_headroom(deme_ctx* ctx, double factor, uint64_t slack);
  * automatic, starting at 0.2 x the mean sphere radius and adapted at each build, within 0.05-0.8 x, to the lists it
  * retires (widened 1.5x when they died within a pass, narrowed 0.75x when they outlasted 400 passes, left alone from
  * 30 passes on; lists shorter-lived than that steer it 1.25x at a time by their candidates x (1 + 2.7 / passes
- * lasted)), and where steps run on the candidates also chosen from the gaps between them and the largest speed; when
- * lists die within 4 passes even at the widest skin, the cell sweep runs every pass for 64 passes
+ * lasted)). Where steps run on the candidates it is instead chosen at each build, within 0.01-0.8 x, from the gaps
+ * between them and the largest speed: the least time per step among skins whose lists last 4 steps, the widest where
+ * none does. When lists die within 4 passes even at the widest skin, the cell sweep runs every pass for 64 passes
  * (doubling while that repeats, up to 4096) before lists are tried again. 0: off (the cell sweep every pass). The
  * build positions are kept in fixed point (a power-of-two unit u, about 2^-31 of twice the bin grid's largest
  * extent); a skin with skin / 2 <= 1 nm + 4u also runs the cell sweep (deme_candidate_stats then reports 0). */
