@@ -445,3 +445,19 @@ def test_margin_lists_over_six_plane_owners():
     assert a.counts().nContacts > 1_000_000
     assert np.all(a.get_state()["aZ"][nc:] != 0.0)
     assert a.path_stats()[2] > 0 and b.path_stats()[2] == 0
+
+
+def test_a_list_that_outgrows_its_buffers_within_a_call():
+    """A lattice without a contact closes up during one call: the contact list that the call ends in, and the one that a
+    rebuild on the way hands its histories through, are many times longer than the buffers the call began with."""
+    r = 0.005
+    g = np.stack(np.meshgrid(*[np.arange(14)] * 3, indexing="ij"), -1).reshape(-1, 3) * (2.01 * r)
+    g -= g.mean(0)
+    sc = scenes.spheres_scene(g, r, (0.4, 0.4, 0.4), vel=-60.0 * g, g=(0.0, 0.0, 0.0), planes=False)
+    a, b = _pair(sc)
+    for chunk, least in ((1, 0), (30, 500), (20, 1000)):
+        a.step(chunk)
+        b.step(chunk)
+        _same(a, b)
+        assert a.counts().nContacts >= least and (chunk > 1 or a.counts().nContacts == 0)
+    assert a.path_stats()[0] >= 40
