@@ -608,7 +608,8 @@ __device__ __forceinline__ bool spec_skip(const SpecGuard& g) {
 // --------------------------------------------------------------------------------------------------------------
 // err: set by the checks of a state (ERRBIT_*), sticky; the force kernel copies it to skip, which the owner update of
 // the same step obeys (that kernel itself checks the state it leaves, so it cannot read err); steps: owner updates
-// done; held: the plane owners left where they are (a bit each); disp: the largest displacements since the build (bits of doubles, spread over DISP_SLOTS words).
+// done; held: the plane owners left where they are (a bit each); disp: the largest displacements since the build (bits of
+// doubles, spread over DISP_SLOTS words).
 struct DirectState {
     // lines of their own: a word read by every wave beside one that atomics change misses the caches
     uint32_t err, pad0[31], skip, pad1[31], steps, held, pad2[30];

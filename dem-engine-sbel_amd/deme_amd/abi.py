@@ -90,7 +90,8 @@ EXPORTED = [
     "deme_change_clump_sizes",
     "deme_clear_motion_rules", "deme_change_family", "deme_jit_render_owner", "deme_jit_render_inspect",
     "deme_prefix_scan_u32", "deme_integrate_owners", "deme_prefix_scan_u32_noalloc", "deme_set_graph_headroom",
-    "deme_graph_stats", "deme_path_stats", "deme_set_pair_sweep", "deme_autotune_sweep", "deme_set_skin", "deme_candidate_stats",
+    "deme_graph_stats", "deme_path_stats", "deme_set_pair_sweep", "deme_autotune_sweep", "deme_set_skin",
+    "deme_candidate_stats",
 ]
 
 _lib = None
