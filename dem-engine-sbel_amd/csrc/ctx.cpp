@@ -524,7 +524,7 @@ int move_packed(deme_ctx* c, const Packing& k, bool down) {
     const size_t slot = (part + 65535) & ~(size_t)65535;
     const size_t chunks = (k.total + slot - 1) / slot;
     const int workers = alone ? 1 : (int)std::min<size_t>(chunks, STAGE_WORKERS);
-    const int depth = alone ? 2 : 1;  // slots of a worker
+    const int depth = alone && chunks > 1 ? 2 : 1;  // slots of a worker
     if (c->stageBytes < slot * workers * depth) {
         if (c->stage) DEME_HIP(c, hipHostFree(c->stage));
         c->stage = nullptr;
